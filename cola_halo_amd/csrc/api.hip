@@ -99,6 +99,7 @@ struct cola_context {
   int fft_schedule = 0;     // radix schedule of the PM transforms (fft_factor)
   CicGeom cic;
   TileGeom tiles;
+  int tile_sides[3] = {0, 0, 0};  // the sides asked for (cola_set_tiling), of the default tiles their dividing name
   BinBuffers bins;
 
   static constexpr int kMassSlots = 64;
@@ -474,13 +475,7 @@ int cola_context_create(int nc, int ngrid, double boxsize, cola_context** out)
   // one y band of each lattice slab (nc^2 particles) per XCD
   c->cic.readout_group = (int)std::max(8LL, (long long)nc * nc / 256 / 8);
   c->grid_floats = (long long)ngrid * ngrid * c->cic.row;
-  // default deposit tile 8 x 8 x 32 cells, halved until it divides ngrid
-  auto pick = [&](int want) {
-    for (int t = want; t > 1; t /= 2)
-      if (ngrid % t == 0) return t;
-    return 1;
-  };
-  if (!make_tile_geom(ngrid, pick(8), pick(8), pick(32), &c->tiles)) return fail(kErrArg);
+  if (!default_tile_geom(ngrid, c->tile_sides, &c->tiles)) return fail(kErrArg);
   const size_t pbytes = sizeof(float) * (size_t)c->np;
   if (hipMalloc(&c->pbuf, pbytes * 15) != hipSuccess) {
     set_error("cannot allocate particle state");
@@ -1471,12 +1466,19 @@ namespace {
 
 int set_deposit_tiles(cola_context* c, int tx, int ty, int tz)
 {
-  TileGeom t;
+  TileGeom t, dflt;
   if (!make_tile_geom(c->ng, tx, ty, tz, &t)) {
     set_error("deposit tile sides must be powers of two dividing ngrid (x side >= 2), <= 4096 cells");
     return kErrArg;
   }
-  if (t.tx == c->tiles.tx && t.ty == c->tiles.ty && t.tz == c->tiles.tz && c->bins.counts) return kOk;
+  // the dividing sides of the default tiles stand for them (ragged or not)
+  int want[3];
+  if (default_tile_geom(c->ng, want, &dflt) && tx == want[0] && ty == want[1] && tz == want[2]) t = dflt;
+  auto named = [&] { c->tile_sides[0] = tx, c->tile_sides[1] = ty, c->tile_sides[2] = tz; };
+  if (t.tx == c->tiles.tx && t.ty == c->tiles.ty && t.tz == c->tiles.tz && c->bins.counts) {
+    named();
+    return kOk;
+  }
   COLA_HIP(hipStreamSynchronize(c->stream));
   drop_step_graph(c);
   COLA_TRY(check_pending(c));
@@ -1485,6 +1487,7 @@ int set_deposit_tiles(cola_context* c, int tx, int ty, int tz)
   bin_free(&c->bins);
   c->bins = nb;
   c->tiles = t;
+  named();
   return kOk;
 }
 
@@ -1633,9 +1636,7 @@ int cola_autotune(cola_context* c, int reps, cola_tuning* out)
   ResNet* const net = c->net;
   c->net = nullptr;  // restored below on every path
   cola_tuning best;
-  best.tile[0] = c->tiles.tx;
-  best.tile[1] = c->tiles.ty;
-  best.tile[2] = c->tiles.tz;
+  for (int a = 0; a < 3; ++a) best.tile[a] = c->tile_sides[a];
   best.fft_log2_cols = c->fft_log2_tile;
   best.fft_log2_rows = c->fft_log2_rows;
   best.fft_log2_xcols = c->fft_log2_xtile;

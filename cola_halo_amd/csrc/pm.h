@@ -41,7 +41,12 @@ struct TileGeom {
   int ntx = 0, nty = 0, ntz = 0;
   long long ntiles = 0;
 };
-bool make_tile_geom(int ng, int tx, int ty, int tz, TileGeom* t);
+// ragged: the last tile of an axis may reach past an (even) grid's end.
+bool make_tile_geom(int ng, int tx, int ty, int tz, TileGeom* t, bool ragged = false);
+// The tiles a context starts with: 8 x 8 x 32, ragged where the grid is no
+// multiple.  want: the largest power-of-two divisors of ng up to those sides,
+// which is the name the tile requests know them by.
+bool default_tile_geom(int ng, int want[3], TileGeom* t);
 
 struct BinBuffers {
   int* counts = nullptr;       // ntiles, zero between steps

@@ -85,7 +85,8 @@ __device__ inline bool cic_with_ghost(float x, float y, float z, const CicGeom& 
 // (x > x_right, so X >= ng - 2 up to rounding), the copy's cells, of which
 // only 0 lies in the grid: the particle's own valid cells are ng-2 and ng-1,
 // in one tile whenever tiles are at least 2 cells wide along x
-// (make_tile_geom), and the ghost adds tile 0.  So every axis touches at
+// (make_tile_geom; so is the last tile of a ragged axis: ng is even), and the
+// ghost adds tile 0.  So every axis touches at
 // most two tiles, and {lo, hi} lists them exactly.  Returns false (no tiles)
 // where cic_cells emits nothing (y or z below -1 cell).
 struct TileSpan {
@@ -543,10 +544,12 @@ __device__ __forceinline__ void deposit_tile(const CicGeom& g, const TileGeom& t
   __syncthreads();
   double s = 0.0;
   const int zmask = t.tz - 1, ymask = t.ty - 1;
+  // the last tiles of a grid that is no multiple of the tile side end at the grid
+  const bool ragged = x0 + t.tx > g.ng || y0 + t.ty > g.ng || z0 + t.tz > g.ng;
   auto cell_value = [&](int e) {
     return (float)(-1.0 + (double)cells[e] * kUnfix);  // pm.c:220 density starts at -1
   };
-  if (t.lz >= 2) {
+  if (t.lz >= 2 && !ragged) {
     // four consecutive z cells per thread: one 16-byte store (rows start on
     // 16-byte boundaries and z0 is a multiple of 4)
     for (int e = threadIdx.x << 2; e < ncell; e += kDepositThreads << 2) {
@@ -565,6 +568,7 @@ __device__ __forceinline__ void deposit_tile(const CicGeom& g, const TileGeom& t
       const int lk = e & zmask;
       const int lj = (e >> t.lz) & ymask;
       const int li = e >> (t.lz + t.ly);
+      if (ragged && (x0 + li >= g.ng || y0 + lj >= g.ng || z0 + lk >= g.ng)) continue;
       const float v = cell_value(e);
       density[((long long)(x0 + li) * g.ng + (y0 + lj)) * g.row + (z0 + lk)] = v;
       s += (double)v;
@@ -979,10 +983,11 @@ static int log2_exact(int v)
   return (1 << l) == v ? l : -1;
 }
 
-bool make_tile_geom(int ng, int tx, int ty, int tz, TileGeom* t)
+bool make_tile_geom(int ng, int tx, int ty, int tz, TileGeom* t, bool ragged)
 {
   // tx >= 2: a ghost's x cells then span at most two x tiles (tile_span)
-  if (tx < 2 || ty <= 0 || tz <= 0 || ng % tx || ng % ty || ng % tz) return false;
+  if (tx < 2 || ty <= 0 || tz <= 0) return false;
+  if (ragged ? ng % 2 != 0 : (ng % tx || ng % ty || ng % tz)) return false;
   if ((long long)tx * ty * tz > 4096) return false;
   const int lx = log2_exact(tx), ly = log2_exact(ty), lz = log2_exact(tz);
   if (lx < 0 || ly < 0 || lz < 0) return false;
@@ -992,11 +997,35 @@ bool make_tile_geom(int ng, int tx, int ty, int tz, TileGeom* t)
   t->lx = lx;
   t->ly = ly;
   t->lz = lz;
-  t->ntx = ng / tx;
-  t->nty = ng / ty;
-  t->ntz = ng / tz;
+  t->ntx = (ng + tx - 1) / tx;
+  t->nty = (ng + ty - 1) / ty;
+  t->ntz = (ng + tz - 1) / tz;
   t->ntiles = (long long)t->ntx * t->nty * t->ntz;
   return t->ntiles <= 0x7fffffffLL;
+}
+
+// Dividing tiles of a grid with few factors of two are tiny (270, 250: 2 x 2
+// x 2, 2.5 M tiles with a workgroup, offsets and repeated particles each), and
+// the step was bound by launching and scanning them.  8 x 8 x 32 with ragged
+// last tiles instead, measured (binning + deposit, dividing -> ragged):
+// 108^3 / 270^3 2880 -> 104 us, 100^3 / 250^3 2320 -> 95 us, 36^3 / 108^3
+// 246 -> 59 us, 120^3 / 360^3 (8 x 8 x 8) 244 -> 148 us, 160^3 / 400^3 (8 x
+// 8 x 16) 263 -> 222 us.  Dividing tiles of 512 cells stay where ragged ones
+// would be fewer than two to a CU (72^3 / 72^3: 70 -> 81 us).
+bool default_tile_geom(int ng, int want[3], TileGeom* t)
+{
+  const int full[3] = {8, 8, 32};
+  bool divides = true;
+  int cells = 1;
+  for (int a = 0; a < 3; ++a) {
+    want[a] = full[a];
+    while (want[a] > 1 && ng % want[a]) want[a] /= 2;
+    divides = divides && want[a] == full[a];
+    cells *= want[a];
+  }
+  if (!make_tile_geom(ng, full[0], full[1], full[2], t, true)) return false;
+  if (!divides && cells >= 512 && t->ntiles < 512) return make_tile_geom(ng, want[0], want[1], want[2], t);
+  return true;
 }
 
 int bin_alloc(BinBuffers* b, const TileGeom& t, long long np)

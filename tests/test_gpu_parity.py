@@ -174,6 +174,31 @@ def test_deposit_tiny_tiles_overflow_workgroup_table(eh_table, clustered):
     assert np.abs(grids[0][:, :, :ng] - ref[:, :, :ng]).max() <= 1e-5 * np.abs(ref[:, :, :ng]).max()
 
 
+@pytest.mark.parametrize("ng", [6, 10, 18, 36, 50, 54, 90])
+def test_deposit_ragged_default_tiles(eh_table, ng):
+    """Grids that the default 8 x 8 x 32 tile does not divide end in partial
+    tiles (widths 2, 4, 6 along x and y, every residue along z): the density
+    equals that of 2 x 1 x 1 tiles bit for bit and the oracle's to the
+    deposit's bound, particles at the faces and beyond the ghost threshold
+    included."""
+    nc, box = 12, 48.0
+    _say(f"deposit ragged tiles ng={ng}")
+    parts = _random_particles(nc, box, 7 + ng, edge_cases=True)
+    wpar = float(np.float32((ng / nc) ** 3))
+    with _context(nc, ng, box, eh_table) as ctx:
+        grids = []
+        for tile in (None, (2, 1, 1)):
+            if tile:
+                ctx.set_tiling(*tile)
+            ctx.set_particles(parts, 0.5, 0.55)
+            ctx.pm_assign()
+            grids.append(ctx.get_density())
+    assert np.array_equal(grids[0], grids[1])
+    ref = np.zeros(orc.padded_real_shape(ng), np.float32)
+    orc.lib().orc_pm_deposit(ng, box, wpar, parts.ctypes.data, len(parts), ref.ctypes.data)
+    assert np.abs(grids[0][:, :, :ng] - ref[:, :, :ng]).max() <= 1e-5 * np.abs(ref[:, :, :ng]).max()
+
+
 # ---------------------------------------------------------------- force
 @pytest.mark.parametrize("nc,ng,box", [(16, 48, 64.0), (32, 96, 100.0), (24, 36, 80.0)])
 def test_force_matches_oracle(eh_table, nc, ng, box):
