@@ -15,12 +15,6 @@ struct PosSource {
   long long np = 0;
 };
 
-// coarse_grid.c:95-121 on an n^3 grid: zero `fix` (n^3 cells, C order),
-// then add every particle's eight CIC weights with periodic wrap as 32.32
-// fixed-point integers (exact for weights >= 2^-9), so the sums do not depend
-// on the order of the atomics and the grid is bit-reproducible.
-int launch_cic_periodic(const PosSource& src, int n, float boxsize, unsigned long long* fix, hipStream_t s);
-
 // coarse_grid.c:59-70: rho = (float) fixed-point sum, grid = nbar_inv * rho - 1
 // (float, as the reference), written to a grid with rows of `row` floats (n
 // for the C-order file layout, 2(n/2+1) for an in-place r2c).  sums[0] += sum
@@ -46,5 +40,6 @@ int launch_power_shells(int n, const float2* delta_k, const ShellBins& b, double
 // Fill n floats / doubles with zero (a kernel, so the call may be captured).
 int launch_fill_zero(float* p, long long n, hipStream_t s);
 int launch_fill_zero(double* p, long long n, hipStream_t s);
+int launch_fill_zero(unsigned long long* p, long long n, hipStream_t s);
 
 }  // namespace cola

@@ -15,46 +15,7 @@ __device__ inline double wave_sum_d(double v)
   return v;
 }
 
-constexpr float kFix = 4294967296.0f;  // 2^32
-constexpr double kUnfix = 1.0 / 4294967296.0;
-
-__device__ inline void add_fix(unsigned long long* cell, float w)
-{
-  atomicAdd(cell, (unsigned long long)rintf(w * kFix));
-}
-
-// coarse_grid.c:95-121.  One thread per particle; the index arithmetic and
-// the weight products follow the reference term by term: X = x * dx_inv in
-// float, ix = floor(X), w = 1 - (X - ix), neighbours (ix + nc) % nc and
-// (ix + 1 + nc) % nc (computed here with a modulo that also holds below -nc,
-// where the reference would index out of bounds).
-__global__ void __launch_bounds__(kThreads)
-k_cic_periodic(PosSource src, int n, float dx_inv, unsigned long long* __restrict__ fix)
-{
-  const long long i = (long long)blockIdx.x * kThreads + threadIdx.x;
-  if (i >= src.np) return;
-  int i0[3], i1[3];
-  float w[3];
-  for (int j = 0; j < 3; ++j) {
-    const float X = src.x[j][i * src.stride] * dx_inv;
-    const int ix = (int)floorf(X);
-    w[j] = 1.0f - (X - (float)ix);
-    int m = ix % n;
-    if (m < 0) m += n;
-    i0[j] = m;
-    i1[j] = m + 1 == n ? 0 : m + 1;
-  }
-  const long long r00 = ((long long)i0[0] * n + i0[1]) * n, r01 = ((long long)i0[0] * n + i1[1]) * n;
-  const long long r10 = ((long long)i1[0] * n + i0[1]) * n, r11 = ((long long)i1[0] * n + i1[1]) * n;
-  add_fix(&fix[r00 + i0[2]], w[0] * w[1] * w[2]);
-  add_fix(&fix[r01 + i0[2]], w[0] * (1 - w[1]) * w[2]);
-  add_fix(&fix[r00 + i1[2]], w[0] * w[1] * (1 - w[2]));
-  add_fix(&fix[r01 + i1[2]], w[0] * (1 - w[1]) * (1 - w[2]));
-  add_fix(&fix[r10 + i0[2]], (1 - w[0]) * w[1] * w[2]);
-  add_fix(&fix[r11 + i0[2]], (1 - w[0]) * (1 - w[1]) * w[2]);
-  add_fix(&fix[r10 + i1[2]], (1 - w[0]) * w[1] * (1 - w[2]));
-  add_fix(&fix[r11 + i1[2]], (1 - w[0]) * (1 - w[1]) * (1 - w[2]));
-}
+constexpr double kUnfix = 1.0 / 4294967296.0;  // the sums are 32.32 fixed point
 
 // coarse_grid.c:63-68: delta = nbar_inv * rho - 1 (float), with the double
 // sums of rho and delta.  Cell c of the n^3 grid goes to (c / n) * row + c % n.
@@ -166,20 +127,11 @@ int launch_fill_zero(double* p, long long n, hipStream_t s)
   return kOk;
 }
 
-int launch_cic_periodic(const PosSource& src, int n, float boxsize, unsigned long long* fix, hipStream_t s)
+int launch_fill_zero(unsigned long long* p, long long n, hipStream_t s)
 {
-  if (n < 1) {
-    set_error("coarse grid: invalid grid size");
-    return kErrArg;
-  }
-  const long long ncell = (long long)n * n * n;
-  hipLaunchKernelGGL(k_fill_zero<unsigned long long>, dim3(capped_blocks(ncell, kThreads * 8LL, 65536)),
-                     dim3(kThreads), 0, s, fix, ncell);
-  COLA_HIP(hipGetLastError());
-  if (src.np == 0) return kOk;
-  const float dx_inv = n / boxsize;  // coarse_grid.c:99
-  hipLaunchKernelGGL(k_cic_periodic, dim3((unsigned)((src.np + kThreads - 1) / kThreads)), dim3(kThreads), 0, s, src,
-                     n, dx_inv, fix);
+  if (n <= 0) return kOk;
+  hipLaunchKernelGGL(k_fill_zero<unsigned long long>, dim3(capped_blocks(n, kThreads * 8LL, 65536)), dim3(kThreads),
+                     0, s, p, n);
   COLA_HIP(hipGetLastError());
   return kOk;
 }

@@ -78,6 +78,9 @@ struct EventPair {
 
 using namespace cola;
 
+// Largest grid of cola_coarse_grid_noalloc.
+constexpr int kNoAllocGrid = 128;
+
 struct cola_context {
   int nc = 0, ng = 0;
   double boxsize = 0;
@@ -139,6 +142,7 @@ struct cola_context {
   long long aux_floats = 0;
   unsigned long long* aux_fix = nullptr;  // fixed-point CIC sums, n^3
   long long aux_fix_cells = 0;
+  GridBins grid_bins;  // tile counters of the output grids
   FftPlan aux_fft;
   int aux_fft_n = 0;
   double* d_aux = nullptr;  // 2 sums + 3 * kMaxShellBins shell accumulators
@@ -491,6 +495,7 @@ int cola_context_create(int nc, int ngrid, double boxsize, cola_context** out)
   }
   st = bin_alloc(&c->bins, c->tiles, c->np);
   if (st) return fail(kErrAlloc);
+  if (grid_bin_alloc(&c->grid_bins, kNoAllocGrid)) return fail(kErrAlloc);
   if (hipMalloc(&c->d_mass, sizeof(double) * cola_context::kMassSlots) != hipSuccess) return fail(kErrAlloc);
   if (hipMemset(c->d_mass, 0, sizeof(double) * cola_context::kMassSlots) != hipSuccess) return fail(kErrHip);
   if (hipHostMalloc(&c->h_prm, sizeof(StepParams) * cola_context::kMassSlots) != hipSuccess) return fail(kErrAlloc);
@@ -533,6 +538,7 @@ int cola_context_destroy(cola_context* c)
   fof_free(&c->fof);
   if (c->aux_grid) (void)hipFree(c->aux_grid);
   if (c->aux_fix) (void)hipFree(c->aux_fix);
+  grid_bin_free(&c->grid_bins);
   if (c->d_aux) (void)hipFree(c->d_aux);
   if (c->stream) (void)hipStreamDestroy(c->stream);
   delete c;
@@ -1743,8 +1749,11 @@ int position_source(cola_context* c, int source, PosSource* src)
   return kOk;
 }
 
-int ensure_aux(cola_context* c, long long floats, long long cells)
+// Buffers of an output grid of n^3 cells held in `floats` floats.
+int ensure_aux(cola_context* c, int n, long long floats)
 {
+  const long long cells = grid_split(n, c->np) > 1 ? (long long)n * n * n : 0;
+  COLA_TRY(grid_bin_alloc(&c->grid_bins, n));
   if (!c->d_aux) COLA_HIP(hipMalloc(&c->d_aux, sizeof(double) * (2 + 3 * kMaxShellBins)));
   if (c->aux_floats < floats) {
     if (c->aux_grid) (void)hipFree(c->aux_grid);
@@ -1771,13 +1780,15 @@ int ensure_aux(cola_context* c, long long floats, long long cells)
   return kOk;
 }
 
-// coarse_grid.c:49-68 on the device: CIC assignment, then delta = rho n^3 / np - 1.
-int deposit_contrast(cola_context* c, const PosSource& src, int n, long long row)
+// coarse_grid.c:49-68 on the device: CIC assignment, then delta = rho n^3 / np
+// - 1.  The particles are sorted in the PM bins' buffer, which is free between
+// the forces of the context's stream.
+int deposit_contrast(cola_context* c, const PosSource& src, int n, long long row, unsigned long long* fix, float* grid,
+                     double* sums)
 {
-  COLA_TRY(launch_cic_periodic(src, n, c->boxf, c->aux_fix, c->stream));
-  COLA_TRY(launch_fill_zero(c->d_aux, 2, c->stream));
   const float nbar_inv = (double)n * n * n / (double)c->np;  // coarse_grid.c:56
-  return launch_density_contrast(n, row, nbar_inv, c->aux_fix, c->aux_grid, c->d_aux, c->stream);
+  return launch_grid_contrast(src, n, c->boxf, c->grid_bins, c->bins.sorted, c->bins.capacity, c->bins.overflow, fix,
+                              row, nbar_inv, grid, sums, c->stream);
 }
 
 }  // namespace
@@ -1789,7 +1800,6 @@ int deposit_contrast(cola_context* c, const PosSource& src, int n, long long row
 // code never passes the array's name to a kernel: it passes the device
 // address hipGetSymbolAddress returns for the current device
 // (noalloc_scratch()).
-constexpr int kNoAllocGrid = 128;
 constexpr long long kNoAllocCells = (long long)kNoAllocGrid * kNoAllocGrid * kNoAllocGrid;
 static __device__ __align__(256) unsigned long long scratch[kNoAllocCells + 32];
 
@@ -1833,8 +1843,8 @@ int cola_coarse_grid(cola_context* c, int n, int source, float* delta_out, doubl
   PosSource src;
   COLA_TRY(position_source(c, source, &src));
   const long long ncell = (long long)n * n * n;
-  COLA_TRY(ensure_aux(c, ncell, ncell));
-  COLA_TRY(deposit_contrast(c, src, n, n));
+  COLA_TRY(ensure_aux(c, n, ncell));
+  COLA_TRY(deposit_contrast(c, src, n, n, c->aux_fix, c->aux_grid, c->d_aux));
   double sums[2] = {0, 0};
   COLA_HIP(hipMemcpyAsync(delta_out, c->aux_grid, sizeof(float) * ncell, hipMemcpyDeviceToHost, c->stream));
   COLA_HIP(hipMemcpyAsync(sums, c->d_aux, sizeof(sums), hipMemcpyDeviceToHost, c->stream));
@@ -1864,11 +1874,9 @@ int cola_coarse_grid_noalloc(cola_context* c, int n, int source, float* delta_de
   COLA_TRY(noalloc_scratch(&fix));
   double* sums = sums_dev ? sums_dev : reinterpret_cast<double*>(fix + kNoAllocCells);
   // the same kernels as cola_coarse_grid; the accumulators and sums are
-  // cleared by fill kernels on the context's stream
-  COLA_TRY(launch_cic_periodic(src, n, c->boxf, fix, c->stream));
-  COLA_TRY(launch_fill_zero(sums, 2, c->stream));
-  const float nbar_inv = (double)n * n * n / (double)c->np;  // coarse_grid.c:56
-  return launch_density_contrast(n, n, nbar_inv, fix, delta_dev, sums, c->stream);
+  // cleared by fill kernels on the context's stream, the tile counters are
+  // the context's (made with it, for grids of up to kNoAllocGrid)
+  return deposit_contrast(c, src, n, n, fix, delta_dev, sums);
 }
 
 int cola_power_spectrum(cola_context* c, int n, int source, double kmin, double kmax, int nbins, int flags,
@@ -1892,8 +1900,8 @@ int cola_power_spectrum(cola_context* c, int n, int source, double kmin, double 
     c->aux_fft_n = n;
   }
   const long long row = 2LL * (n / 2 + 1);
-  COLA_TRY(ensure_aux(c, (long long)n * n * row, (long long)n * n * n));
-  COLA_TRY(deposit_contrast(c, src, n, row));
+  COLA_TRY(ensure_aux(c, n, (long long)n * n * row));
+  COLA_TRY(deposit_contrast(c, src, n, row, c->aux_fix, c->aux_grid, c->d_aux));
   COLA_TRY(c->aux_fft.r2c(c->aux_grid, c->stream));
   ShellBins b;
   b.kmin = kmin;

@@ -4,6 +4,7 @@
 
 #include <hip/hip_runtime.h>
 
+#include "analysis.h"
 #include "cosmo.h"
 
 namespace cola {
@@ -87,6 +88,25 @@ struct StepParams {
 int launch_deposit_tiles(const CicGeom& g, const TileGeom& t, const BinBuffers& b, float* density, double* ring,
                          const StepParams* prm, hipStream_t s);
 int launch_zero_mass(double* ring, const StepParams* prm, hipStream_t s);
+// Output grids (coarse_grid.c:95-121): counters and offsets of their tiles.
+struct GridBins {
+  int* counts = nullptr;  // tiles (zero between calls), then tiles + 1 offsets, then the scan's sums
+  long long tiles = 0;
+};
+TileGeom grid_tile_geom(int n);
+int grid_bin_alloc(GridBins* b, int n);  // at least the tiles of an n^3 grid (keeps what is large enough)
+void grid_bin_free(GridBins* b);
+// Workgroups that share a tile's particles: above 1 the grid needs the
+// fixed-point sums fix[n^3], at 1 none.
+int grid_split(int n, long long np);
+// coarse_grid.c:49-70 on n^3 cells: counting sort of the positions into tiles
+// (sorted: scratch of `capacity` >= 8 np entries of three floats), CIC sums
+// in LDS, grid = nbar_inv * rho - 1 with rows of `row` floats, sums = the
+// sums of rho and of delta.  Kernels only.
+int launch_grid_contrast(const PosSource& src, int n, float boxsize, const GridBins& b, float* sorted,
+                         long long capacity, int* overflow, unsigned long long* fix, long long row, float nbar_inv,
+                         float* grid, double* sums, hipStream_t s);
+
 // pm.c:359-412 + 505-532: readout of the three force grids into p.f.
 // fsum: null, or the three sums of a residual added to the force grids,
 // whose mean is taken off every particle's force.  fi: null (gather from

@@ -11,10 +11,12 @@
 // (pm.c:416-502, 505-532) is reproduced exactly: a particle with
 // x > L - L/Ng also deposits (and reads back) through a copy at x - L whose
 // weights are recomputed from that shifted position.
+#include "analysis.h"
 #include "common.h"
 #include "pm.h"
 
 #include <algorithm>
+#include <type_traits>
 #include <vector>
 
 namespace cola {
@@ -150,6 +152,37 @@ __device__ inline int span_key(const TileSpan& s, const TileGeom& t, int k)
   return (a * t.nty + b) * t.ntz + c;
 }
 
+// ---- output grids (coarse_grid.c:95-121) -------------------------------------
+// One axis of a position's periodic CIC: X = x * dx_inv in float, ix =
+// floor(X), the two cells ix and ix + 1 modulo n (any ix), the weight of the
+// first.
+struct GridGeom {
+  int n;
+  float dx_inv;  // coarse_grid.c:99  n / boxsize
+};
+
+struct GridAxis {
+  int i0, i1;
+  float w;
+};
+
+__device__ inline GridAxis grid_axis(float x, const GridGeom& g)
+{
+  const float X = x * g.dx_inv;
+  const int ix = (int)floorf(X);
+  GridAxis a;
+  a.w = 1.0f - (X - (float)ix);
+  // most positions lie within a period of the grid: no division for them
+  int m = ix < 0 ? ix + g.n : ix >= g.n ? ix - g.n : ix;
+  if (m < 0 || m >= g.n) {
+    m = ix % g.n;
+    if (m < 0) m += g.n;
+  }
+  a.i0 = m;
+  a.i1 = m + 1 == g.n ? 0 : m + 1;
+  return a;
+}
+
 __device__ inline void wrap1(float& x, float L)
 {
   if (x < 0.0f)
@@ -245,11 +278,44 @@ __device__ inline LaneRun lane_run(int key, bool active)
 // lane of a workgroup's chunk keeps adjacent lanes on adjacent particles.
 constexpr int kBinPer = 4;
 
+// What the binning bins: the particles of a PM deposit, or the positions of
+// an output grid (wrapped periodically, whatever their range).
+struct PmBin {
+  const DevParticles& p;
+  const CicGeom& g;
+  const TileGeom& t;
+  __device__ long long np() const { return p.np; }
+  __device__ float at(int a, long long i) const { return p.x[a][i]; }
+  __device__ void put(int a, long long i, float v) const { p.x[a][i] = v; }
+  __device__ bool span(float x, float y, float z, TileSpan& s) const { return tile_span(x, y, z, g, t, s); }
+};
+
+template <int STRIDE>
+struct GridBin {
+  const PosSource& src;
+  const GridGeom& g;
+  const TileGeom& t;
+  __device__ long long np() const { return src.np; }
+  __device__ float at(int a, long long i) const { return src.x[a][i * STRIDE]; }
+  __device__ void put(int, long long, float) const {}
+  __device__ bool span(float x, float y, float z, TileSpan& s) const
+  {
+    const GridAxis ax = grid_axis(x, g), ay = grid_axis(y, g), az = grid_axis(z, g);
+    s.x0 = min(ax.i0, ax.i1) >> t.lx;
+    s.x1 = max(ax.i0, ax.i1) >> t.lx;
+    s.y0 = min(ay.i0, ay.i1) >> t.ly;
+    s.y1 = max(ay.i0, ay.i1) >> t.ly;
+    s.z0 = min(az.i0, az.i1) >> t.lz;
+    s.z1 = max(az.i0, az.i1) >> t.lz;
+    return true;
+  }
+};
+
 // Block blk of the counting pass (the kernels below run it for their own
 // block index or for a block of one member of a batched launch).
-__device__ __forceinline__ void bin_count_block(const DevParticles& p, const CicGeom& g, const TileGeom& t,
-                                                int* __restrict__ counts, int* __restrict__ overflow, int wrap_first,
-                                                float L, long long blk)
+template <class B>
+__device__ __forceinline__ void bin_count_block(const B& b, const TileGeom& t, int* __restrict__ counts,
+                                                int* __restrict__ overflow, int wrap_first, float L, long long blk)
 {
   __shared__ BinHash h;
   float px[kBinPer], py[kBinPer], pz[kBinPer];
@@ -257,10 +323,10 @@ __device__ __forceinline__ void bin_count_block(const DevParticles& p, const Cic
 #pragma unroll
   for (int q = 0; q < kBinPer; ++q) {
     const long long i = (blk * kBinPer + q) * kThreads + threadIdx.x;
-    live[q] = i < p.np;
-    px[q] = live[q] ? p.x[0][i] : 0.0f;
-    py[q] = live[q] ? p.x[1][i] : 0.0f;
-    pz[q] = live[q] ? p.x[2][i] : 0.0f;
+    live[q] = i < b.np();
+    px[q] = live[q] ? b.at(0, i) : 0.0f;
+    py[q] = live[q] ? b.at(1, i) : 0.0f;
+    pz[q] = live[q] ? b.at(2, i) : 0.0f;
   }
   hash_clear(h);
   TileSpan ts[kBinPer];
@@ -275,11 +341,11 @@ __device__ __forceinline__ void bin_count_block(const DevParticles& p, const Cic
         wrap1(x, L);
         wrap1(y, L);
         wrap1(z, L);
-        if (x != px[q]) p.x[0][i] = x;
-        if (y != py[q]) p.x[1][i] = y;
-        if (z != pz[q]) p.x[2][i] = z;
+        if (x != px[q]) b.put(0, i, x);
+        if (y != py[q]) b.put(1, i, y);
+        if (z != pz[q]) b.put(2, i, z);
       }
-      if (!tile_span(x, y, z, g, t, ts[q])) atomicOr(overflow, 1);
+      if (!b.span(x, y, z, ts[q])) atomicOr(overflow, 1);
       nk[q] = span_count(ts[q]);
     }
   }
@@ -311,7 +377,7 @@ __global__ void __launch_bounds__(kThreads)
 k_bin_count(DevParticles p, CicGeom g, TileGeom t, int* __restrict__ counts, int* __restrict__ overflow, int wrap_first,
             float L)
 {
-  bin_count_block(p, g, t, counts, overflow, wrap_first, L, blockIdx.x);
+  bin_count_block(PmBin{p, g, t}, t, counts, overflow, wrap_first, L, blockIdx.x);
 }
 
 // Claims the entries' slots by counting each tile's counter back down to zero
@@ -319,10 +385,10 @@ k_bin_count(DevParticles p, CicGeom g, TileGeom t, int* __restrict__ counts, int
 // counter's value c, and its entry of rank r in the tile gets position
 // offsets[tile] + c - 1 - r.  Entries that found no table slot claim theirs
 // one by one from the counter.
-__device__ __forceinline__ void bin_scatter_block(const DevParticles& p, const CicGeom& g, const TileGeom& t,
-                                                  int* __restrict__ counts, const int* __restrict__ offsets,
-                                                  float* __restrict__ sorted, long long capacity,
-                                                  int* __restrict__ overflow, long long blk)
+template <class B>
+__device__ __forceinline__ void bin_scatter_block(const B& b, const TileGeom& t, int* __restrict__ counts,
+                                                  const int* __restrict__ offsets, float* __restrict__ sorted,
+                                                  long long capacity, int* __restrict__ overflow, long long blk)
 {
   __shared__ BinHash h;
   __shared__ long long base[kHashSlots];
@@ -331,10 +397,10 @@ __device__ __forceinline__ void bin_scatter_block(const DevParticles& p, const C
 #pragma unroll
   for (int q = 0; q < kBinPer; ++q) {
     const long long i = (blk * kBinPer + q) * kThreads + threadIdx.x;
-    live[q] = i < p.np;
-    px[q] = live[q] ? p.x[0][i] : 0.0f;
-    py[q] = live[q] ? p.x[1][i] : 0.0f;
-    pz[q] = live[q] ? p.x[2][i] : 0.0f;
+    live[q] = i < b.np();
+    px[q] = live[q] ? b.at(0, i) : 0.0f;
+    py[q] = live[q] ? b.at(1, i) : 0.0f;
+    pz[q] = live[q] ? b.at(2, i) : 0.0f;
   }
   hash_clear(h);
   TileSpan ts[kBinPer];
@@ -343,7 +409,7 @@ __device__ __forceinline__ void bin_scatter_block(const DevParticles& p, const C
   for (int q = 0; q < kBinPer; ++q) {
     nk[q] = 0;
     if (live[q]) {
-      tile_span(px[q], py[q], pz[q], g, t, ts[q]);
+      b.span(px[q], py[q], pz[q], ts[q]);
       nk[q] = span_count(ts[q]);
     }
   }
@@ -364,14 +430,14 @@ __device__ __forceinline__ void bin_scatter_block(const DevParticles& p, const C
         const bool act = k < nk[q];
         const int key = act ? span_key(ts[q], t, k) : 0;
         const LaneRun run = lane_run(key, act);
-        int sl = -1, b = 0;
+        int sl = -1, rank = 0;
         if (run.is_head) {
           sl = hash_slot(h, key);
-          if (sl >= 0) b = atomicAdd(&h.cnt[sl], run.len);
+          if (sl >= 0) rank = atomicAdd(&h.cnt[sl], run.len);
         }
         sl = __shfl(sl, run.head);
-        b = __shfl(b, run.head);
-        if (sl >= 0) code[q][k] = sl << 16 | (b + lane - run.head);
+        rank = __shfl(rank, run.head);
+        if (sl >= 0) code[q][k] = sl << 16 | (rank + lane - run.head);
       }
     }
   }
@@ -409,7 +475,7 @@ __global__ void __launch_bounds__(kThreads)
 k_bin_scatter(DevParticles p, CicGeom g, TileGeom t, int* __restrict__ counts, const int* __restrict__ offsets,
               float* __restrict__ sorted, long long capacity, int* __restrict__ overflow)
 {
-  bin_scatter_block(p, g, t, counts, offsets, sorted, capacity, overflow, blockIdx.x);
+  bin_scatter_block(PmBin{p, g, t}, t, counts, offsets, sorted, capacity, overflow, blockIdx.x);
 }
 
 // ---- exclusive scan of the tile counts -------------------------------------
@@ -618,6 +684,114 @@ __global__ void __launch_bounds__(kThreads)
 k_sum_doubles(const double* __restrict__ v, long long n, double* ring, const StepParams* __restrict__ prm)
 {
   sum_doubles_block(v, n, ring, prm, blockIdx.x);
+}
+
+// ---- output grids: one workgroup per tile, or several -----------------------
+// The eight weights of coarse_grid.c:103-120 of the entries [beg, end) added
+// to the tile's LDS cells (fixed point as above, so the grid is the same bit
+// for bit however its particles are shared out).
+//
+// One 64-bit global atomic per weight made the grid of 256^3 particles cost
+// 5.2 ms (256^3 cells) and of 512^3 particles 39 ms (128^3 cells), bound by
+// the L2's atomics.  Binned into tiles like the PM deposit, the weights are
+// added in LDS and a cell is written once: 1.57 ms at 256^3 (count .47,
+// scatter .54, tiles .57) and 4.6 ms.  The floor, positions read and cells
+// written once, is 0.05 and 0.34 ms; the rest is the sort and, on coarse
+// grids, lanes of a wavefront adding to the same cells.
+__device__ __forceinline__ void grid_tile_add(const GridGeom& g, const TileGeom& t, const float* __restrict__ sorted,
+                                              int beg, int end, int x0, int y0, int z0, unsigned long long* cells)
+{
+  for (int k = beg + (int)threadIdx.x; k < end; k += kDepositThreads) {
+    const GridAxis ax = grid_axis(sorted[3LL * k + 0], g), ay = grid_axis(sorted[3LL * k + 1], g),
+                   az = grid_axis(sorted[3LL * k + 2], g);
+    auto add = [&](int i, int j, int kk, float w) {
+      const unsigned li = (unsigned)(i - x0), lj = (unsigned)(j - y0), lk = (unsigned)(kk - z0);
+      if (li < (unsigned)t.tx && lj < (unsigned)t.ty && lk < (unsigned)t.tz)
+        atomicAdd(&cells[(((li << t.ly) + lj) << t.lz) + lk], (unsigned long long)rintf(w * kFix));
+    };
+    add(ax.i0, ay.i0, az.i0, ax.w * ay.w * az.w);
+    add(ax.i0, ay.i1, az.i0, ax.w * (1 - ay.w) * az.w);
+    add(ax.i0, ay.i0, az.i1, ax.w * ay.w * (1 - az.w));
+    add(ax.i0, ay.i1, az.i1, ax.w * (1 - ay.w) * (1 - az.w));
+    add(ax.i1, ay.i0, az.i0, (1 - ax.w) * ay.w * az.w);
+    add(ax.i1, ay.i1, az.i0, (1 - ax.w) * (1 - ay.w) * az.w);
+    add(ax.i1, ay.i0, az.i1, (1 - ax.w) * ay.w * (1 - az.w));
+    add(ax.i1, ay.i1, az.i1, (1 - ax.w) * (1 - ay.w) * (1 - az.w));
+  }
+}
+
+// SPLIT false: a workgroup owns a tile and writes its contrast (the value and
+// the sums of k_density_contrast).  SPLIT true: nsplit workgroups share a
+// tile's particles and add their cells to the fixed-point grid fix[n^3].
+template <bool SPLIT>
+__global__ void __launch_bounds__(kDepositThreads)
+k_grid_tiles(GridGeom g, TileGeom t, const int* __restrict__ offsets, const float* __restrict__ sorted, int nsplit,
+             long long row, float nbar_inv, unsigned long long* __restrict__ fix, float* __restrict__ grid,
+             double* __restrict__ sums)
+{
+  extern __shared__ unsigned long long cells[];
+  const int tile = SPLIT ? (int)(blockIdx.x / (unsigned)nsplit) : (int)blockIdx.x;
+  const int tz = tile % t.ntz, ty = (tile / t.ntz) % t.nty, tx = tile / (t.ntz * t.nty);
+  const int x0 = tx << t.lx, y0 = ty << t.ly, z0 = tz << t.lz;
+  const int ncell = 1 << (t.lx + t.ly + t.lz);
+  int beg = offsets[tile], end = offsets[tile + 1];
+  if (SPLIT) {
+    const int part = (int)(blockIdx.x % (unsigned)nsplit);
+    const int len = (end - beg + nsplit - 1) / nsplit;
+    beg = min(end, beg + part * len);
+    end = min(end, beg + len);
+    if (beg >= end) return;
+  }
+  for (int e = threadIdx.x; e < ncell; e += kDepositThreads) cells[e] = 0ULL;
+  __syncthreads();
+  grid_tile_add(g, t, sorted, beg, end, x0, y0, z0, cells);
+  __syncthreads();
+  const int zmask = t.tz - 1, ymask = t.ty - 1;
+  double s_in = 0.0, s_out = 0.0;
+  for (int e = threadIdx.x; e < ncell; e += kDepositThreads) {
+    const int k = z0 + (e & zmask), j = y0 + ((e >> t.lz) & ymask), i = x0 + (e >> (t.lz + t.ly));
+    if (i >= g.n || j >= g.n || k >= g.n) continue;
+    const long long line = (long long)i * g.n + j;
+    if (SPLIT) {
+      if (cells[e]) atomicAdd(&fix[line * g.n + k], cells[e]);
+    } else {
+      const float rho = (float)((double)cells[e] * kUnfix);
+      const float d = nbar_inv * rho - 1.0f;
+      grid[line * row + k] = d;
+      s_in += (double)rho;
+      s_out += (double)d;
+    }
+  }
+  if (!SPLIT) {
+    __shared__ double part[2][kDepositThreads / 64];
+    s_in = wave_sum(s_in);
+    s_out = wave_sum(s_out);
+    if (__lane_id() == 0) {
+      part[0][threadIdx.x >> 6] = s_in;
+      part[1][threadIdx.x >> 6] = s_out;
+    }
+    __syncthreads();
+    if (threadIdx.x < 2) {
+      double tot = 0.0;
+      for (int w = 0; w < kDepositThreads / 64; ++w) tot += part[threadIdx.x][w];
+      unsafeAtomicAdd(&sums[threadIdx.x], tot);
+    }
+  }
+}
+
+template <int STRIDE>
+__global__ void __launch_bounds__(kThreads)
+k_grid_count(PosSource src, GridGeom g, TileGeom t, int* __restrict__ counts)
+{
+  bin_count_block(GridBin<STRIDE>{src, g, t}, t, counts, nullptr, 0, 0.0f, blockIdx.x);
+}
+
+template <int STRIDE>
+__global__ void __launch_bounds__(kThreads)
+k_grid_scatter(PosSource src, GridGeom g, TileGeom t, int* __restrict__ counts, const int* __restrict__ offsets,
+               float* __restrict__ sorted, long long capacity, int* __restrict__ overflow)
+{
+  bin_scatter_block(GridBin<STRIDE>{src, g, t}, t, counts, offsets, sorted, capacity, overflow, blockIdx.x);
 }
 
 // ---- readout (pm.c:359-412) -------------------------------------------------
@@ -893,7 +1067,8 @@ k_bin_count_batch(const PmMember* __restrict__ ms, const int* __restrict__ start
 {
   const int m = batch_find(start, n, blockIdx.x);
   const PmMember& M = ms[m];
-  bin_count_block(M.p, M.g, M.t, M.b.counts, M.b.overflow, 1, M.boxsize, (long long)blockIdx.x - start[m]);
+  bin_count_block(PmBin{M.p, M.g, M.t}, M.t, M.b.counts, M.b.overflow, 1, M.boxsize,
+                  (long long)blockIdx.x - start[m]);
 }
 
 __global__ void __launch_bounds__(kThreads)
@@ -924,7 +1099,7 @@ k_bin_scatter_batch(const PmMember* __restrict__ ms, const int* __restrict__ sta
 {
   const int m = batch_find(start, n, blockIdx.x);
   const PmMember& M = ms[m];
-  bin_scatter_block(M.p, M.g, M.t, M.b.counts, M.b.offsets, M.b.sorted, M.b.capacity, M.b.overflow,
+  bin_scatter_block(PmBin{M.p, M.g, M.t}, M.t, M.b.counts, M.b.offsets, M.b.sorted, M.b.capacity, M.b.overflow,
                     (long long)blockIdx.x - start[m]);
 }
 
@@ -1102,6 +1277,102 @@ int launch_deposit_tiles(const CicGeom& g, const TileGeom& t, const BinBuffers& 
   const long long per = (long long)kThreads * 16;
   hipLaunchKernelGGL(k_sum_doubles, dim3((unsigned)((t.ntiles + per - 1) / per)), dim3(kThreads), 0, s, b.tile_sums,
                      t.ntiles, ring, prm);
+  COLA_HIP(hipGetLastError());
+  return kOk;
+}
+
+TileGeom grid_tile_geom(int n)
+{
+  TileGeom t;
+  t.ntx = (n + t.tx - 1) / t.tx;
+  t.nty = (n + t.ty - 1) / t.ty;
+  t.ntz = (n + t.tz - 1) / t.tz;
+  t.ntiles = (long long)t.ntx * t.nty * t.ntz;
+  return t;
+}
+
+int grid_bin_alloc(GridBins* b, int n)
+{
+  const TileGeom t = grid_tile_geom(n);
+  if (t.ntiles * kDepositThreads > 0xffffffffLL) {  // one launch's threads: n > 3200, where a grid's sums exceed the HBM
+    set_error("unable to allocate the output grid");
+    return kErrAlloc;
+  }
+  if (b->tiles >= t.ntiles) return kOk;
+  grid_bin_free(b);
+  const long long nsums = (t.ntiles + kScanChunk - 1) / kScanChunk;
+  if (hipMalloc(&b->counts, sizeof(int) * (2 * t.ntiles + nsums + 2)) != hipSuccess) {
+    (void)hipGetLastError();
+    b->counts = nullptr;
+    set_error("unable to allocate the output grid");
+    return kErrAlloc;
+  }
+  COLA_HIP(hipMemset(b->counts, 0, sizeof(int) * t.ntiles));
+  b->tiles = t.ntiles;
+  return kOk;
+}
+
+void grid_bin_free(GridBins* b)
+{
+  if (b->counts) (void)hipFree(b->counts);
+  *b = GridBins{};
+}
+
+// Particles of a tile that one workgroup takes alone: above, the tiles are
+// few for the particles (a coarse grid of a large run) and each is shared.
+// One workgroup per tile against shares of 4096, 256^3 particles: 8^3 cells
+// 111.6 -> 0.85 ms, 32^3 7.38 -> 0.95, 64^3 1.85 -> 1.01, 100^3 0.99 -> 0.79;
+// 64^3 particles on 7^3 1.27 -> 0.06 ms.  Shares of 65536 were slower (0.93,
+// 1.24, 1.32, 1.00, 0.36 ms), 8192 and 16384 in between.
+constexpr long long kGridTileShare = 4096;
+
+int grid_split(int n, long long np)
+{
+  const long long per = np / grid_tile_geom(n).ntiles;
+  return (int)std::min<long long>(1024, (per + kGridTileShare - 1) / kGridTileShare);
+}
+
+int launch_grid_contrast(const PosSource& src, int n, float boxsize, const GridBins& b, float* sorted,
+                         long long capacity, int* overflow, unsigned long long* fix, long long row, float nbar_inv,
+                         float* grid, double* sums, hipStream_t s)
+{
+  GridGeom g;
+  g.n = n;
+  g.dx_inv = n / boxsize;
+  const TileGeom t = grid_tile_geom(n);
+  if (n < 1 || t.ntiles > b.tiles || (src.stride != 1 && src.stride != 8)) {
+    set_error("coarse grid: invalid grid size");
+    return kErrArg;
+  }
+  BinBuffers bb;
+  bb.counts = b.counts;
+  bb.offsets = b.counts + b.tiles;
+  bb.block_sums = bb.offsets + b.tiles + 1;
+  const int nsplit = grid_split(n, src.np);
+  const unsigned nb = bin_blocks(src.np);
+  auto bin = [&](auto stride) {
+    constexpr int S = decltype(stride)::value;
+    hipLaunchKernelGGL(k_grid_count<S>, dim3(nb), dim3(kThreads), 0, s, src, g, t, bb.counts);
+    COLA_TRY(launch_bin_scan(t, bb, s));
+    hipLaunchKernelGGL(k_grid_scatter<S>, dim3(nb), dim3(kThreads), 0, s, src, g, t, bb.counts, bb.offsets, sorted,
+                       capacity, overflow);
+    return (int)kOk;
+  };
+  if (src.stride == 1)
+    COLA_TRY(bin(std::integral_constant<int, 1>{}));
+  else
+    COLA_TRY(bin(std::integral_constant<int, 8>{}));
+  const size_t lds = sizeof(unsigned long long) * t.tx * t.ty * t.tz;
+  COLA_TRY(launch_fill_zero(sums, 2, s));
+  if (nsplit <= 1) {
+    hipLaunchKernelGGL(k_grid_tiles<false>, dim3((unsigned)t.ntiles), dim3(kDepositThreads), lds, s, g, t, bb.offsets,
+                       sorted, 1, row, nbar_inv, fix, grid, sums);
+  } else {
+    COLA_TRY(launch_fill_zero(fix, (long long)n * n * n, s));
+    hipLaunchKernelGGL(k_grid_tiles<true>, dim3((unsigned)(t.ntiles * nsplit)), dim3(kDepositThreads), lds, s, g, t,
+                       bb.offsets, sorted, nsplit, row, nbar_inv, fix, grid, sums);
+    COLA_TRY(launch_density_contrast(n, row, nbar_inv, fix, grid, sums, s));
+  }
   COLA_HIP(hipGetLastError());
   return kOk;
 }

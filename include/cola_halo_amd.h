@@ -250,8 +250,9 @@ int cola_coarse_grid(cola_context* ctx, int n, int source, float* delta_out, dou
 
 /* No counterpart in the reference.  For callers that cannot allocate device
    memory (code under HIP graph capture, tight serving loops, harnesses that
-   forbid hipMalloc): cola_coarse_grid's kernels with the CIC accumulators in
-   a static device array of the library (16 MiB per GPU, held until the
+   forbid hipMalloc): cola_coarse_grid's kernels in the context's own buffers,
+   with the fixed-point sums of cells that several workgroups add to in a
+   static device array of the library (16 MiB per GPU, held until the
    process ends), so the call allocates nothing.  n <= 128 (COLA_ERR_ARG
    beyond).  delta_dev is DEVICE memory for n^3 floats (C order, as
    cola_coarse_grid's delta_out); sums_dev is NULL or DEVICE memory for the

@@ -118,3 +118,55 @@ def test_power_spectrum_of_initial_conditions_is_linear_theory(eh_table):
     ratio = pb / (d * d * plin)
     tol = 5 / np.sqrt(cnt / 2) + 0.03
     assert np.all(np.abs(ratio - 1) < tol), (ratio, tol)
+
+
+def _contrast_exact(x, n, box):
+    """coarse_grid.c:95-121 in float32, term by term, the weights summed as
+    32.32 fixed-point integers: the value of every cell, whatever the order."""
+    f = np.float32
+    i0, w = [], []
+    for a in range(3):
+        X = x[:, a] * (f(n) / f(box))
+        ix = np.floor(X)
+        w.append(f(1) - (X - ix))
+        i0.append(ix.astype(np.int64) % n)
+    fix = np.zeros((n, n, n), np.uint64)
+    for bx in (0, 1):
+        for by in (0, 1):
+            for bz in (0, 1):
+                wt = ((f(1) - w[0] if bx else w[0]) * (f(1) - w[1] if by else w[1])) * (f(1) - w[2] if bz else w[2])
+                np.add.at(fix, ((i0[0] + bx) % n, (i0[1] + by) % n, (i0[2] + bz) % n),
+                          np.rint(wt * f(2.0 ** 32)).astype(np.uint64))
+    rho = (fix.astype(np.float64) / 2.0 ** 32).astype(np.float32)
+    return f(float(n) ** 3 / len(x)) * rho - f(1)
+
+
+@pytest.mark.parametrize("nc,n", [(8, 1), (8, 2), (8, 9), (8, 33), (8, 70), (16, 8), (48, 3), (48, 8), (48, 31),
+                                  (64, 7), (64, 32)])
+def test_output_grid_cells_exact(nc, n):
+    """Every cell of the density grid equals the fixed-point sum, on grids
+    smaller than a tile, ragged ones and ones whose tiles several workgroups
+    share (64^3 particles on one tile), with positions on faces, outside the
+    box and in a dense clump; the snapshot records and the particle state
+    (both strides) agree."""
+    box = 40.0
+    print(f"output grid nc={nc} n={n}", flush=True)
+    rng = np.random.default_rng(n + nc)
+    npart = nc ** 3
+    x = rng.uniform(-1.4 * box, 2.4 * box, (npart, 3)).astype(np.float32)
+    x[: npart // 2] = (rng.uniform(0, box, 3) + rng.normal(0, 0.5, (npart // 2, 3))).astype(np.float32)
+    x[0], x[1], x[2] = 0.0, box, np.nextafter(np.float32(box), np.float32(0))
+    x[3] = -1e-7
+    snap = np.zeros(npart, ch.PARTICLE_MIN_DTYPE)
+    snap["x"], snap["id"] = x, np.arange(1, npart + 1)
+    parts = np.zeros(npart, ch.PARTICLE_DTYPE)
+    parts["x"], parts["id"] = x, snap["id"]
+    with ch.Context(nc, nc, box) as ctx:
+        ctx.set_snapshot_records(snap)
+        ctx.set_particles(parts, 0.5, 0.5)
+        delta, sums = ctx.coarse_grid(n, "snapshot")
+        again, _ = ctx.coarse_grid(n, "particles")
+    ref = _contrast_exact(x, n, box)
+    assert np.array_equal(delta, ref)
+    assert np.array_equal(again, ref)
+    assert sums[0] == pytest.approx(npart, rel=1e-6)
