@@ -37,8 +37,7 @@ struct ResNet {
   float* d_y = nullptr;
   // gradients at layer outputs [n^3][16] (bf16), two buffers
   unsigned short* d_g[2] = {nullptr, nullptr};
-  float* d_wpart = nullptr;  // per-wave partial weight gradients
-  int wpart_waves = 0;
+  float* d_wpart = nullptr;  // partial weight gradients of k_conv_wgrad's units
   double* d_loss = nullptr;
   float* d_a = nullptr;      // scale factor of standalone evaluations
   double* d_fsum = nullptr;  // sums of the residual the last corrected force added, per component

@@ -67,12 +67,6 @@ __device__ inline unsigned short feature_of(float delta, float scale) { return f
 
 __device__ inline int wrapi(int v, int n) { return v < 0 ? v + n : (v >= n ? v - n : v); }
 
-__device__ inline long long cell_at(int x, int y, int z, int t, int sign, int n)
-{
-  const int dx = t / 9 - 1, dy = (t / 3) % 3 - 1, dz = t % 3 - 1;
-  return ((long long)wrapi(x + sign * dx, n) * n + wrapi(y + sign * dy, n)) * n + wrapi(z + sign * dz, n);
-}
-
 enum ConvMode { kFwdRelu = 0, kFwdLinear = 1, kBwdData = 2, kFwdAdd = 3 };
 
 // Outputs of a convolution by mode: bf16 activations (kFwdRelu; kBwdData
@@ -1361,74 +1355,239 @@ k_conv12r(const float* __restrict__ delta, long long row, float in_scale, const 
 }
 
 // Weight gradient of one layer: dW[t][ci][co] = sum_cells X[cell + d_t][ci]
-// G[cell][co] (M = ci, N = co, K = 32 cells along z per MFMA; all 27 taps
-// accumulate in registers) and db[co] = sum_cells G[cell][co].  Each wave
-// writes its partial sums to part[wave][27 * 256 + 16].
-template <int CIN>
-__global__ void __launch_bounds__(kThreads)
-k_conv_wgrad(const unsigned short* __restrict__ X, const unsigned short* __restrict__ G, int n,
-             float* __restrict__ part)
+// G[cell][co] (M = ci, N = co, K = 32 cells along z per product; all 27 taps
+// accumulate in registers) and db[co] = sum_cells G[cell][co].
+//
+// Both operands have K along the cells while the activations are channel
+// last, so a lane's 8 values of K lie 8 cells apart: read with 2-byte loads
+// from memory (27 taps x 8 per product operand) the pass took 0.41 ms per
+// 16-channel layer and 1.50 ms for the 8-channel input at 192^3, bound by
+// load instructions at 10% of the HBM rate.  Here a workgroup owns 8 y x 32 z
+// cells and marches along x; each plane of X (10 rows, with its halo) and of
+// G goes through LDS once, transposed on the way ([row][channel][z], pairs of
+// cells packed from two 16-byte loads), so an operand is one 16-byte read
+// and its z-shifted neighbours are two more dwords and four v_alignbit each.
+// Wave w owns G rows 2w and 2w + 1 and holds their operands of planes p + 1,
+// p, p - 1, so X plane p is read once for its nine (dx, dz) taps of each row
+// pair.  54 products of a step are 864 MFMA clocks per SIMD and the HBM needs
+// 0.09 ms for both arrays; measured 0.14 ms (16 channels) and 0.12 ms (8).
+// The layer's 8-channel input fills both halves of M: rows 0-7 take dz = -1
+// (then +1), rows 8-15 dz = 0.
+// Every workgroup writes its sums to part[unit][27 * 256 + 16].
+constexpr int kWgRows = 8;                   // G rows of a unit
+constexpr int kWgZ = 32;                     // cells along z
+constexpr int kWgXStride = 28;               // dwords of one channel of an X row (56 cells: 8 + 32 + 2 used)
+constexpr int kWgGStride = 20;               // of a G row (32 used): strides that spread 16 channels over the banks
+constexpr int kWgXPairs = kWgZ / 2 + 2;      // cell pairs of an X row: z0 - 2 .. z0 + 33
+constexpr int kWgXRow = 16 * kWgXStride, kWgGRow = 16 * kWgGStride;
+constexpr int kWgXPlane = (kWgRows + 2) * kWgXRow, kWgGPlane = kWgRows * kWgGRow;
+constexpr size_t kWgBytes = sizeof(unsigned) * 2 * (kWgXPlane + kWgGPlane);
+constexpr int kWgPart = 27 * 256 + 16;       // floats of one unit's sums
+static_assert(kWgBytes >= sizeof(float) * kWgPart, "the waves' sums meet in the planes' LDS");
+
+// Two cells' 8 channels as 8 dwords (channel c: cell 0 low, cell 1 high) at
+// channel stride `stride`.
+__device__ inline void wg_put(unsigned* dst, int stride, uint4 a, uint4 b)
 {
-  const int lane = threadIdx.x & 63, g = lane >> 4, r = lane & 15;
-  floatx4 acc[27];
+  const unsigned av[4] = {a.x, a.y, a.z, a.w}, bv[4] = {b.x, b.y, b.z, b.w};
 #pragma unroll
-  for (int t = 0; t < 27; ++t) acc[t] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-  float bsum = 0.0f;
-  const long long nblk = (long long)n * n * (n / 32);
-  const long long nwaves = (long long)gridDim.x * (kThreads / 64);
-  const long long wave = (long long)blockIdx.x * (kThreads / 64) + (threadIdx.x >> 6);
-  for (long long blk = wave; blk < nblk; blk += nwaves) {
-    const int zb = (int)(blk % (n / 32));
-    const long long xy = blk / (n / 32);
-    const int y = (int)(xy % n), x = (int)(xy / n);
-    const int z0 = zb * 32 + 8 * g;
-    unsigned short bv[8];
-    const long long base = ((long long)x * n + y) * n + z0;
-#pragma unroll
-    for (int j = 0; j < 8; ++j) {
-      bv[j] = G[(base + j) * 16 + r];
-      bsum += bf2f(bv[j]);
-    }
-    bf16x8 bop;
-    __builtin_memcpy(&bop, bv, 16);
-#pragma unroll
-    for (int t = 0; t < 27; ++t) {
-      unsigned short av[8];
-#pragma unroll
-      for (int j = 0; j < 8; ++j) av[j] = r < CIN ? X[cell_at(x, y, z0 + j, t, 1, n) * CIN + r] : (unsigned short)0;
-      bf16x8 aop;
-      __builtin_memcpy(&aop, av, 16);
-      acc[t] = __builtin_amdgcn_mfma_f32_16x16x32_bf16(aop, bop, acc[t], 0, 0, 0);
-    }
+  for (int k = 0; k < 4; ++k) {
+    dst[(2 * k) * stride] = (av[k] & 0xffffu) | (bv[k] << 16);
+    dst[(2 * k + 1) * stride] = (av[k] >> 16) | (bv[k] & 0xffff0000u);
   }
-  float* p = part + wave * (27 * 256 + 16);
-#pragma unroll
-  for (int t = 0; t < 27; ++t)
-#pragma unroll
-    for (int i = 0; i < 4; ++i) p[(t * 16 + 4 * g + i) * 16 + r] = acc[t][i];
-  // bias: lanes r, r + 16, r + 32, r + 48 hold the same channel
-  bsum += __shfl_xor(bsum, 16);
-  bsum += __shfl_xor(bsum, 32);
-  if (g == 0) p[27 * 256 + r] = bsum;
 }
 
-// Sum of the per-wave partials (fixed order) into the fp32 gradient of one
-// layer, in the master layout W[t][ci][co] then b[co].
-__global__ void k_wgrad_reduce(const float* __restrict__ part, int nwaves, int cin, int cout, float* __restrict__ grad)
+template <int CIN>
+__global__ void __launch_bounds__(kThreads) __attribute__((amdgpu_waves_per_eu(2)))
+k_conv_wgrad(const unsigned short* __restrict__ X, const unsigned short* __restrict__ G, int n, int march,
+             float* __restrict__ part)
 {
+  extern __shared__ uint4 wg_lds[];
+  unsigned* const xs = reinterpret_cast<unsigned*>(wg_lds);
+  unsigned* const gs = xs + 2 * kWgXPlane;
+  constexpr int kHalves = CIN / 8;
+  constexpr int kXItems = (kWgRows + 2) * kWgXPairs * kHalves;
+  constexpr int kXRounds = (kXItems + kThreads - 1) / kThreads;
+  constexpr int kDz = CIN == 16 ? 3 : 2;  // products per (dx, dy)
+  const int tid = threadIdx.x, lane = tid & 63, g = lane >> 4, r = lane & 15, wave = tid >> 6;
+  const int nz = n / kWgZ, ny = n / kWgRows;
+  const int u = blockIdx.x;
+  const int z0 = u % nz * kWgZ, y0 = u / nz % ny * kWgRows;
+  const int x0 = u / (nz * ny) * march, x1 = min(n, x0 + march);
+
+  // this thread's share of a plane: X items (row, cell pair, half), one G item
+  int xsrc[kXRounds], xdst[kXRounds];
+  uint4 xa[kXRounds], xb[kXRounds];
+#pragma unroll
+  for (int k = 0; k < kXRounds; ++k) {
+    const int it = min(tid + k * kThreads, kXItems - 1);  // the spare lanes repeat the last item
+    const int h = it % kHalves, pr = it / kHalves % kWgXPairs, row = it / (kHalves * kWgXPairs);
+    const int z = wrapi(z0 - 2 + 2 * pr, n), y = wrapi(y0 - 1 + row, n);
+    xsrc[k] = (y * n + z) * CIN + 8 * h;
+    xdst[k] = row * kWgXRow + 8 * h * kWgXStride + 3 + pr;  // cell z at position z - z0 + 8
+  }
+  const int gh = tid & 1, gp_ = (tid >> 1) & 15, grow = tid >> 5;
+  const int gsrc = ((y0 + grow) * n + z0 + 2 * gp_) * 16 + 8 * gh;
+  const int gdst = grow * kWgGRow + 8 * gh * kWgGStride + gp_;
+  static_assert(kWgRows * (kWgZ / 2) * 2 == kThreads, "one G item per thread");
+  uint4 ga, gb;
+  const long long plane = (long long)n * n;
+
+  auto load_x = [&](int p) {
+    const unsigned short* b = X + (long long)wrapi(p, n) * plane * CIN;
+#pragma unroll
+    for (int k = 0; k < kXRounds; ++k) {
+      xa[k] = *reinterpret_cast<const uint4*>(b + xsrc[k]);
+      xb[k] = *reinterpret_cast<const uint4*>(b + xsrc[k] + CIN);
+    }
+  };
+  auto load_g = [&](int q) {
+    const unsigned short* b = G + (long long)q * plane * 16;
+    ga = *reinterpret_cast<const uint4*>(b + gsrc);
+    gb = *reinterpret_cast<const uint4*>(b + gsrc + 16);
+  };
+  auto put_x = [&](int p) {
+    unsigned* d = xs + (p & 1) * kWgXPlane;
+#pragma unroll
+    for (int k = 0; k < kXRounds; ++k) wg_put(d + xdst[k], kWgXStride, xa[k], xb[k]);
+  };
+  auto put_g = [&](int q) { wg_put(gs + (q & 1) * kWgGPlane + gdst, kWgGStride, ga, gb); };
+
+  floatx4 acc[9][kDz];
+#pragma unroll
+  for (int t = 0; t < 9; ++t)
+#pragma unroll
+    for (int d = 0; d < kDz; ++d) acc[t][d] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+  float bsum = 0.0f;
+  const uint4 zero4 = make_uint4(0u, 0u, 0u, 0u);
+  uint4 gop[3][2];  // G operands of planes p + 1, p, p - 1 (dx = -1, 0, +1), rows 2w, 2w + 1
+#pragma unroll
+  for (int d = 0; d < 3; ++d) gop[d][0] = gop[d][1] = zero4;
+
+  load_x(x0 - 1);
+  load_g(x0);
+  put_x(x0 - 1);
+  put_g(x0);
+  __syncthreads();
+  const int xch = CIN == 16 ? r : (r & 7);
+  for (int p = x0 - 1; p <= x1; ++p) {
+    const bool more_x = p < x1, more_g = p + 2 < x1;
+    if (more_x) load_x(p + 1);
+    if (more_g) load_g(p + 2);
+#pragma unroll
+    for (int i = 0; i < 2; ++i) {
+      gop[2][i] = gop[1][i];
+      gop[1][i] = gop[0][i];
+      gop[0][i] = zero4;
+    }
+    if (p + 1 < x1) {
+      const unsigned* gl = gs + ((p + 1) & 1) * kWgGPlane + 2 * wave * kWgGRow + r * kWgGStride + 4 * g;
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const uint4 v = *reinterpret_cast<const uint4*>(gl + i * kWgGRow);
+        gop[0][i] = v;
+        const unsigned w4[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+        for (int k = 0; k < 4; ++k) {
+          bsum += bf2f((unsigned short)(w4[k] & 0xffffu));
+          bsum += bf2f((unsigned short)(w4[k] >> 16));
+        }
+      }
+    }
+    const unsigned* xl = xs + (p & 1) * kWgXPlane + 2 * wave * kWgXRow + xch * kWgXStride + 4 + 4 * g;
+#pragma unroll
+    for (int j = 0; j < 4; ++j) {  // X row y0 + 2w + j - 1
+      const uint4 a = *reinterpret_cast<const uint4*>(xl + j * kWgXRow);
+      const unsigned lo = xl[j * kWgXRow - 1], hi = xl[j * kWgXRow + 4];
+      const uint4 am = make_uint4(__builtin_amdgcn_alignbit(a.x, lo, 16), __builtin_amdgcn_alignbit(a.y, a.x, 16),
+                                  __builtin_amdgcn_alignbit(a.z, a.y, 16), __builtin_amdgcn_alignbit(a.w, a.z, 16));
+      const uint4 ap = make_uint4(__builtin_amdgcn_alignbit(a.y, a.x, 16), __builtin_amdgcn_alignbit(a.z, a.y, 16),
+                                  __builtin_amdgcn_alignbit(a.w, a.z, 16), __builtin_amdgcn_alignbit(hi, a.w, 16));
+      uint4 op[kDz];
+      if constexpr (CIN == 16) {
+        op[0] = am;
+        op[1] = a;
+        op[2] = ap;
+      } else {
+        op[0] = sel4(r < 8, am, a);
+        op[1] = sel4(r < 8, ap, zero4);
+      }
+#pragma unroll
+      for (int i = 0; i < 2; ++i) {
+        const int dy = j - 1 - i;  // of G row i
+        if (dy < -1 || dy > 1) continue;
+#pragma unroll
+        for (int dx = 0; dx < 3; ++dx)
+#pragma unroll
+          for (int d = 0; d < kDz; ++d)
+            acc[3 * dx + dy + 1][d] = mfma(gop[dx][i], op[d], acc[3 * dx + dy + 1][d]);  // rows ci, columns co
+      }
+    }
+    if (more_x) put_x(p + 1);
+    if (more_g) put_g(p + 2);
+    __syncthreads();  // the next planes are in LDS, this step's operand reads are done
+  }
+
+  // the four waves' sums, added in wave order in LDS
+  float* const sums = reinterpret_cast<float*>(wg_lds);
+  bsum += __shfl_xor(bsum, 16);  // lanes r, r + 16, r + 32, r + 48 hold the same channel
+  bsum += __shfl_xor(bsum, 32);
+  for (int w = 0; w < kThreads / 64; ++w) {
+    if (wave == w) {
+      auto put = [&](int at, float v) { sums[at] = w == 0 ? v : sums[at] + v; };
+#pragma unroll
+      for (int t = 0; t < 9; ++t)
+#pragma unroll
+        for (int d = 0; d < kDz; ++d)
+#pragma unroll
+          for (int i = 0; i < 4; ++i) {
+            const int m = 4 * g + i;
+            if constexpr (CIN == 16) {
+              put(((3 * t + d) * 16 + m) * 16 + r, acc[t][d][i]);
+            } else if (d == 0) {
+              put(((3 * t + (m >> 3)) * 16 + (m & 7)) * 16 + r, acc[t][d][i]);
+            } else if (m < 8) {
+              put(((3 * t + 2) * 16 + m) * 16 + r, acc[t][d][i]);
+            }
+          }
+      if (g == 0) put(27 * 256 + r, bsum);
+    }
+    __syncthreads();
+  }
+  float* const out = part + (long long)u * kWgPart;
+  for (int e = tid; e < kWgPart; e += kThreads) out[e] = sums[e];
+}
+
+// Sum of the units' partials (fixed order) into the fp32 gradient of one
+// layer, in the master layout W[t][ci][co] then b[co].  A workgroup sums 64
+// entries, 16 strided shares of the units each (one thread per entry summing
+// 2048 partials in turn took 0.49 ms per layer, now 0.014 ms).
+constexpr int kReduceShares = 16;
+
+__global__ void __launch_bounds__(64 * kReduceShares)
+k_wgrad_reduce(const float* __restrict__ part, int units, int cin, int cout, float* __restrict__ grad)
+{
+  __shared__ float share[kReduceShares][64];
   const int nw = 27 * cin * cout;
-  const int p = blockIdx.x * blockDim.x + threadIdx.x;
-  if (p >= nw + cout) return;
-  int src;
+  const int e = threadIdx.x & 63, q = threadIdx.x >> 6;
+  const int p = blockIdx.x * 64 + e;
+  int src = 27 * 256;
   if (p < nw) {
     const int t = p / (cin * cout), ci = (p / cout) % cin, co = p % cout;
     src = (t * 16 + ci) * 16 + co;
-  } else {
+  } else if (p < nw + cout) {
     src = 27 * 256 + (p - nw);
   }
   float s = 0.0f;
-  for (int w = 0; w < nwaves; ++w) s += part[(long long)w * (27 * 256 + 16) + src];
-  grad[p] = s;
+#pragma unroll 8
+  for (int w = q; w < units; w += kReduceShares) s += part[(long long)w * kWgPart + src];
+  share[q][e] = s;
+  __syncthreads();
+  if (q == 0 && p < nw + cout) {
+    float tot = 0.0f;
+    for (int k = 0; k < kReduceShares; ++k) tot += share[k][e];
+    grad[p] = tot;
+  }
 }
 
 // Tap of chunk c for lane-group half h (0: lane groups 0, 1; 1: groups 2, 3)
@@ -1680,7 +1839,6 @@ long long param_offset(int layer)
 unsigned grid_cells(long long n) { return (unsigned)((n + kThreads - 1) / kThreads); }
 
 constexpr int kConvBlocks = 512;  // two workgroups per CU on 256 CUs
-constexpr int kWgradBlocks = 512;
 
 template <typename T>
 int dev_alloc(T** p, long long count)
@@ -1725,7 +1883,6 @@ int resnet_init(ResNet* r, int n, unsigned seed)
   COLA_TRY(dev_alloc(&r->d_fi, 3 * nc));
   COLA_TRY(dev_alloc(&r->d_trash, 256));
   COLA_TRY(dev_alloc(&r->d_a, 1));
-  r->wpart_waves = kWgradBlocks * (kThreads / 64);
   // He-normal initial weights (std sqrt(2 / fan_in)), zero biases and moments
   std::vector<float> p(kNetParams, 0.0f);
   std::mt19937 gen(seed);
@@ -1815,6 +1972,26 @@ ConvLaunch conv_launch_roll(int n)
   return c;
 }
 
+// k_conv_wgrad: one workgroup per unit, two resident per CU; a march of m G
+// planes takes m + 2 steps; the march with the least work on the busiest CU.
+ConvLaunch wgrad_launch(int n)
+{
+  const long long cols = (long long)(n / kWgRows) * (n / kWgZ);
+  long long best = -1;
+  ConvLaunch c{1, n};
+  for (int nseg = 1; nseg <= n; ++nseg) {
+    const int march = (n + nseg - 1) / nseg;
+    const long long units = (long long)((n + march - 1) / march) * cols;
+    const long long cost = (units + 511) / 512 * (march + 2);
+    if (best < 0 || cost < best) {
+      best = cost;
+      c.blocks = (unsigned)units;
+      c.march = march;
+    }
+  }
+  return c;
+}
+
 // k_conv3h: one workgroup per CU; a march of m output planes takes
 // ceil((m + 4) / 3) rotations; the march with the least work on the busiest
 // workgroup.
@@ -1858,6 +2035,8 @@ int conv_lds_attributes()
   for (const void* k : kr) COLA_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kRollRingBytes));
   COLA_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_conv3h), hipFuncAttributeMaxDynamicSharedMemorySize,
                                (int)kConv3hBytes));
+  const void* kw[] = {reinterpret_cast<const void*>(&k_conv_wgrad<8>), reinterpret_cast<const void*>(&k_conv_wgrad<16>)};
+  for (const void* k : kw) COLA_HIP(hipFuncSetAttribute(k, hipFuncAttributeMaxDynamicSharedMemorySize, (int)kWgBytes));
   COLA_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&k_conv8), hipFuncAttributeMaxDynamicSharedMemorySize,
                                (int)kRing8Bytes));
   done = true;
@@ -2048,10 +2227,11 @@ int resnet_backward(ResNet* r, const unsigned short* tb, const float* tf, hipStr
 {
   const int n = r->n;
   const long long nc = (long long)n * n * n;
+  const ConvLaunch wl = wgrad_launch(n);
   if (!r->d_g[0]) {
     COLA_TRY(dev_alloc(&r->d_g[0], nc * 16));
     COLA_TRY(dev_alloc(&r->d_g[1], nc * 16));
-    COLA_TRY(dev_alloc(&r->d_wpart, (long long)r->wpart_waves * (27 * 256 + 16)));
+    COLA_TRY(dev_alloc(&r->d_wpart, (long long)wl.blocks * kWgPart));
   }
   COLA_TRY(conv_lds_attributes());
   hipLaunchKernelGGL(k_zero1, dim3(1), dim3(64), 0, s, r->d_loss);
@@ -2062,12 +2242,14 @@ int resnet_backward(ResNet* r, const unsigned short* tb, const float* tf, hipStr
   unsigned short* Gp = r->d_g[1];
   for (int l = kNetLayers - 1; l >= 0; --l) {
     if (kNetCin[l] == 8)
-      hipLaunchKernelGGL(k_conv_wgrad<8>, dim3(kWgradBlocks), dim3(kThreads), 0, s, X[l], G, n, r->d_wpart);
+      hipLaunchKernelGGL(k_conv_wgrad<8>, dim3(wl.blocks), dim3(kThreads), kWgBytes, s, X[l], G, n, wl.march,
+                         r->d_wpart);
     else
-      hipLaunchKernelGGL(k_conv_wgrad<16>, dim3(kWgradBlocks), dim3(kThreads), 0, s, X[l], G, n, r->d_wpart);
+      hipLaunchKernelGGL(k_conv_wgrad<16>, dim3(wl.blocks), dim3(kThreads), kWgBytes, s, X[l], G, n, wl.march,
+                         r->d_wpart);
     const int np = 27 * kNetCin[l] * kNetCout[l] + kNetCout[l];
-    hipLaunchKernelGGL(k_wgrad_reduce, dim3((np + 255) / 256), dim3(256), 0, s, r->d_wpart, r->wpart_waves,
-                       kNetCin[l], kNetCout[l], r->d_grad + param_offset(l));
+    hipLaunchKernelGGL(k_wgrad_reduce, dim3((np + 63) / 64), dim3(64 * kReduceShares), 0, s, r->d_wpart,
+                       (int)wl.blocks, kNetCin[l], kNetCout[l], r->d_grad + param_offset(l));
     if (l == 0) break;
     // gradient at the output of layer l - 1: data gradient of layer l masked by relu'(h_{l-1})
     const ConvLaunch cl = conv_launch(n);

@@ -121,6 +121,30 @@ def test_gradient_matches_oracle():
         assert rel <= 5e-2, (kind, a, rel)
 
 
+@pytest.mark.parametrize("n", [64, 128])
+def test_gradient_of_a_tiled_input(n):
+    """An input and target of period 32 on a grid 2 or 4 times as large (8
+    and 64 times the cells: the mean loss's gradient scales by a power of two
+    per cell, so every bfloat16 value keeps its mantissa) has the gradient of
+    the 32^3 grid up to the order of the fp32 sums, whatever the units the
+    sums are cut into (marches of 1, 2 and 16 planes at 32^3, 64^3, 128^3).
+    Bound: a sum of 2 M terms in units of a few thousand, rounded at 2^-24
+    each step, stays within 1e-5 of its norm."""
+    print(f"net gradient tiled n={n}", flush=True)
+    params, x = _setup(32, 17)
+    target = np.random.default_rng(18).standard_normal((32, 32, 32, 3)).astype(np.float32)
+    got = {}
+    for m in (32, n):
+        k = m // 32
+        with ch.ResidualNet(m) as net:
+            net.set_params(params)
+            net.set_scales(1.0, 1.0)
+            loss, got[m] = net.gradient(np.tile(x, (k, k, k, 1)), np.tile(target, (k, k, k, 1)))
+    for kind, a, b in _blocks():
+        rel = np.linalg.norm(got[n][a:b] - got[32][a:b]) / np.linalg.norm(got[32][a:b])
+        assert rel <= 1e-5, (kind, a, rel)
+
+
 def test_adam_steps_follow_the_published_update():
     """Two Adam steps (Kingma & Ba 2015, Algorithm 1: beta1 0.9, beta2 0.999,
     eps 1e-8, moments m = b1 m + (1 - b1) g, v = b2 v + (1 - b2) g^2, bias
