@@ -63,7 +63,7 @@ def launches_per_phase(phase, stats):
     return 1
 
 
-def kernel_cost(phase, nc, ng):
+def kernel_cost(phase, nc, ng, net=False):
     """(algorithmic HBM bytes, MFMA flops, kernel) of one launch: each input
     array read once and each output array written once (FP32 PM arrays,
     bfloat16 activations), per the canonical per-phase model."""
@@ -76,9 +76,12 @@ def kernel_cost(phase, nc, ng):
         "fft_y_fwd": (16 * n_c, 0, "fft_tile (y columns)"),
         "fft_x_fwd": (16 * n_c, 0, "fft_tile (x columns)"),
         "fft_x_inv": (16 * n_c, 0, "fft_tile (x columns)"),
-        "fft_x_fused": (32 * n_c, 0, "fft_x_fused"),  # reads delta_k once, writes the three F_k
-        "fft_y_inv": (16 * n_c, 0, "fft_tile (y columns)"),
-        "fft_z_c2r": (8 * n_c + 4 * n_g, 0, "fft_tile (z c2r rows)"),
+        # reads delta_k once, writes the spectra of F_x and of what F_y and F_z share
+        "fft_x_fused": (24 * n_c, 0, "fft_x_fused"),
+        # mean of two launches: F_x in place; the shared spectrum to F_y and F_z
+        "fft_y_inv": (20 * n_c, 0, "fft_yinv"),
+        # a plain run's one launch writes the records of three components, a corrected run has one per component
+        "fft_z_c2r": ((1 if net else 3) * (8 * n_c + 4 * n_g), 0, "fft_tile (z c2r rows)" if net else "fft_c2r3"),
         "deposit": (4 * n_g + 12 * n_p, 0, "k_deposit_tiles"),
         "readout_kick_drift": (12 * n_g + 72 * n_p, 0, "k_readout_kick_drift"),
         "bin_count": (12 * n_p, 0, "k_bin_count"),
@@ -125,7 +128,7 @@ def roofline(stats, nc, ng, net=False):
     (and MFMA flops) per launch over the mean launch time; the binding roof
     is the larger of bytes / 8 TB/s and flops / 2.5 PFLOP/s (dense BF16)."""
     dom, (dom_ms, dom_n) = max(stats.items(), key=lambda kv: kv[1][0])
-    cost = kernel_cost(dom, nc, ng)
+    cost = kernel_cost(dom, nc, ng, net)
     if cost is None or dom_n == 0:
         return None
     nbytes, flops, kname = cost

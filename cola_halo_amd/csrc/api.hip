@@ -92,7 +92,7 @@ struct cola_context {
   DevParticles p;
   float* pbuf = nullptr;
   float* density = nullptr;
-  float* fgrid[3] = {nullptr, nullptr, nullptr};
+  float* fgrid = nullptr;  // force lines (ForceLines): 3 cic.row floats per line
   long long grid_floats = 0;
 
   FftPlan pm_fft, lpt_fft;
@@ -130,6 +130,7 @@ struct cola_context {
   bool have_force = false;
   bool have_grids = false;
   bool fi_force = false;  // the last force was corrected: its grids are the net's interleaved d_fi
+  bool force_records = false;  // fgrid holds records (or, corrected, the plain components apart)
   bool density_is_real = false;
 
   DevParticleMin* d_snap = nullptr;
@@ -275,10 +276,10 @@ int alloc_grids(cola_context* c)
   if (c->have_grids) return kOk;
   const size_t bytes = sizeof(float) * c->grid_floats;
   COLA_HIP(hipMalloc(&c->density, bytes));
-  for (int a = 0; a < 3; ++a) COLA_HIP(hipMalloc(&c->fgrid[a], bytes));
+  COLA_HIP(hipMalloc(&c->fgrid, 3 * bytes));
   // the row padding is never written by the deposit; keep it finite
   COLA_HIP(hipMemset(c->density, 0, bytes));
-  for (int a = 0; a < 3; ++a) COLA_HIP(hipMemset(c->fgrid[a], 0, bytes));
+  COLA_HIP(hipMemset(c->fgrid, 0, 3 * bytes));
   c->have_grids = true;
   return kOk;
 }
@@ -344,7 +345,6 @@ KOpParams pm_kop(const cola_context* c)
 int pm_fields(cola_context* c)
 {
   const KOpParams kp = pm_kop(c);
-  float* const out[3] = {c->fgrid[0], c->fgrid[1], c->fgrid[2]};
   // the net's features come from the real-space density before the r2c
   // overwrites it; its last layer adds its output to the force grids
   // with fuse34 (by input planes) layer 3 runs with the last layer after the transforms
@@ -370,17 +370,20 @@ int pm_fields(cola_context* c)
     phase_end(c, kPhNetHidden);
   }
   c->density_is_real = false;
-  COLA_TRY(c->pm_fft.forces(c->density, out, kp, c->stream));
+  // the readout gathers records; the net's last layer reads the components
+  // apart and writes the corrected records
+  COLA_TRY(c->pm_fft.forces(c->density, c->fgrid, kp, c->net == nullptr, c->stream));
   if (fused34) {
     phase_begin(c, kPhNetConv34);
-    COLA_TRY(resnet_layer3_head(c->net, out, c->cic.row, c->stream));
+    COLA_TRY(resnet_layer3_head(c->net, c->fgrid, c->cic.row, 3 * c->cic.row, c->stream));
     phase_end(c, kPhNetConv34);
   } else if (c->net) {
     phase_begin(c, kPhNetHead);
-    COLA_TRY(resnet_head_add(c->net, out, c->cic.row, c->stream));
+    COLA_TRY(resnet_head_add(c->net, c->fgrid, c->cic.row, 3 * c->cic.row, c->stream));
     phase_end(c, kPhNetHead);
   }
   c->fi_force = c->net != nullptr;
+  c->force_records = c->net == nullptr;
   return kOk;
 }
 
@@ -389,9 +392,13 @@ bool valid(const cola_context* c) { return c != nullptr; }
 // The learned residual's sums over the grid of the last force (its mean is
 // taken off the particles' forces), or null without a net.
 const double* net_sums(const cola_context* c) { return c->net ? c->net->d_fsum : nullptr; }
-// The corrected force grids, interleaved [cell][3] (what the readout
-// gathers), or null without a net (the readout then reads fgrid[0..2]).
-const float* net_fi(const cola_context* c) { return c->net ? c->net->d_fi : nullptr; }
+// What the readout gathers from: the transforms' force lines, or with a net
+// its corrected force grid [cell][3].
+ForceLines force_lines(const cola_context* c)
+{
+  if (c->net) return ForceLines{c->net->d_fi, 3LL * c->ng};
+  return ForceLines{c->fgrid, 3 * c->cic.row};
+}
 
 int require_particles(cola_context* c)
 {
@@ -524,8 +531,7 @@ int cola_context_destroy(cola_context* c)
   bin_free(&c->bins);
   if (c->pbuf) (void)hipFree(c->pbuf);
   if (c->density) (void)hipFree(c->density);
-  for (int a = 0; a < 3; ++a)
-    if (c->fgrid[a]) (void)hipFree(c->fgrid[a]);
+  if (c->fgrid) (void)hipFree(c->fgrid);
   if (c->d_mass) (void)hipFree(c->d_mass);
   if (c->step_graph) (void)hipGraphExecDestroy(c->step_graph);
   if (c->h_prm) (void)hipHostFree(c->h_prm);
@@ -827,7 +833,7 @@ int cola_pm_calculate_forces(cola_context* c)
   COLA_TRY(check_pending(c));
   COLA_TRY(pm_fields(c));
   phase_begin(c, kPhReadout);
-  COLA_TRY(launch_readout(c->p, c->cic, c->fgrid[0], c->fgrid[1], c->fgrid[2], net_sums(c), net_fi(c), c->stream));
+  COLA_TRY(launch_readout(c->p, c->cic, force_lines(c), net_sums(c), c->stream));
   phase_end(c, kPhReadout);
   c->have_force = true;
   return kOk;
@@ -876,8 +882,7 @@ int step_kernels(cola_context* c)
   COLA_TRY(assign_kernels(c, true));
   COLA_TRY(pm_fields(c));
   phase_begin(c, kPhReadoutKickDrift);
-  COLA_TRY(launch_readout_kick_drift(c->p, c->cic, c->fgrid[0], c->fgrid[1], c->fgrid[2], c->d_prm, net_sums(c),
-                                     net_fi(c), c->stream));
+  COLA_TRY(launch_readout_kick_drift(c->p, c->cic, force_lines(c), c->d_prm, net_sums(c), c->stream));
   phase_end(c, kPhReadoutKickDrift);
   return kOk;
 }
@@ -1022,7 +1027,7 @@ int ensemble_build(cola_ensemble* e)
   const int n = (int)e->ctx.size();
   std::vector<PmMember> ms(n);
   std::vector<const FftPlan*> plans(n);
-  std::vector<float*> dens(n), outs(3 * n);
+  std::vector<float*> dens(n), outs(n);
   std::vector<KOpParams> kps(n);
   for (int m = 0; m < n; ++m) {
     cola_context* c = e->ctx[m];
@@ -1042,13 +1047,13 @@ int ensemble_build(cola_ensemble* e)
     M.t = c->tiles;
     M.b = c->bins;
     M.density = c->density;
-    for (int a = 0; a < 3; ++a) M.f[a] = c->fgrid[a];
+    M.f = force_lines(c);
     M.ring = c->d_mass;
     M.prm = e->d_prm + m;
     M.boxsize = c->boxf;
     plans[m] = &c->pm_fft;
     dens[m] = c->density;
-    for (int a = 0; a < 3; ++a) outs[3 * m + a] = c->fgrid[a];
+    outs[m] = c->fgrid;
     kps[m] = pm_kop(c);
     e->gen[m] = c->config_gen;
   }
@@ -1384,19 +1389,31 @@ int cola_get_force_grid(cola_context* c, int axis, float* out, size_t n_out)
   if (!valid(c) || !out || axis < 0 || axis > 2 || n_out < host_grid_floats(c)) return kErrArg;
   if (!c->have_grids) return kErrState;
   COLA_HIP(hipStreamSynchronize(c->stream));
-  if (c->fi_force && c->net) {
-    // the corrected force lives interleaved in the net's grid
-    const long long cells = (long long)c->ng * c->ng * c->ng;
-    std::vector<float> fi(3 * (size_t)cells);
-    COLA_HIP(hipMemcpy(fi.data(), c->net->d_fi, sizeof(float) * fi.size(), hipMemcpyDeviceToHost));
-    const long long hrow = 2 * (c->ng / 2 + 1);
-    for (long long line = 0; line < (long long)c->ng * c->ng; ++line) {
-      for (int z = 0; z < c->ng; ++z) out[line * hrow + z] = fi[(line * c->ng + z) * 3 + axis];
-      out[line * hrow + c->ng] = out[line * hrow + c->ng + 1] = 0.0f;
-    }
+  const bool fi = c->fi_force && c->net;
+  if (!fi && !c->force_records) {  // the components apart, one row each per line
+    const long long lines = (long long)c->ng * c->ng, hrow = 2 * (c->ng / 2 + 1);
+    COLA_HIP(hipMemcpy2D(out, sizeof(float) * hrow, c->fgrid + axis * c->cic.row, sizeof(float) * 3 * c->cic.row,
+                         sizeof(float) * c->ng, (size_t)lines, hipMemcpyDeviceToHost));
+    for (long long r = 0; r < lines; ++r) out[r * hrow + c->ng] = out[r * hrow + c->ng + 1] = 0.0f;
     return kOk;
   }
-  return grid_to_host(c, c->fgrid[axis], out);
+  // records F[z][3] per line, of the transforms or of the net's corrected
+  // grid: copied a few lines at a time, one component picked on the host
+  const ForceLines fl = fi ? ForceLines{c->net->d_fi, 3LL * c->ng} : ForceLines{c->fgrid, 3 * c->cic.row};
+  const long long lines = (long long)c->ng * c->ng, hrow = 2 * (c->ng / 2 + 1);
+  const long long chunk = std::max(1LL, std::min(lines, (1LL << 24) / (3LL * c->ng)));
+  std::vector<float> rec((size_t)(3LL * c->ng * chunk));
+  for (long long l0 = 0; l0 < lines; l0 += chunk) {
+    const long long nl = std::min(chunk, lines - l0);
+    COLA_HIP(hipMemcpy2D(rec.data(), sizeof(float) * 3 * c->ng, fl.f + l0 * fl.line, sizeof(float) * fl.line,
+                         sizeof(float) * 3 * c->ng, (size_t)nl, hipMemcpyDeviceToHost));
+    for (long long l = 0; l < nl; ++l) {
+      float* o = out + (l0 + l) * hrow;
+      for (int z = 0; z < c->ng; ++z) o[z] = rec[(size_t)((l * c->ng + z) * 3 + axis)];
+      o[c->ng] = o[c->ng + 1] = 0.0f;
+    }
+  }
+  return kOk;
 }
 
 double cola_last_mass_sum(const cola_context* c) { return c ? c->last_mass : 0.0; }
@@ -2258,9 +2275,8 @@ int cola_resnet_add_pair(cola_resnet* h, cola_context* coarse, cola_context* fin
   if (!st) st = check_pending(coarse);
   if (!st) st = check_pending(fine);
   if (!st) {
-    const float* const cf[3] = {coarse->fgrid[0], coarse->fgrid[1], coarse->fgrid[2]};
-    const float* const ff[3] = {fine->fgrid[0], fine->fgrid[1], fine->fgrid[2]};
-    st = resnet_store_pair(&h->r, dcopy, coarse->cic.row, cf, ff, fine->cic.row, coarse->a_x, h->stream);
+    st = resnet_store_pair(&h->r, dcopy, coarse->cic.row, ForceLines{coarse->fgrid, 3 * coarse->cic.row},
+                           ForceLines{fine->fgrid, 3 * fine->cic.row}, coarse->a_x, h->stream);
   }
   if (!st && hipStreamSynchronize(h->stream) != hipSuccess) st = kErrHip;
   if (dcopy) (void)hipFree(dcopy);
@@ -2509,18 +2525,17 @@ int cola_fft_time(int n, int reps, double* ms_out)
   FftPlan plan;
   COLA_TRY(plan.init(n, -1, -1, true));  // the PM layout: rows padded to 128 bytes
   const long long floats = (long long)n * n * 2 * plan.nzp;
-  float* buf[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};  // work, pristine copy, 3 force grids
+  float* buf[3] = {nullptr, nullptr, nullptr};  // work, pristine copy, force lines
   hipEvent_t e0 = nullptr, e1 = nullptr;
   int st = kOk;
-  for (int b = 0; b < 5 && !st; ++b)
-    if (hipMalloc(&buf[b], sizeof(float) * floats) != hipSuccess) st = kErrAlloc;
+  for (int b = 0; b < 3 && !st; ++b)
+    if (hipMalloc(&buf[b], sizeof(float) * floats * (b == 2 ? 3 : 1)) != hipSuccess) st = kErrAlloc;
   if (!st && (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess)) st = kErrHip;
   if (!st) {
     hipLaunchKernelGGL(k_fill_pattern, dim3((unsigned)((floats + 255) / 256)), dim3(256), 0, nullptr, buf[1], floats,
                        12345u);
     KOpParams kp;
     kp.f1 = 1.0f;
-    float* const out[3] = {buf[2], buf[3], buf[4]};
     double tot[3] = {0, 0, 0};
     for (int r = 0; r <= reps && !st; ++r) {  // r = 0 warms up
       for (int which = 0; which < 3 && !st; ++which) {
@@ -2534,7 +2549,7 @@ int cola_fft_time(int n, int reps, double* ms_out)
         else if (which == 1)
           st = plan.c2r(nullptr, buf[0], KOp::None, KOpParams{}, nullptr);
         else
-          st = plan.forces(buf[0], out, kp, nullptr);
+          st = plan.forces(buf[0], buf[2], kp, true, nullptr);
         (void)hipEventRecord(e1, nullptr);
         float ms = 0;
         if (!st && (hipEventSynchronize(e1) != hipSuccess || hipEventElapsedTime(&ms, e0, e1) != hipSuccess))

@@ -21,6 +21,7 @@
 namespace cola {
 
 constexpr int kFftMaxThreads = 1024;
+constexpr int kFftC2r3Threads = 320;  // per component of the z c2r of three (a workgroup has three groups)
 constexpr int kFftMaxTile = 12288;  // n * T complex values per workgroup (96 KiB)
 
 // One radix pass: radix R, L = product of the earlier radices, m = n / R,
@@ -40,13 +41,14 @@ struct FftRadices {
 // transform: the k-space operators of the PM force and of 2LPT.
 enum class KOp : int {
   None = 0,
-  PmPoisson = 1,  // pm.c:322-346  F = i f2 delta, f2 = f1 n_axis / |n|^2
+  PmPoisson = 1,  // pm.c:322-346  F_x = i f2 delta, f2 = f1 n_x / |n|^2
+  PmCommon = 4,   // i f1 / |n|^2 delta, which F_y and F_z are n_y and n_z times
   LptGrad = 2,    // lpt.c:379-395 i k_dir * disp
   Lpt2 = 3,       // lpt.c:479-486 source * k_axis / (i k^2)
 };
 
 struct KOpParams {
-  int axis = 0;       // PmPoisson / Lpt2 axis, LptGrad derivative direction
+  int axis = 0;       // Lpt2 axis, LptGrad derivative direction
   float f1 = 0.0f;    // pm.c:317
   double box = 0.0;   // lpt.c kvec = n * 2 * pi / Box
 };
@@ -64,6 +66,7 @@ struct FftPlan {
   FftRadices rad;
   float2* d_tw = nullptr;  // exp(-2 pi i k / n), k < n
   FftPassGeom grows, gy, gx;
+  FftPassGeom gz3;  // z c2r of three components: threads of one component
   int xgroup = 8;  // adjacent column tiles per XCD dispatch group (measured best)
   // Complex row stride of the half spectrum (>= n/2+1): rows padded to a
   // multiple of 16 complex values start on 128-byte lines, so column tiles
@@ -92,17 +95,20 @@ struct FftPlan {
   // then y, then c2r over z, in place on out.
   int c2r(const float2* in_k, float* out, KOp op, const KOpParams& kp, hipStream_t s) const;
   // The PM force fields in one sequence (pm.c:282-355): r2c of the padded
-  // real density (in place; destroyed), then for each axis the Poisson
-  // gradient and c2r into out[axis].  The forward x pass, the three Poisson
-  // operators and the three inverse x passes run as one fused kernel
-  // (hook pass 6); delta(k) is never written to memory.
-  int forces(float* density, float* const out[3], const KOpParams& kp, hipStream_t s) const;
+  // real density (in place; destroyed), Poisson gradient and c2r of the three
+  // components into `force`: per line (x, y) three slots of 2 nzp floats (on
+  // the way, the components' spectra).  records: the line's first 3 n floats
+  // are its records F[z][3]; else each slot holds its component's n values.
+  // Where can_fuse() holds, the forward x pass, the Poisson operator and the
+  // inverse x passes run as one fused kernel (hook pass 6) and delta(k) is
+  // never written to memory.
+  int forces(float* density, float* force, const KOpParams& kp, bool records, hipStream_t s) const;
   bool can_fuse() const;
 };
 
 // One launch of a batched force transform: one pass of every grid.
 struct FftBatchStage {
-  int pass = 0;  // 0 z r2c, 1 y forward, 2 fused x, 3 y inverse (3 axes), 4 z c2r (3 axes)
+  int pass = 0;  // 0 z r2c, 1 y forward, 2 fused x, 3 y inverse (two jobs a grid), 4 z c2r of the three components
   int emax = 0, rs = 0, threads = 0;
   size_t lds = 0;
   int blocks = 0, njobs = 0;
@@ -111,9 +117,8 @@ struct FftBatchStage {
 };
 
 // The force transforms (FftPlan::forces) of many grids, batched per pass
-// over the workgroups of every grid: z r2c, y forward, fused x, the y inverse
-// of the three axes, the z c2r of the three axes (instead of nine launches
-// per grid).  Each grid keeps its own plan's radix schedule and tile
+// over the workgroups of every grid: z r2c, y forward, fused x, y inverse, z
+// c2r (instead of six launches per grid).  Each grid keeps its own plan's radix schedule and tile
 // shapes; a launch runs its jobs with the widest workgroup and register
 // tile any of them needs, and the butterflies of a job do not depend on
 // either, so the outputs equal each plan's forces() bit for bit.
@@ -124,9 +129,9 @@ struct FftBatchStage {
 struct FftForcesBatch {
   std::vector<FftBatchStage> stages;
   void* d_mem = nullptr;
-  // plans[i] transforms density[i] (destroyed) into out[3 i + axis] with
-  // the operator parameters kp[i].
-  int init(const FftPlan* const* plans, float* const* density, float* const* out, const KOpParams* kp, int n,
+  // plans[i] transforms density[i] (destroyed) into force[i] with the
+  // operator parameters kp[i].
+  int init(const FftPlan* const* plans, float* const* density, float* const* force, const KOpParams* kp, int n,
            bool merge_all);
   int run(hipStream_t s) const;
   void destroy();
@@ -146,6 +151,6 @@ bool fft_factor(int n, FftRadices* r, int schedule = 0);
 // Register slots one thread needs for tile width 2^log2T with the given
 // workgroup size (0 if the tile exceeds kFftMaxTile or 24 slots).
 int fft_emax(const FftRadices& r, int log2T, int threads);
-FftPassGeom pass_geom(const FftRadices& r, int log2T);
+FftPassGeom pass_geom(const FftRadices& r, int log2T, int max_threads = kFftMaxThreads);
 
 }  // namespace cola

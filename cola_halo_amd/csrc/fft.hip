@@ -150,11 +150,11 @@ __device__ inline double kvec_lpt(int i, int n, double box)
 template <KOp OP>
 __device__ inline float2 apply_kop(float2 v, int ix, int iy, int iz, int n, const KOpParams& kp)
 {
-  if constexpr (OP == KOp::PmPoisson) {
+  if constexpr (OP == KOp::PmPoisson || OP == KOp::PmCommon) {
     const int I0 = wave_pm(ix, n), J0 = wave_pm(iy, n), K = iz;
     if (I0 == 0 && J0 == 0 && K == 0) return make_float2(0.0f, 0.0f);
-    const float di = (float)(kp.axis == 0 ? I0 : (kp.axis == 1 ? J0 : K));
-    const float f2 = kp.f1 / (float)(K * K + I0 * I0 + J0 * J0) * di;
+    const float g = kp.f1 / (float)(K * K + I0 * I0 + J0 * J0);
+    const float f2 = OP == KOp::PmPoisson ? g * (float)I0 : g;
     return make_float2(-f2 * v.y, f2 * v.x);
   } else if constexpr (OP == KOp::LptGrad) {
     const int idx = kp.axis == 0 ? ix : (kp.axis == 1 ? iy : iz);
@@ -182,6 +182,9 @@ struct TileArgs {
   int ncols;             // valid columns (kCols) or row pairs (kR2C / kC2R)
   long long sr;          // kCols: stride between positions of one transform
   long long bs;          // kCols: batch stride (blockIdx.y)
+  long long sr_out, bs_out;  // kCols: the same of the outputs
+  long long row_out = 0;     // x pass: row stride of the outputs where it is not nz
+  long long axis_in = 0;     // c2r of force lines: the next component's row
   long long rs_in;       // kR2C: real row stride (floats); kC2R: complex row stride
   long long rs_out;      // kR2C: complex row stride; kC2R: real row stride (floats)
   int nz;                // x pass: columns are (y, kz) pairs with kz < nz (the row stride)
@@ -190,6 +193,12 @@ struct TileArgs {
   int kz_valid = 0;      // x pass: tiles lying wholly in kz >= kz_valid (row padding) return at once
   KOpParams kp;
 };
+
+void set_strides(TileArgs& A, long long sr, long long bs)
+{
+  A.sr = A.sr_out = sr;
+  A.bs = A.bs_out = bs;
+}
 
 // An x-pass tile of 2^log2T columns starting at c0 that holds only padding
 // columns (kz_valid <= kz < nz within one row).
@@ -240,15 +249,19 @@ constexpr int tile_waves_per_eu(int mode, KOp op, int emax, int rs)
   return 6;
 }
 
+// What a column pass of wave numbers multiplies by: the position's wave
+// number on the load, or the column's on the store (both 0: nothing).
+enum YScale : int { kYPlain = 0, kYByPosition = 1, kYByColumn = 2 };
+
 // Workgroup blk of a pass whose grid is nblk workgroups (the kernel's own
 // grid, or one job's share of a batched launch).
-template <int DIR, int MODE, KOp OP, int EMAX, int RS>
-__device__ __forceinline__ void tile_run(const void* __restrict__ in_, void* __restrict__ out_,
-                                         const float2* __restrict__ tw, const TileArgs& A, int blk, int nblk)
+// YS: the pass may scale (yscale); ROW_OUT: its outputs have rows of their own.
+template <int DIR, int MODE, KOp OP, int EMAX, int RS, bool YS = false, bool ROW_OUT = false>
+__device__ __forceinline__ void tile_run(const void* in_, void* out_, const float2* __restrict__ tw, const TileArgs& A,
+                                         int blk, int nblk, int tid, int yscale = kYPlain, bool stage_twiddles = true)
 {
   extern __shared__ float2 smem[];
   const int n = A.P.n;
-  const int tid = threadIdx.x;
   const int nthr = blockDim.x;
   const int log2T = A.log2T;
   const int T = 1 << log2T;
@@ -265,7 +278,8 @@ __device__ __forceinline__ void tile_run(const void* __restrict__ in_, void* __r
   }
   float2* tws = smem;
   float2* lds = smem + n;
-  for (int k = tid; k < n; k += nthr) tws[k] = tw[k];
+  if (stage_twiddles)
+    for (int k = tid; k < n; k += nthr) tws[k] = tw[k];
 
   auto lidx = [&](int r, int c) { return MODE == kCols ? (r << log2T) + c : c * (n + 1) + r; };
   auto split = [&](int u, const FftPass& p, int& c, int& b) {
@@ -305,6 +319,13 @@ __device__ __forceinline__ void tile_run(const void* __restrict__ in_, void* __r
         for (int s = 0; s < R; ++s) {
           const float2* leg = in + (long long)(s * p.m) * A.sr;
           reg[q * R + s] = live ? leg[lane] : make_float2(0.0f, 0.0f);
+        }
+        if (YS && yscale == kYByPosition) {
+#pragma unroll
+          for (int s = 0; s < R; ++s) {
+            const float w = (float)wave_pm(b + s * p.m, n);
+            reg[q * R + s] = make_float2(w * reg[q * R + s].x, w * reg[q * R + s].y);
+          }
         }
         // the operator runs after all of this butterfly's loads are issued
         if constexpr (OP != KOp::None) {
@@ -418,10 +439,16 @@ __device__ __forceinline__ void tile_run(const void* __restrict__ in_, void* __r
       if (u < nb && c0 + c < A.ncols) {
         // last pass: L = n / R = m, so b div L = 0 and the outputs sit at b + t*m
         if (MODE == kCols) {
-          float2* out = static_cast<float2*>(out_) + (long long)batch * A.bs + c0;
-          const unsigned lane = (unsigned)b * (unsigned)A.sr + (unsigned)c;
+          float2* out = static_cast<float2*>(out_) + (long long)batch * A.bs_out + c0;
+          if (ROW_OUT) out += (long long)fdiv((unsigned)(c0 + c), (unsigned)A.nz, A.magNz) * (A.row_out - A.nz);
+          const unsigned lane = (unsigned)b * (unsigned)A.sr_out + (unsigned)c;
+          if (YS && yscale == kYByColumn) {
+            const float w = (float)(c0 + c);
 #pragma unroll
-          for (int t = 0; t < R; ++t) out[(long long)(t * p.m) * A.sr + lane] = reg[q * R + t];
+            for (int t = 0; t < R; ++t) reg[q * R + t] = make_float2(w * reg[q * R + t].x, w * reg[q * R + t].y);
+          }
+#pragma unroll
+          for (int t = 0; t < R; ++t) out[(long long)(t * p.m) * A.sr_out + lane] = reg[q * R + t];
         } else {
           float* out = static_cast<float*>(out_) + (2LL * c0) * A.rs_out;
           const unsigned lane = (unsigned)(2 * c) * (unsigned)A.rs_out + (unsigned)b;
@@ -492,10 +519,140 @@ template <int DIR, int MODE, KOp OP, int EMAX, int RS>
 __global__ void __launch_bounds__(kFftMaxThreads) __attribute__((amdgpu_waves_per_eu(tile_waves_per_eu(MODE, OP, EMAX, RS))))
 fft_tile(const void* __restrict__ in_, void* __restrict__ out_, const float2* __restrict__ tw, TileArgs A)
 {
-  tile_run<DIR, MODE, OP, EMAX, RS>(in_, out_, tw, A, blockIdx.x, gridDim.x);
+  // (the operators of the force spectra write lines of three)
+  constexpr bool row_out = OP == KOp::PmPoisson || OP == KOp::PmCommon;
+  tile_run<DIR, MODE, OP, EMAX, RS, false, row_out>(in_, out_, tw, A, blockIdx.x, gridDim.x, threadIdx.x);
 }
 
-// ---- fused x pass: forward x FFT, then per axis Poisson + inverse x FFT ----
+// ---- z c2r of the three force components of a line ---------------------------
+// One workgroup: T pairs of lines, whose three half spectra (rows axis_in
+// apart) become one line of records F[z][3] in their place.  A third of the
+// threads takes each component: its two rows are packed into one complex
+// transform as in the row pass; the last pass leaves its component of the
+// records in LDS, and the lines go out whole (storing a component every 12
+// bytes from registers took 3.88 ms at 768^3).  The readout then gathers one
+// record per CIC corner, 4 grid lines per particle instead of 12: the z pass
+// takes 3.45 ms for the three launches' 3.03 at 768^3 (0.83 for 1.09 at 480^3)
+// and the readout of 256^3 particles 1.08 for 2.16.
+template <int EMAX, int RS>
+__device__ __forceinline__ void c2r3_run(float* data, const float2* __restrict__ tw, const TileArgs& A, int blk)
+{
+  extern __shared__ float2 smem[];
+  const int n = A.P.n;
+  const int log2T = A.log2T;
+  const int c0 = blk << log2T;
+  const int nthr = (int)blockDim.x / 3;
+  const int axis = __builtin_amdgcn_readfirstlane((int)threadIdx.x / nthr);  // whole wavefronts: nthr is a multiple of 64
+  const int tid = (int)threadIdx.x - axis * nthr;
+  float2* const lds = smem + n + axis * ((n + 1) << log2T);
+  float* const stage = reinterpret_cast<float*>(smem + n);  // the lines' records, over the three tiles
+  for (int k = threadIdx.x; k < n; k += (int)blockDim.x) smem[k] = tw[k];
+  const int np_ = A.P.npass;
+  const int h = n / 2;
+  const float2* in = reinterpret_cast<const float2*>(data) + (2LL * c0) * A.rs_in + axis * A.axis_in;
+
+  for (int pi = 0; pi < np_; ++pi) {
+    radix_dispatch<RS>(A.P.pass[pi].R, [&](auto Rc) {
+      constexpr int R = decltype(Rc)::value;
+      const FftPass& p = A.P.pass[pi];
+      const int nb = p.m << log2T;
+      const bool last = pi == np_ - 1;
+      float2 reg[EMAX];
+      if (pi == 0) {
+#pragma unroll
+        for (int q = 0; q < EMAX / R; ++q) {
+          const int u = tid + q * nthr;
+          const int c = (int)fdiv((unsigned)u, (unsigned)p.m, p.magM), b = u - c * p.m;
+          const bool live = u < nb && c0 + c < A.ncols;
+          const unsigned rowa = (unsigned)(2 * c) * (unsigned)A.rs_in, rowb = rowa + (unsigned)A.rs_in;
+#pragma unroll
+          for (int s = 0; s < R; ++s) {
+            const int r = b + s * p.m;
+            float2 v = make_float2(0.0f, 0.0f);
+            if (live) {
+              // Hermitian extension of both half spectra; Im of kz = 0, n/2 dropped
+              const unsigned rr = (unsigned)(r <= h ? r : n - r);
+              float2 a = in[rowa + rr], bb = in[rowb + rr];
+              if (r == 0 || r == h) {
+                a.y = 0.0f;
+                bb.y = 0.0f;
+              } else if (r > h) {
+                a.y = -a.y;
+                bb.y = -bb.y;
+              }
+              v = make_float2(a.x - bb.y, a.y + bb.x);
+            }
+            reg[q * R + s] = v;
+          }
+        }
+      } else {
+#pragma unroll
+        for (int q = 0; q < EMAX / R; ++q) {
+          const int u = tid + q * nthr;
+          if (u < nb) {
+            const int c = (int)fdiv((unsigned)u, (unsigned)p.m, p.magM), b = u - c * p.m;
+#pragma unroll
+            for (int s = 0; s < R; ++s) reg[q * R + s] = lds[c * (n + 1) + b + s * p.m];
+          }
+        }
+        __syncthreads();
+      }
+#pragma unroll
+      for (int q = 0; q < EMAX / R; ++q) {
+        const int u = tid + q * nthr;
+        if (u < nb) {
+          const int c = (int)fdiv((unsigned)u, (unsigned)p.m, p.magM), b = u - c * p.m;
+          const int i = (int)fdiv((unsigned)b, (unsigned)p.L, p.magL);
+          const int j = b - i * p.L;
+          if (p.L > 1) {
+#pragma unroll
+            for (int s = 1; s < R; ++s) reg[q * R + s] = twiddle<1>(reg[q * R + s], smem[s * j * p.twstep]);
+          }
+          dft<R, 1>(&reg[q * R]);
+          if (!last) {
+            const int o = i * R * p.L + j;
+#pragma unroll
+            for (int t = 0; t < R; ++t) lds[c * (n + 1) + o + t * p.L] = reg[q * R + t];
+          } else {
+            float* const o = stage + 6 * c * n + 3 * b + axis;
+#pragma unroll
+            for (int t = 0; t < R; ++t) {
+              o[3 * (t * p.m)] = reg[q * R + t].x;
+              o[3 * (t * p.m + n)] = reg[q * R + t].y;
+            }
+          }
+        }
+      }
+      __syncthreads();
+    });
+  }
+  // the lines' records, contiguous: 16 bytes a lane (8 where n is no multiple of 4)
+  const int lines = 2 * min(1 << log2T, A.ncols - c0);
+  auto copy = [&](auto v) {
+    using V = decltype(v);
+    constexpr int W = sizeof(V) / sizeof(float);
+    const int per = 3 * n / W;
+    for (int l = 0; l < lines; ++l) {
+      V* const o = reinterpret_cast<V*>(data + (2LL * c0 + l) * A.rs_out);
+      const V* const st = reinterpret_cast<const V*>(stage + 3 * l * n);
+      for (int k = threadIdx.x; k < per; k += (int)blockDim.x) o[k] = st[k];
+    }
+  };
+  if (n % 4 == 0)
+    copy(float4{});
+  else
+    copy(float2{});
+}
+
+template <int EMAX, int RS>
+__global__ void __launch_bounds__(kFftMaxThreads)
+    __attribute__((amdgpu_waves_per_eu(tile_waves_per_eu(kC2R, KOp::None, EMAX, RS))))
+fft_c2r3(float* data, const float2* __restrict__ tw, TileArgs A)
+{
+  c2r3_run<EMAX, RS>(data, tw, A, blockIdx.x);
+}
+
+// ---- fused x pass: forward x FFT, then Poisson + inverse x FFT twice ---------
 // Column layout helpers (LDS [r][c], column fastest).
 struct ColCtx {
   float2* lds;
@@ -559,17 +716,121 @@ __device__ inline void col_load_lds(float2 (&reg)[EMAX], const FftPass& p, const
 }
 
 
+// ---- y inverse of the force spectra ------------------------------------------
+// The x pass leaves two spectra: F_x and the common one G = i f1 / k^2 delta
+// (after the x inverse), of which F_y = n_y G and F_z = n_z G.  n_z is
+// constant along y, so F_z's transform is n_z times that of G: a workgroup
+// whose job has a second output loads its tile of G once into registers and
+// transforms it twice, unscaled (written times n_z to out2), then times n_y
+// (in place).  Two grids in and three out here and one in and two out in the
+// x pass, where three in and three out and one in and three out were: bound
+// by the HBM as before, at 768^3 the x pass takes 2.98 ms for 3.52, the two y
+// launches 2.41 for the three's 2.45; 480^3 0.90 for 1.00 and 0.76 for 1.16.
+// (Reading the tile a second time instead of keeping it: 4.18 ms at 768^3.)
+template <int EMAX, int RS>
+__device__ __forceinline__ void yinv_run(const float2* in, float2* out, float2* out2, const float2* __restrict__ tw,
+                                         const TileArgs& A, int blk, int nblk)
+{
+  extern __shared__ float2 smem[];
+  const int n = A.P.n;
+  const int nthr = blockDim.x;
+  const int log2T = A.log2T;
+  const int lb = xcd_group_remap(blk, nblk, A.xgroup);
+  const int batch = lb / A.tpb_pad;
+  const int tile = lb - batch * A.tpb_pad;
+  if (tile >= A.tpb) return;  // padding workgroup (before any barrier)
+  const int c0 = tile << log2T;
+  for (int k = threadIdx.x; k < n; k += nthr) smem[k] = tw[k];
+  const int np_ = A.P.npass;
+  const int tmask = (1 << log2T) - 1;
+  const long long base = (long long)batch * A.bs + c0;
+  using Tile = float2[EMAX];
+  Tile keep;
+  radix_dispatch<RS>(A.P.pass[0].R, [&](auto Rc) {
+    constexpr int R = decltype(Rc)::value;
+    const FftPass& p = A.P.pass[0];
+#pragma unroll
+    for (int q = 0; q < EMAX / R; ++q) {
+      const int u = (int)threadIdx.x + q * nthr;
+      const int c = u & tmask, b = u >> log2T;
+      const bool live = u < (p.m << log2T) && c0 + c < A.ncols;
+      const unsigned lane = (unsigned)b * (unsigned)A.sr + (unsigned)c;
+#pragma unroll
+      for (int s = 0; s < R; ++s)
+        keep[q * R + s] = live ? in[base + (long long)(s * p.m) * A.sr + lane] : make_float2(0.0f, 0.0f);
+    }
+  });
+  const int reps = out2 ? 2 : 1;
+#pragma unroll 1
+  for (int rep = 0; rep < reps; ++rep) {
+    // indexes are computed anew in each repetition: kept across it they spill
+    int tid = threadIdx.x;
+    asm volatile("" : "+v"(tid));
+    const ColCtx x{smem + n, smem, tid, nthr, log2T};
+    float2* const o = (out2 && rep == 0 ? out2 : out) + base;
+    for (int pi = 0; pi < np_; ++pi) {
+      const bool last = pi == np_ - 1;
+      radix_dispatch<RS>(A.P.pass[pi].R, [&](auto Rc) {
+        constexpr int R = decltype(Rc)::value;
+        const FftPass& p = A.P.pass[pi];
+        Tile reg;
+        if (pi == 0) {
+#pragma unroll
+          for (int q = 0; q < EMAX / R; ++q) {
+            const int b = (tid + q * nthr) >> log2T;
+#pragma unroll
+            for (int s = 0; s < R; ++s) {
+              const float w = rep == 1 ? (float)wave_pm(b + s * p.m, n) : 1.0f;
+              const float2 v = keep[q * R + s];
+              reg[q * R + s] = make_float2(w * v.x, w * v.y);
+            }
+          }
+        } else {
+          col_load_lds<R, EMAX>(reg, p, x);
+          __syncthreads();
+        }
+        col_compute<R, EMAX, 1>(reg, p, x);
+        if (!last) {
+          col_store_lds<R, EMAX>(reg, p, x);
+        } else {
+#pragma unroll
+          for (int q = 0; q < EMAX / R; ++q) {
+            const int u = tid + q * nthr;
+            const int c = u & tmask, b = u >> log2T;
+            if (u < (p.m << log2T) && c0 + c < A.ncols) {
+              const float w = out2 && rep == 0 ? (float)(c0 + c) : 1.0f;
+              const unsigned lane = (unsigned)b * (unsigned)A.sr + (unsigned)c;
+#pragma unroll
+              for (int t = 0; t < R; ++t)
+                o[(long long)(t * p.m) * A.sr + lane] = make_float2(w * reg[q * R + t].x, w * reg[q * R + t].y);
+            }
+          }
+        }
+      });
+      if (!last) __syncthreads();
+    }
+  }
+}
+
+template <int EMAX, int RS>
+__global__ void __launch_bounds__(kFftMaxThreads)
+    __attribute__((amdgpu_waves_per_eu(tile_waves_per_eu(kCols, KOp::None, EMAX, RS))))
+fft_yinv(const float2* in, float2* out, float2* out2, const float2* __restrict__ tw, TileArgs A)
+{
+  yinv_run<EMAX, RS>(in, out, out2, tw, A, blockIdx.x, gridDim.x);
+}
+
 // One workgroup: T columns (y, kz) of the half spectrum after the forward z
-// and y passes.  Forward x FFT (plan A.P, radix R_LAST last), then for each
-// axis the PM Poisson operator (pm.c:322-346) and the inverse x FFT with the
-// radices in reverse order (A.P2, radix R_LAST first): the forward's last
-// butterflies are exactly the inverse's first, so delta(k) stays in registers
-// and never goes to memory.  Outputs: the three x-inverted force spectra.
+// and y passes.  Forward x FFT (plan A.P, radix R_LAST last), then the PM
+// Poisson operator (pm.c:322-346) and the inverse x FFT with the radices in
+// reverse order (A.P2, radix R_LAST first): the forward's last butterflies
+// are exactly the inverse's first, so delta(k) stays in registers and never
+// goes to memory.  Outputs: the x-inverted spectrum of F_x and the common
+// spectrum of F_y and F_z (yinv_run scales it by n_y and n_z).
 template <int R_LAST, int EMAX, int RS>
 __device__ __forceinline__ void fused_run(const float2* __restrict__ in, float2* __restrict__ out0,
-                                          float2* __restrict__ out1, float2* __restrict__ out2,
-                                          const float2* __restrict__ tw, const TileArgs& A, const FftRadices& Pinv,
-                                          int blk, int nblk)
+                                          float2* __restrict__ out1, const float2* __restrict__ tw, const TileArgs& A,
+                                          const FftRadices& Pinv, int blk, int nblk)
 {
   extern __shared__ float2 smem[];
   const int n = A.P.n;
@@ -645,8 +906,7 @@ __device__ __forceinline__ void fused_run(const float2* __restrict__ in, float2*
   // Two inverse transforms instead of three: along a column (fixed ky, kz)
   // the y and z force spectra are n_y and n_z times the same i f1 / k^2
   // delta (pm.c:336-341 with n_y, n_z constant in x), and the x transform is
-  // linear, so transform 1 is that common spectrum and its outputs are
-  // written twice, scaled by n_y and by n_z; transform 0 carries n_x.
+  // linear, so transform 1 is that common spectrum; transform 0 carries n_x.
 #pragma unroll 1
   for (int axis = 0; axis < 2; ++axis) {
     Tile reg;
@@ -689,22 +949,11 @@ __device__ __forceinline__ void fused_run(const float2* __restrict__ in, float2*
             const int u = tid + q * nthr;
             const int c = u & tmask, b = u >> log2T;
             if (u < nb && c0 + c < A.ncols) {
-              const unsigned lane = (unsigned)b * (unsigned)A.sr + (unsigned)c;
-              if (axis == 0) {
+              const int iy = (int)fdiv((unsigned)(c0 + c), (unsigned)A.nz, A.magNz);
+              float2* out = (axis == 0 ? out0 : out1) + c0 + (long long)iy * (A.row_out - A.nz);
+              const unsigned lane = (unsigned)b * (unsigned)A.sr_out + (unsigned)c;
 #pragma unroll
-                for (int t = 0; t < R; ++t) out0[c0 + (long long)(t * p.m) * A.sr + lane] = r2[q * R + t];
-              } else {
-                const int col = c0 + c;
-                const int iy = (int)fdiv((unsigned)col, (unsigned)A.nz, A.magNz);
-                const float fy = (float)wave_pm(iy, n), fz = (float)(col - iy * A.nz);
-#pragma unroll
-                for (int t = 0; t < R; ++t) {
-                  const float2 v = r2[q * R + t];
-                  const long long at = c0 + (long long)(t * p.m) * A.sr + lane;
-                  out1[at] = make_float2(fy * v.x, fy * v.y);
-                  out2[at] = make_float2(fz * v.x, fz * v.y);
-                }
-              }
+              for (int t = 0; t < R; ++t) out[(long long)(t * p.m) * A.sr_out + lane] = r2[q * R + t];
             }
           }
         }
@@ -717,9 +966,9 @@ __device__ __forceinline__ void fused_run(const float2* __restrict__ in, float2*
 template <int R_LAST, int EMAX, int RS>
 __global__ void __launch_bounds__(kFftMaxThreads)
 fft_x_fused(const float2* __restrict__ in, float2* __restrict__ out0, float2* __restrict__ out1,
-            float2* __restrict__ out2, const float2* __restrict__ tw, TileArgs A, FftRadices Pinv)
+            const float2* __restrict__ tw, TileArgs A, FftRadices Pinv)
 {
-  fused_run<R_LAST, EMAX, RS>(in, out0, out1, out2, tw, A, Pinv, blockIdx.x, gridDim.x);
+  fused_run<R_LAST, EMAX, RS>(in, out0, out1, tw, A, Pinv, blockIdx.x, gridDim.x);
 }
 
 unsigned magic_for(int d)
@@ -733,6 +982,8 @@ size_t tile_lds_bytes(int mode, int n, int log2T)
   const size_t data = mode == kCols ? ((size_t)n << log2T) : ((size_t)(n + 1) << log2T);
   return sizeof(float2) * (data + n);
 }
+
+size_t c2r3_lds_bytes(int n, int log2T) { return sizeof(float2) * (3 * ((size_t)(n + 1) << log2T) + n); }
 
 template <int DIR, int MODE, KOp OP, int E, int RS>
 int launch_e(dim3 grid, int threads, size_t lds, hipStream_t s, const void* in, void* out, const float2* tw,
@@ -789,6 +1040,7 @@ void set_groups(TileArgs& A, int tpb, int group)
 struct TileJob {
   const void* in;
   void* out;
+  void* out2;  // y inverse: the second output, or null
   const float2* tw;
   TileArgs A;
   int blocks;
@@ -796,7 +1048,7 @@ struct TileJob {
 
 struct FusedJob {
   const float2* in;
-  float2* out[3];
+  float2* out[2];
   const float2* tw;
   TileArgs A;
   FftRadices Pinv;
@@ -812,7 +1064,31 @@ fft_tile_jobs(const TileJob* __restrict__ jobs, const int* __restrict__ start, i
   const TileJob& J = jobs[j];
   const int lb = (int)blockIdx.x - start[j];
   if (lb >= J.blocks) return;  // alignment padding (before any barrier)
-  tile_run<DIR, MODE, KOp::None, EMAX, RS>(J.in, J.out, J.tw, J.A, lb, J.blocks);
+  tile_run<DIR, MODE, KOp::None, EMAX, RS>(J.in, J.out, J.tw, J.A, lb, J.blocks, threadIdx.x);
+}
+
+// (6 waves per SIMD at 8 values per thread: with 8 the tables' arguments spill)
+template <int EMAX, int RS>
+__global__ void __launch_bounds__(kFftMaxThreads)
+    __attribute__((amdgpu_waves_per_eu(tile_waves_per_eu(kC2R, KOp::None, EMAX, RS))))
+fft_yinv_jobs(const TileJob* __restrict__ jobs, const int* __restrict__ start, int njobs)
+{
+  const int j = batch_find(start, njobs, blockIdx.x);
+  const TileJob& J = jobs[j];
+  const int lb = (int)blockIdx.x - start[j];
+  if (lb >= J.blocks) return;
+  yinv_run<EMAX, RS>(static_cast<const float2*>(J.in), static_cast<float2*>(J.out), static_cast<float2*>(J.out2), J.tw,
+                     J.A, lb, J.blocks);
+}
+
+template <int EMAX, int RS>
+__global__ void __launch_bounds__(kFftMaxThreads)
+    __attribute__((amdgpu_waves_per_eu(tile_waves_per_eu(kC2R, KOp::None, EMAX, RS))))
+fft_c2r3_jobs(const TileJob* __restrict__ jobs, const int* __restrict__ start, int njobs)
+{
+  const int j = batch_find(start, njobs, blockIdx.x);
+  const TileJob& J = jobs[j];
+  c2r3_run<EMAX, RS>(static_cast<float*>(J.out), J.tw, J.A, (int)blockIdx.x - start[j]);
 }
 
 template <int EMAX, int RS>
@@ -826,7 +1102,7 @@ fft_x_fused_jobs(const FusedJob* __restrict__ jobs, const int* __restrict__ star
   // the last forward radix is a template constant of the fused pass
   // (FftPlan::can_fuse admits 3, 4, 5 and 8)
   auto run = [&](auto Rc) {
-    fused_run<decltype(Rc)::value, EMAX, RS>(J.in, J.out[0], J.out[1], J.out[2], J.tw, J.A, J.Pinv, lb, J.blocks);
+    fused_run<decltype(Rc)::value, EMAX, RS>(J.in, J.out[0], J.out[1], J.tw, J.A, J.Pinv, lb, J.blocks);
   };
   switch (J.A.P.pass[J.A.P.npass - 1].R) {
     case 3: run(std::integral_constant<int, 3>{}); break;
@@ -921,13 +1197,13 @@ int fft_emax(const FftRadices& r, int log2T, int threads)
 // Threads for a tile: the fewest (a multiple of 64, at most
 // kFftMaxThreads) that keep every thread within 8 register slots, else within
 // the smallest slot count reachable.
-FftPassGeom pass_geom(const FftRadices& r, int log2T)
+FftPassGeom pass_geom(const FftRadices& r, int log2T, int max_threads)
 {
   FftPassGeom best;
   best.log2T = log2T;
   const long long elems = (long long)r.n << log2T;
   const int t0 = (int)std::max<long long>(64, std::min<long long>(kFftMaxThreads, ((elems / 8 + 63) / 64) * 64));
-  for (int t = t0; t <= kFftMaxThreads; t += 64) {
+  for (int t = std::min(t0, max_threads); t <= max_threads; t += 64) {
     const int e = fft_emax(r, log2T, t);
     if (e == 0) continue;
     if (best.emax == 0 || e < best.emax) {
@@ -972,6 +1248,28 @@ int FftPlan::init(int n_, int log2T_cols, int log2T_rows, bool pad_rows, int log
   gy = pick(log2T_cols >= 0 ? log2T_cols : std::min(3, cap_log2(n)), n / 2 + 1);
   grows = pick(log2T_rows >= 0 ? log2T_rows : 1, (long long)n * n / 2);
   if (gx.emax == 0 || gy.emax == 0 || grows.emax == 0) return kErrUnsupported;
+  // the z c2r of three components: the row pairs asked for, or one pair (768^3
+  // 3.45 ms against 3.66 of two; 384^3 0.40, 0.45; 270^3 0.160, 0.180) unless
+  // that leaves over half of its threads idle, then the fewest with the least
+  // idle (192^3: two 0.049 against one 0.062; 480^3: four 0.83 against 0.96 of
+  // two and 1.11 of one), as three groups of threads and their tiles allow
+  double best = 0.0;
+  for (int l = log2T_rows >= 0 ? grows.log2T : 0; l >= 0 && l <= 2;) {
+    const FftPassGeom g =
+        c2r3_lds_bytes(n, l) <= 160 * 1024 ? pass_geom(rad, l, kFftC2r3Threads) : FftPassGeom{};
+    const double busy = g.emax ? (double)((long long)n << l) / (8.0 * g.threads) : 0.0;
+    if (busy > best) {
+      best = busy;
+      gz3 = g;
+    }
+    if (log2T_rows >= 0) {
+      if (gz3.emax) break;
+      --l;
+    } else {
+      if (l == 0 && best >= 0.5) break;
+      ++l;
+    }
+  }
   std::vector<float2> tw(n);
   for (int k = 0; k < n; ++k) {
     const double a = -2.0 * kPiD * (double)k / (double)n;
@@ -1010,8 +1308,7 @@ int FftPlan::r2c(float* data, hipStream_t s) const
   // y: columns kz of each x plane
   A.log2T = gy.log2T;
   A.ncols = (int)nz;
-  A.sr = np_;
-  A.bs = (long long)n * np_;
+  set_strides(A, np_, (long long)n * np_);
   set_groups(A, grid_x(nz, gy.log2T), xgroup);
   mark(1, 1);
   COLA_TRY((launch_tile<-1, kCols, KOp::None>(gy, dim3(A.tpb_pad * n), s, cdata, cdata, d_tw, A)));
@@ -1020,8 +1317,7 @@ int FftPlan::r2c(float* data, hipStream_t s) const
   const long long ncols = (long long)n * np_;
   A.log2T = gx.log2T;
   A.ncols = (int)ncols;
-  A.sr = ncols;
-  A.bs = 0;
+  set_strides(A, ncols, 0);
   A.nz = (int)np_;
   A.kz_valid = np_ > nz ? (int)nz : 0;
   set_groups(A, grid_x(ncols, gx.log2T), xgroup);
@@ -1054,7 +1350,7 @@ static FftRadices reversed(const FftRadices& r)
 
 template <int RL, int E, int RS>
 static int launch_fused_e(const FftPassGeom& g, int grid, hipStream_t s, const float2* in, float2* o0, float2* o1,
-                          float2* o2, const float2* tw, const TileArgs& A, const FftRadices& Pinv)
+                          const float2* tw, const TileArgs& A, const FftRadices& Pinv)
 {
   static bool attr = false;
   if (!attr) {
@@ -1063,20 +1359,20 @@ static int launch_fused_e(const FftPassGeom& g, int grid, hipStream_t s, const f
     attr = true;
   }
   hipLaunchKernelGGL((fft_x_fused<RL, E, RS>), dim3(grid), dim3(g.threads), tile_lds_bytes(kCols, A.P.n, g.log2T), s,
-                     in, o0, o1, o2, tw, A, Pinv);
+                     in, o0, o1, tw, A, Pinv);
   return kOk;
 }
 
 template <int RL>
 static int launch_fused_r(const FftPassGeom& g, int grid, hipStream_t s, const float2* in, float2* o0, float2* o1,
-                          float2* o2, const float2* tw, const TileArgs& A, const FftRadices& Pinv)
+                          const float2* tw, const TileArgs& A, const FftRadices& Pinv)
 {
   if (g.emax <= 8) {
     if constexpr (RL == 3 || RL == 4 || RL == 8)
-      if (radices_348(A.P)) return launch_fused_e<RL, 8, kRs348>(g, grid, s, in, o0, o1, o2, tw, A, Pinv);
-    return launch_fused_e<RL, 8, kRsAll>(g, grid, s, in, o0, o1, o2, tw, A, Pinv);
+      if (radices_348(A.P)) return launch_fused_e<RL, 8, kRs348>(g, grid, s, in, o0, o1, tw, A, Pinv);
+    return launch_fused_e<RL, 8, kRsAll>(g, grid, s, in, o0, o1, tw, A, Pinv);
   }
-  return launch_fused_e<RL, 12, kRsAll>(g, grid, s, in, o0, o1, o2, tw, A, Pinv);
+  return launch_fused_e<RL, 12, kRsAll>(g, grid, s, in, o0, o1, tw, A, Pinv);
 }
 
 bool FftPlan::can_fuse() const
@@ -1088,19 +1384,23 @@ bool FftPlan::can_fuse() const
 
 namespace {
 
-// The launches of FftPlan::forces (fused path) for one grid: z r2c, y
-// forward, fused x, then per axis y inverse and z c2r.
+// The launches of FftPlan::forces for one grid: z r2c, y forward, x (fused
+// where the plan can), y inverse of F_x and of the common spectrum, z c2r of
+// the three components.
 struct ForceJobs {
-  TileJob zr2c, yfwd, yinv[3], zc2r[3];
+  TileJob zr2c, yfwd, yinv[2];
+  TileJob zc2r, zslot[3];  // records, or the components apart
   FusedJob x;
 };
 
-void make_force_jobs(const FftPlan& P, float* density, float* const out[3], const KOpParams& kp, ForceJobs* J)
+void make_force_jobs(const FftPlan& P, float* density, float* force, const KOpParams& kp, ForceJobs* J)
 {
   const int n = P.n;
   const long long nz = n / 2 + 1, np_ = P.nzp;
   const int npairs = n * n / 2;
   float2* cdata = reinterpret_cast<float2*>(density);
+  float2* cforce = reinterpret_cast<float2*>(force);
+  const long long frow = 3 * np_;  // a line of force: three spectra, then n records
   TileArgs A;
   A.P = P.rad;
   A.kp = kp;
@@ -1112,47 +1412,84 @@ void make_force_jobs(const FftPlan& P, float* density, float* const out[3], cons
   A.ncols = npairs;
   A.rs_in = 2 * np_;
   A.rs_out = np_;
-  J->zr2c = TileJob{density, cdata, P.d_tw, A, grid_x(npairs, P.grows.log2T)};
+  J->zr2c = TileJob{density, cdata, nullptr, P.d_tw, A, grid_x(npairs, P.grows.log2T)};
   A.log2T = P.gy.log2T;
   A.ncols = (int)nz;
-  A.sr = np_;
-  A.bs = (long long)n * np_;
+  set_strides(A, np_, (long long)n * np_);
   set_groups(A, grid_x(nz, P.gy.log2T), P.xgroup);
-  J->yfwd = TileJob{cdata, cdata, P.d_tw, A, A.tpb_pad * n};
-  // fused x: forward, Poisson per axis, inverse (row padding tiles return at once)
+  J->yfwd = TileJob{cdata, cdata, nullptr, P.d_tw, A, A.tpb_pad * n};
+  // x: forward, Poisson, inverse (row padding tiles return at once)
   const long long ncols = (long long)n * np_;
   A.log2T = P.gx.log2T;
   A.ncols = (int)ncols;
-  A.sr = ncols;
-  A.bs = 0;
+  set_strides(A, ncols, 0);
+  A.sr_out = n * frow;
+  A.row_out = frow;
   A.kz_valid = np_ > nz ? (int)nz : 0;
   set_groups(A, grid_x(ncols, P.gx.log2T), P.xgroup);
   FusedJob& x = J->x;
   x.in = cdata;
-  for (int a = 0; a < 3; ++a) x.out[a] = reinterpret_cast<float2*>(out[a]);
+  for (int a = 0; a < 2; ++a) x.out[a] = cforce + a * np_;
   x.tw = P.d_tw;
   x.A = A;
   x.Pinv = reversed(P.rad);
   x.blocks = A.tpb_pad;
-  // per axis: y inverse, z c2r
-  for (int a = 0; a < 3; ++a) {
-    TileArgs B;
-    B.P = P.rad;
-    B.kz_valid = 0;
-    B.log2T = P.gy.log2T;
-    B.ncols = (int)nz;
-    B.sr = np_;
-    B.bs = (long long)n * np_;
-    set_groups(B, grid_x(nz, P.gy.log2T), P.xgroup);
-    J->yinv[a] = TileJob{x.out[a], x.out[a], P.d_tw, B, B.tpb_pad * n};
-    B.log2T = P.grows.log2T;
-    B.ncols = npairs;
-    B.rs_in = np_;
-    B.rs_out = 2 * np_;
-    B.zero_pad = np_ == nz;
-    J->zc2r[a] = TileJob{x.out[a], out[a], P.d_tw, B, grid_x(npairs, P.grows.log2T)};
-  }
+  TileArgs B;
+  B.P = P.rad;
+  B.kz_valid = 0;
+  B.log2T = P.gy.log2T;
+  B.ncols = (int)nz;
+  set_strides(B, frow, n * frow);
+  set_groups(B, grid_x(nz, P.gy.log2T), P.xgroup);
+  J->yinv[0] = TileJob{x.out[0], x.out[0], nullptr, P.d_tw, B, B.tpb_pad * n};
+  J->yinv[1] = TileJob{x.out[1], x.out[1], cforce + 2 * np_, P.d_tw, B, B.tpb_pad * n};
+  B.log2T = P.gz3.log2T;
+  B.ncols = npairs;
+  B.rs_in = frow;
+  B.axis_in = np_;
+  B.rs_out = 2 * frow;
+  J->zc2r = TileJob{force, force, nullptr, P.d_tw, B, grid_x(npairs, P.gz3.log2T)};
+  B.log2T = P.grows.log2T;
+  for (int a = 0; a < 3; ++a)
+    J->zslot[a] = TileJob{cforce + a * np_, force + 2 * a * np_, nullptr, P.d_tw, B, grid_x(npairs, P.grows.log2T)};
 }
+
+// The launchers of the y inverse and the z c2r, one grid or a batch of jobs
+// (start: the jobs' first workgroups), by register tile and radix set.
+template <template <int, int> class K, class... Args>
+int launch_variant(int emax, bool rs348, dim3 grid, int threads, size_t lds, hipStream_t s, Args... args)
+{
+  auto go = [&](auto k) -> int {
+    using L = decltype(k);
+    static bool attr = false;
+    if (!attr) {
+      COLA_HIP(hipFuncSetAttribute(L::fn(), hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
+      attr = true;
+    }
+    L::run(grid, threads, lds, s, args...);
+    return kOk;
+  };
+  if (emax <= 8) return rs348 ? go(K<8, kRs348>{}) : go(K<8, kRsAll>{});
+  if (emax <= 12) return go(K<12, kRsAll>{});
+  if (emax <= 16) return go(K<16, kRsAll>{});
+  return go(K<24, kRsAll>{});
+}
+
+#define COLA_FFT_VARIANT(NAME, KERNEL)                                                              \
+  template <int E, int RS>                                                                          \
+  struct NAME {                                                                                     \
+    static const void* fn() { return reinterpret_cast<const void*>(&KERNEL<E, RS>); }               \
+    template <class... Args>                                                                        \
+    static void run(dim3 grid, int threads, size_t lds, hipStream_t s, Args... args)                \
+    {                                                                                               \
+      hipLaunchKernelGGL((KERNEL<E, RS>), grid, dim3(threads), lds, s, args...);                    \
+    }                                                                                               \
+  };
+COLA_FFT_VARIANT(YInv, fft_yinv)
+COLA_FFT_VARIANT(YInvJobs, fft_yinv_jobs)
+COLA_FFT_VARIANT(C2R3, fft_c2r3)
+COLA_FFT_VARIANT(C2R3Jobs, fft_c2r3_jobs)
+#undef COLA_FFT_VARIANT
 
 template <int DIR, int MODE, int E, int RS>
 int launch_jobs_e(const FftBatchStage& st, hipStream_t s)
@@ -1196,28 +1533,23 @@ int launch_fused_jobs_e(const FftBatchStage& st, hipStream_t s)
 
 }  // namespace
 
-int FftPlan::forces(float* density, float* const out[3], const KOpParams& kp, hipStream_t s) const
+int FftPlan::forces(float* density, float* force, const KOpParams& kp, bool records, hipStream_t s) const
 {
-  if (!can_fuse()) {
-    COLA_TRY(r2c(density, s));
-    KOpParams k = kp;
-    for (int a = 0; a < 3; ++a) {
-      k.axis = a;
-      COLA_TRY(c2r(reinterpret_cast<const float2*>(density), out[a], KOp::PmPoisson, k, s));
-    }
-    return kOk;
+  if (records && gz3.emax == 0) {
+    set_error("force transforms: the grid's rows exceed a workgroup's LDS");
+    return kErrUnsupported;
   }
   auto mark = [&](int pass, int begin) {
     if (hook) hook(hook_user, pass, begin);
   };
   ForceJobs J;
-  make_force_jobs(*this, density, out, kp, &J);
+  make_force_jobs(*this, density, force, kp, &J);
   auto tile = [&](auto dir, auto mode, const FftPassGeom& g, const TileJob& t) {
     return launch_tile<decltype(dir)::value, decltype(mode)::value, KOp::None>(g, dim3(t.blocks), s, t.in, t.out,
                                                                               t.tw, t.A);
   };
   using Fwd = std::integral_constant<int, -1>;
-  using Inv = std::integral_constant<int, 1>;
+  const bool rs348 = radices_348(rad);
   mark(0, 1);
   COLA_TRY(tile(Fwd{}, std::integral_constant<int, kR2C>{}, grows, J.zr2c));
   mark(0, 0);
@@ -1225,38 +1557,67 @@ int FftPlan::forces(float* density, float* const out[3], const KOpParams& kp, hi
   COLA_TRY(tile(Fwd{}, std::integral_constant<int, kCols>{}, gy, J.yfwd));
   mark(1, 0);
   const FusedJob& x = J.x;
-  mark(6, 1);
-  switch (rad.pass[rad.npass - 1].R) {
-    case 3: COLA_TRY(launch_fused_r<3>(gx, x.blocks, s, x.in, x.out[0], x.out[1], x.out[2], d_tw, x.A, x.Pinv)); break;
-    case 4: COLA_TRY(launch_fused_r<4>(gx, x.blocks, s, x.in, x.out[0], x.out[1], x.out[2], d_tw, x.A, x.Pinv)); break;
-    case 5: COLA_TRY(launch_fused_r<5>(gx, x.blocks, s, x.in, x.out[0], x.out[1], x.out[2], d_tw, x.A, x.Pinv)); break;
-    default: COLA_TRY(launch_fused_r<8>(gx, x.blocks, s, x.in, x.out[0], x.out[1], x.out[2], d_tw, x.A, x.Pinv)); break;
+  if (can_fuse()) {
+    mark(6, 1);
+    switch (rad.pass[rad.npass - 1].R) {
+      case 3: COLA_TRY(launch_fused_r<3>(gx, x.blocks, s, x.in, x.out[0], x.out[1], d_tw, x.A, x.Pinv)); break;
+      case 4: COLA_TRY(launch_fused_r<4>(gx, x.blocks, s, x.in, x.out[0], x.out[1], d_tw, x.A, x.Pinv)); break;
+      case 5: COLA_TRY(launch_fused_r<5>(gx, x.blocks, s, x.in, x.out[0], x.out[1], d_tw, x.A, x.Pinv)); break;
+      default: COLA_TRY(launch_fused_r<8>(gx, x.blocks, s, x.in, x.out[0], x.out[1], d_tw, x.A, x.Pinv)); break;
+    }
+    mark(6, 0);
+  } else {
+    // x forward in place, then the inverse of each spectrum with its operator on the load
+    TileArgs F = x.A;
+    set_strides(F, F.sr, 0);
+    F.row_out = 0;
+    mark(2, 1);
+    COLA_TRY((launch_tile<-1, kCols, KOp::None>(gx, dim3(x.blocks), s, x.in, density, d_tw, F)));
+    mark(2, 0);
+    mark(3, 1);
+    COLA_TRY((launch_tile<1, kCols, KOp::PmPoisson>(gx, dim3(x.blocks), s, x.in, x.out[0], d_tw, x.A)));
+    mark(3, 0);
+    mark(3, 1);
+    COLA_TRY((launch_tile<1, kCols, KOp::PmCommon>(gx, dim3(x.blocks), s, x.in, x.out[1], d_tw, x.A)));
+    mark(3, 0);
   }
-  mark(6, 0);
-  for (int a = 0; a < 3; ++a) {
+  for (const TileJob& t : J.yinv) {
     mark(4, 1);
-    COLA_TRY(tile(Inv{}, std::integral_constant<int, kCols>{}, gy, J.yinv[a]));
+    COLA_TRY((launch_variant<YInv>(gy.emax, rs348, dim3(t.blocks), gy.threads, tile_lds_bytes(kCols, n, gy.log2T), s,
+                                   static_cast<const float2*>(t.in), static_cast<float2*>(t.out),
+                                   static_cast<float2*>(t.out2), t.tw, t.A)));
     mark(4, 0);
+  }
+  using Inv = std::integral_constant<int, 1>;
+  for (int a = 0; a < 3 && !records; ++a) {
     mark(5, 1);
-    COLA_TRY(tile(Inv{}, std::integral_constant<int, kC2R>{}, grows, J.zc2r[a]));
+    COLA_TRY(tile(Inv{}, std::integral_constant<int, kC2R>{}, grows, J.zslot[a]));
     mark(5, 0);
   }
+  if (!records) {
+    COLA_HIP(hipGetLastError());
+    return kOk;
+  }
+  mark(5, 1);
+  COLA_TRY((launch_variant<C2R3>(gz3.emax, rs348, dim3(J.zc2r.blocks), 3 * gz3.threads, c2r3_lds_bytes(n, gz3.log2T),
+                                 s, force, static_cast<const float2*>(d_tw), J.zc2r.A)));
+  mark(5, 0);
   COLA_HIP(hipGetLastError());
   return kOk;
 }
 
-int FftForcesBatch::init(const FftPlan* const* plans, float* const* density, float* const* out, const KOpParams* kp,
+int FftForcesBatch::init(const FftPlan* const* plans, float* const* density, float* const* force, const KOpParams* kp,
                          int n, bool merge_all)
 {
   destroy();
-  if (n <= 0 || !plans || !density || !out || !kp) return kErrArg;
+  if (n <= 0 || !plans || !density || !force || !kp) return kErrArg;
   std::vector<ForceJobs> fj(n);
   for (int i = 0; i < n; ++i) {
-    if (!plans[i] || !plans[i]->can_fuse()) {
+    if (!plans[i] || !plans[i]->can_fuse() || plans[i]->gz3.emax == 0) {
       set_error("batched force transforms need plans whose x pass fuses");
       return kErrUnsupported;
     }
-    make_force_jobs(*plans[i], density[i], out + 3 * i, kp[i], &fj[i]);
+    make_force_jobs(*plans[i], density[i], force[i], kp[i], &fj[i]);
   }
   // the jobs of the five passes and each job's own launch geometry
   struct Pass {
@@ -1274,12 +1635,12 @@ int FftForcesBatch::init(const FftPlan* const* plans, float* const* density, flo
     ps[1].g.push_back(&P.gy);
     ps[2].xj.push_back(fj[i].x);
     ps[2].g.push_back(&P.gx);
-    for (int a = 0; a < 3; ++a) {
-      ps[3].tj.push_back(fj[i].yinv[a]);
+    for (const TileJob& t : fj[i].yinv) {
+      ps[3].tj.push_back(t);
       ps[3].g.push_back(&P.gy);
-      ps[4].tj.push_back(fj[i].zc2r[a]);
-      ps[4].g.push_back(&P.grows);
     }
+    ps[4].tj.push_back(fj[i].zc2r);
+    ps[4].g.push_back(&P.gz3);
   }
   auto align_up = [](size_t v, size_t a) { return (v + a - 1) / a * a; };
   auto round_e = [](int e) { return e <= 8 ? 8 : e <= 12 ? 12 : e <= 16 ? 16 : 24; };
@@ -1307,7 +1668,7 @@ int FftForcesBatch::init(const FftPlan* const* plans, float* const* density, flo
       }
       emax = std::max(emax, e);
       all348 = all348 && radices_348(A.P);
-      st.lds = std::max(st.lds, tile_lds_bytes(p.mode, A.P.n, A.log2T));
+      st.lds = std::max(st.lds, k == 4 ? c2r3_lds_bytes(A.P.n, A.log2T) : tile_lds_bytes(p.mode, A.P.n, A.log2T));
     }
     st.emax = round_e(emax);
     if (fused && st.emax > 12) {
@@ -1322,7 +1683,7 @@ int FftForcesBatch::init(const FftPlan* const* plans, float* const* density, flo
       at = (at + al - 1) / al * al;
       start[j] = (int)at;
       at += blocks(j);
-      if (at > 0x7fffffffLL || at * st.threads > 0xffffffffLL) {
+      if (at > 0x7fffffffLL || at * st.threads * (k == 4 ? 3 : 1) > 0xffffffffLL) {
         set_error("batched force transforms: too many workgroups for one launch");
         return kErrUnsupported;
       }
@@ -1394,8 +1755,14 @@ int FftForcesBatch::run(hipStream_t s) const
           COLA_TRY((launch_fused_jobs_e<12, kRsAll>(st, s)));
         }
         break;
-      case 3: COLA_TRY((launch_jobs<1, kCols>(st, s))); break;
-      default: COLA_TRY((launch_jobs<1, kC2R>(st, s))); break;
+      case 3:
+        COLA_TRY((launch_variant<YInvJobs>(st.emax, st.rs == kRs348, dim3(st.blocks), st.threads, st.lds, s,
+                                           static_cast<const TileJob*>(st.jobs), st.start, st.njobs)));
+        break;
+      default:
+        COLA_TRY((launch_variant<C2R3Jobs>(st.emax, st.rs == kRs348, dim3(st.blocks), 3 * st.threads, st.lds, s,
+                                           static_cast<const TileJob*>(st.jobs), st.start, st.njobs)));
+        break;
     }
   }
   COLA_HIP(hipGetLastError());
@@ -1426,17 +1793,13 @@ int FftPlan::c2r(const float2* in_k, float* out, KOp op, const KOpParams& kp, hi
   const long long ncols = (long long)n * np_;
   A.log2T = gx.log2T;
   A.ncols = (int)ncols;
-  A.sr = ncols;
-  A.bs = 0;
+  set_strides(A, ncols, 0);
   A.kz_valid = np_ > nz ? (int)nz : 0;
   set_groups(A, grid_x(ncols, gx.log2T), xgroup);
   const float2* src = in_k ? in_k : cout;
   const dim3 grid(A.tpb_pad);
   mark(3, 1);
   switch (op) {
-    case KOp::PmPoisson:
-      COLA_TRY((launch_tile<1, kCols, KOp::PmPoisson>(gx, grid, s, src, cout, d_tw, A)));
-      break;
     case KOp::LptGrad:
       COLA_TRY((launch_tile<1, kCols, KOp::LptGrad>(gx, grid, s, src, cout, d_tw, A)));
       break;
@@ -1451,8 +1814,7 @@ int FftPlan::c2r(const float2* in_k, float* out, KOp op, const KOpParams& kp, hi
   // y
   A.log2T = gy.log2T;
   A.ncols = (int)nz;
-  A.sr = np_;
-  A.bs = (long long)n * np_;
+  set_strides(A, np_, (long long)n * np_);
   A.kz_valid = 0;
   set_groups(A, grid_x(nz, gy.log2T), xgroup);
   mark(4, 1);

@@ -107,16 +107,20 @@ int launch_grid_contrast(const PosSource& src, int n, float boxsize, const GridB
                          long long capacity, int* overflow, unsigned long long* fix, long long row, float nbar_inv,
                          float* grid, double* sums, hipStream_t s);
 
-// pm.c:359-412 + 505-532: readout of the three force grids into p.f.
-// fsum: null, or the three sums of a residual added to the force grids,
-// whose mean is taken off every particle's force.  fi: null (gather from
-// fx, fy, fz), or one interleaved grid fi[cell][3] of the same forces.
-int launch_readout(const DevParticles& p, const CicGeom& g, const float* fx, const float* fy, const float* fz,
-                   const double* fsum, const float* fi, hipStream_t s);
+// A force grid: per line (x ng + y) the records F[z][3], lines `line` floats
+// apart (6 nzp where the transforms left them, 3 ng in the net's grid).
+struct ForceLines {
+  const float* f = nullptr;
+  long long line = 0;
+};
+
+// pm.c:359-412 + 505-532: readout of the force grid into p.f.
+// fsum: null, or the three sums of a residual added to the force grid,
+// whose mean is taken off every particle's force.
+int launch_readout(const DevParticles& p, const CicGeom& g, const ForceLines& f, const double* fsum, hipStream_t s);
 // Readout fused with cola.c:104-112 kick and cola.c:142-149 drift.
-int launch_readout_kick_drift(const DevParticles& p, const CicGeom& g, const float* fx, const float* fy,
-                              const float* fz, const StepParams* prm, const double* fsum, const float* fi,
-                              hipStream_t s);
+int launch_readout_kick_drift(const DevParticles& p, const CicGeom& g, const ForceLines& f, const StepParams* prm,
+                              const double* fsum, hipStream_t s);
 int launch_kick(const DevParticles& p, const KickFactors& k, hipStream_t s);
 int launch_drift(const DevParticles& p, const DriftFactors& d, hipStream_t s);
 
@@ -139,7 +143,7 @@ struct PmMember {
   TileGeom t;
   BinBuffers b;
   float* density;
-  const float* f[3];       // force grids the readout gathers from
+  ForceLines f;            // what the readout gathers from
   double* ring;            // mass-check ring (ring[prm->slot] gets the grid sum)
   const StepParams* prm;   // this step's values of the realization
   float boxsize;

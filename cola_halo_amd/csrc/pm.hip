@@ -801,13 +801,17 @@ k_grid_scatter(PosSource src, GridGeom g, TileGeom t, int* __restrict__ counts, 
 // XCD, so the shared grid lines are read once into that XCD's L2 (256^3 on
 // 768^3: groups of 8 took the fused readout from 2.0 to 1.68 ms).
 
-// One axis of the CIC gather at one position, term order of pm.c:397-410.
 struct Gather3 {
   float f[3];
 };
 
-__device__ inline Gather3 cic_gather(float x, float y, float z, const CicGeom& g, const float* __restrict__ g0,
-                                     const float* __restrict__ g1, const float* __restrict__ g2)
+// The three components of the CIC gather at one position, term order of
+// pm.c:397-410, from lines of records fi[z][3] (`line` floats apart): a
+// corner's components are one 12-byte record, so a particle touches four grid
+// lines instead of the twelve of three separate grids: the fused readout,
+// bound by those gathers, takes 1.08 ms for 2.16 (256^3 on 768^3), 0.39 for
+// 0.74 (192^3 on 480^3).
+__device__ inline Gather3 cic_gather(float x, float y, float z, const CicGeom& g, const ForceLines& fl)
 {
   const int ng = g.ng;
   const float X = x * g.scale;
@@ -832,57 +836,7 @@ __device__ inline Gather3 cic_gather(float x, float y, float z, const CicGeom& g
   if (J1 >= ng) J1 = 0;
   int K1 = K + 1;
   if (K1 >= ng) K1 = 0;
-  const float* grids[3] = {g0, g1, g2};
-  const long long row = g.row;
-  if (0 <= iI && iI < ng) {
-    const long long a = ((long long)iI * ng + J) * row, b = ((long long)iI * ng + J1) * row;
-#pragma unroll
-    for (int ax = 0; ax < 3; ++ax) {
-      const float* m = grids[ax];
-      r.f[ax] += m[a + K] * T3 * T1 * T2 + m[a + K1] * D3 * T1 * T2 + m[b + K] * T3 * T1 * D2 + m[b + K1] * D3 * T1 * D2;
-    }
-  }
-  if (0 <= I1 && I1 < ng) {
-    const long long a = ((long long)I1 * ng + J) * row, b = ((long long)I1 * ng + J1) * row;
-#pragma unroll
-    for (int ax = 0; ax < 3; ++ax) {
-      const float* m = grids[ax];
-      r.f[ax] += m[a + K] * T3 * D1 * T2 + m[a + K1] * D3 * D1 * T2 + m[b + K] * T3 * D1 * D2 + m[b + K1] * D3 * D1 * D2;
-    }
-  }
-  return r;
-}
-
-// The same gather from one interleaved grid fi[cell][3] (cells unpadded,
-// C order): the three components of a corner are one 12-byte record, so a
-// particle touches four grid lines instead of twelve.  Same index, weight
-// and term order as cic_gather.
-__device__ inline Gather3 cic_gather_fi(float x, float y, float z, const CicGeom& g, const float* __restrict__ fi)
-{
-  const int ng = g.ng;
-  const float X = x * g.scale;
-  const float Y = y * g.scale;
-  const float Z = z * g.scale;
-  int iI = (int)floorf(X);
-  int J = (int)Y;
-  int K = (int)Z;
-  const float D1 = X - (float)iI;
-  const float D2 = Y - (float)J;
-  const float D3 = Z - (float)K;
-  const float T1 = 1.0f - D1;
-  const float T2 = 1.0f - D2;
-  const float T3 = 1.0f - D3;
-  Gather3 r;
-  r.f[0] = r.f[1] = r.f[2] = 0.0f;
-  if (J < 0 || K < 0) return r;
-  if (J >= ng) J = 0;
-  if (K >= ng) K = 0;
-  const int I1 = iI + 1;
-  int J1 = J + 1;
-  if (J1 >= ng) J1 = 0;
-  int K1 = K + 1;
-  if (K1 >= ng) K1 = 0;
-  auto rec = [&](long long line, int k) { return *reinterpret_cast<const float3*>(fi + (line * ng + k) * 3); };
+  auto rec = [&](long long line, int k) { return *reinterpret_cast<const float3*>(fl.f + line * fl.line + 3 * k); };
   if (0 <= iI && iI < ng) {
     const long long a = (long long)iI * ng + J, b = (long long)iI * ng + J1;
     const float3 aK = rec(a, K), aK1 = rec(a, K1), bK = rec(b, K), bK1 = rec(b, K1);
@@ -904,13 +858,11 @@ __device__ inline Gather3 cic_gather_fi(float x, float y, float z, const CicGeom
 
 // Force at a particle: its own gather plus, beyond the ghost threshold, the
 // gather at its ghost position added afterwards (pm.c:526-531).
-template <bool FI>
-__device__ inline Gather3 particle_force(float x, float y, float z, const CicGeom& g, const float* g0, const float* g1,
-                                         const float* g2)
+__device__ inline Gather3 particle_force(float x, float y, float z, const CicGeom& g, const ForceLines& fl)
 {
-  Gather3 f = FI ? cic_gather_fi(x, y, z, g, g0) : cic_gather(x, y, z, g, g0, g1, g2);
+  Gather3 f = cic_gather(x, y, z, g, fl);
   if (x > g.x_right) {
-    const Gather3 h = FI ? cic_gather_fi(x + g.shift, y, z, g, g0) : cic_gather(x + g.shift, y, z, g, g0, g1, g2);
+    const Gather3 h = cic_gather(x + g.shift, y, z, g, fl);
 #pragma unroll
     for (int a = 0; a < 3; ++a) f.f[a] += h.f[a];
   }
@@ -927,15 +879,12 @@ __device__ inline void residual_mean(const double* __restrict__ fsum, float inv_
   for (int a = 0; a < 3; ++a) m[a] = fsum ? (float)(fsum[a] * (double)inv_cells) : 0.0f;
 }
 
-// FI: g0 is the interleaved grid fi[cell][3] (g1, g2 unused).
-template <bool FI>
 __global__ void __launch_bounds__(kThreads)
-k_readout(DevParticles p, CicGeom g, const float* __restrict__ g0, const float* __restrict__ g1,
-          const float* __restrict__ g2, const double* __restrict__ fsum, float inv_cells)
+k_readout(DevParticles p, CicGeom g, ForceLines fl, const double* __restrict__ fsum, float inv_cells)
 {
   const long long i = (long long)xcd_group_remap(blockIdx.x, gridDim.x, g.readout_group) * kThreads + threadIdx.x;
   if (i >= p.np) return;
-  Gather3 f = particle_force<FI>(p.x[0][i], p.x[1][i], p.x[2][i], g, g0, g1, g2);
+  Gather3 f = particle_force(p.x[0][i], p.x[1][i], p.x[2][i], g, fl);
   float m[3];
   residual_mean(fsum, inv_cells, m);
 #pragma unroll
@@ -956,11 +905,8 @@ __device__ inline float drift1(float x, float v, float dx1, float dx2, const Dri
 }
 
 // Block blk of nblk (the member's own grid) of the fused readout.
-template <bool FI>
 __device__ __forceinline__ void readout_kick_drift_block(const DevParticles& p, const CicGeom& g,
-                                                         const float* __restrict__ g0, const float* __restrict__ g1,
-                                                         const float* __restrict__ g2,
-                                                         const StepParams* __restrict__ prm,
+                                                         const ForceLines& fl, const StepParams* __restrict__ prm,
                                                          const double* __restrict__ fsum, float inv_cells, int blk,
                                                          int nblk)
 {
@@ -971,7 +917,7 @@ __device__ __forceinline__ void readout_kick_drift_block(const DevParticles& p, 
   float x[3];
 #pragma unroll
   for (int a = 0; a < 3; ++a) x[a] = p.x[a][i];
-  Gather3 f = particle_force<FI>(x[0], x[1], x[2], g, g0, g1, g2);
+  Gather3 f = particle_force(x[0], x[1], x[2], g, fl);
   if (fsum) {
     float m[3];
     residual_mean(fsum, inv_cells, m);
@@ -987,13 +933,11 @@ __device__ __forceinline__ void readout_kick_drift_block(const DevParticles& p, 
   }
 }
 
-template <bool FI>
 __global__ void __launch_bounds__(kThreads)
-k_readout_kick_drift(DevParticles p, CicGeom g, const float* __restrict__ g0, const float* __restrict__ g1,
-                     const float* __restrict__ g2, const StepParams* __restrict__ prm, const double* __restrict__ fsum,
-                     float inv_cells)
+k_readout_kick_drift(DevParticles p, CicGeom g, ForceLines fl, const StepParams* __restrict__ prm,
+                     const double* __restrict__ fsum, float inv_cells)
 {
-  readout_kick_drift_block<FI>(p, g, g0, g1, g2, prm, fsum, inv_cells, blockIdx.x, gridDim.x);
+  readout_kick_drift_block(p, g, fl, prm, fsum, inv_cells, blockIdx.x, gridDim.x);
 }
 
 __global__ void __launch_bounds__(kThreads) k_kick(DevParticles p, KickFactors kf)
@@ -1130,7 +1074,7 @@ k_readout_kick_drift_batch(const PmMember* __restrict__ ms, const int* __restric
   const int nb = (int)((M.p.np + kThreads - 1) / kThreads);
   const int lb = (int)blockIdx.x - start[m];
   if (lb >= nb) return;  // alignment padding
-  readout_kick_drift_block<false>(M.p, M.g, M.f[0], M.f[1], M.f[2], M.prm, nullptr, 0.0f, lb, nb);
+  readout_kick_drift_block(M.p, M.g, M.f, M.prm, nullptr, 0.0f, lb, nb);
 }
 
 unsigned blocks_for(long long n) { return (unsigned)((n + kThreads - 1) / kThreads); }
@@ -1377,33 +1321,22 @@ int launch_grid_contrast(const PosSource& src, int n, float boxsize, const GridB
   return kOk;
 }
 
-int launch_readout(const DevParticles& p, const CicGeom& g, const float* fx, const float* fy, const float* fz,
-                   const double* fsum, const float* fi, hipStream_t s)
+int launch_readout(const DevParticles& p, const CicGeom& g, const ForceLines& f, const double* fsum, hipStream_t s)
 {
   if (p.np == 0) return kOk;
   const float inv_cells = (float)(1.0 / ((double)g.ng * g.ng * g.ng));
-  if (fi)
-    hipLaunchKernelGGL(k_readout<true>, dim3(blocks_for(p.np)), dim3(kThreads), 0, s, p, g, fi, fi, fi, fsum,
-                       inv_cells);
-  else
-    hipLaunchKernelGGL(k_readout<false>, dim3(blocks_for(p.np)), dim3(kThreads), 0, s, p, g, fx, fy, fz, fsum,
-                       inv_cells);
+  hipLaunchKernelGGL(k_readout, dim3(blocks_for(p.np)), dim3(kThreads), 0, s, p, g, f, fsum, inv_cells);
   COLA_HIP(hipGetLastError());
   return kOk;
 }
 
-int launch_readout_kick_drift(const DevParticles& p, const CicGeom& g, const float* fx, const float* fy,
-                              const float* fz, const StepParams* prm, const double* fsum, const float* fi,
-                              hipStream_t s)
+int launch_readout_kick_drift(const DevParticles& p, const CicGeom& g, const ForceLines& f, const StepParams* prm,
+                              const double* fsum, hipStream_t s)
 {
   if (p.np == 0) return kOk;
   const float inv_cells = (float)(1.0 / ((double)g.ng * g.ng * g.ng));
-  if (fi)
-    hipLaunchKernelGGL(k_readout_kick_drift<true>, dim3(blocks_for(p.np)), dim3(kThreads), 0, s, p, g, fi, fi, fi, prm,
-                       fsum, inv_cells);
-  else
-    hipLaunchKernelGGL(k_readout_kick_drift<false>, dim3(blocks_for(p.np)), dim3(kThreads), 0, s, p, g, fx, fy, fz,
-                       prm, fsum, inv_cells);
+  hipLaunchKernelGGL(k_readout_kick_drift, dim3(blocks_for(p.np)), dim3(kThreads), 0, s, p, g, f, prm, fsum,
+                     inv_cells);
   COLA_HIP(hipGetLastError());
   return kOk;
 }

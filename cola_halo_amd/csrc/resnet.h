@@ -10,6 +10,8 @@
 
 #include <vector>
 
+#include "pm.h"
+
 namespace cola {
 
 constexpr int kNetLayers = 4;
@@ -63,8 +65,8 @@ void resnet_free(ResNet* r);
 int resnet_pack(ResNet* r, hipStream_t s);
 // stores a training pair: features of the coarse density, target = fine force
 // at the coincident points (fine cell 2i) minus coarse force, and a
-int resnet_store_pair(ResNet* r, const float* coarse_delta, long long crow, const float* const coarse_f[3],
-                      const float* const fine_f[3], long long frow, float a, hipStream_t s);
+int resnet_store_pair(ResNet* r, const float* coarse_delta, long long crow, const ForceLines& coarse_f,
+                      const ForceLines& fine_f, float a, hipStream_t s);
 // mean loss over stored samples [first, first + count); train: epochs over
 // samples [0, ntrain) in shuffled order, one Adam step per sample
 int resnet_eval(ResNet* r, int first, int count, double* loss, hipStream_t s);
@@ -79,16 +81,15 @@ int resnet_forward(ResNet* r, hipStream_t s);
 int resnet_forward_features(ResNet* r, const unsigned short* feat, const float* pa, float a, hipStream_t s);
 // inference in parts around the PM force FFTs: the feature grid d_f1 from
 // the real-space density grid (rows of `row` floats) before the r2c, layers
-// 1-3 (a read from pa), and layer 4 added to the force grids:
-// out[a] = out[a] + out_scale * y[a]
+// 1-3 (a read from pa), and layer 4 added to the force components
 int resnet_features(ResNet* r, const float* delta, long long row, hipStream_t s);
 int resnet_body(ResNet* r, const float* pa, hipStream_t s);
 // resnet_body in its two launches groups: layer 1 (from d_f1), layers 2-3
 int resnet_layer1(ResNet* r, const float* pa, hipStream_t s);
 int resnet_layers23(ResNet* r, hipStream_t s);
-// out[a] + out_scale * y[a] into d_fi[cell][a] (the force grids keep the
-// plain force; d_fsum gets the sums of the residual added)
-int resnet_head_add(ResNet* r, float* const out[3], long long row, hipStream_t s);
+// force component a (f + a slot, lines `line` floats apart) + out_scale * y[a]
+// into d_fi[cell][a] (d_fsum gets the sums of the residual added)
+int resnet_head_add(ResNet* r, float* f, long long slot, long long line, hipStream_t s);
 // The inference path with the first two layers fused (fuse12): h2 straight
 // from the real-space density grid (features, layer 1 and layer 2 in one
 // launch, a read from pa), then layer 3; equal to resnet_features,
@@ -98,7 +99,7 @@ int resnet_layer3(ResNet* r, hipStream_t s);
 // Layer 3 and the last layer in one launch (from h2, after the force
 // transforms): the corrected force into d_fi as resnet_layer3 followed by
 // resnet_head_add, bit for bit, without writing h3.  By input planes only.
-int resnet_layer3_head(ResNet* r, float* const out[3], long long row, hipStream_t s);
+int resnet_layer3_head(ResNet* r, float* f, long long slot, long long line, hipStream_t s);
 // loss against target (bf16 [3][n^3] or fp32 [3][n^3]) and gradient into d_grad
 int resnet_backward(ResNet* r, const unsigned short* target_bf16, const float* target_f32, hipStream_t s);
 int resnet_adam(ResNet* r, float lr, hipStream_t s);

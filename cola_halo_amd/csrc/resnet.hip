@@ -71,8 +71,8 @@ enum ConvMode { kFwdRelu = 0, kFwdLinear = 1, kBwdData = 2, kFwdAdd = 3 };
 
 // Outputs of a convolution by mode: bf16 activations (kFwdRelu; kBwdData
 // masked by relu'(hprev)), the fp32 net output y [3][n^3] (kFwdLinear), or
-// scale * y added in place to three grids with rows of `row` floats
-// (kFwdAdd: the corrected PM force, out[a] = out[a] + out_scale * y[a]).
+// scale * y added to three force components add[a] with lines `row` floats
+// apart (kFwdAdd: the corrected PM force).
 struct ConvOut {
   unsigned short* bf = nullptr;
   float* f = nullptr;
@@ -255,7 +255,7 @@ k_conv16(const unsigned short* __restrict__ in, const unsigned short* __restrict
   const int wz = (threadIdx.x >> 6) & 1, wy = threadIdx.x >> 7;
   const int zc = 1 + 16 * wz + r;          // brick z of the lane's cell
   const int zs = lo ? zc - 1 : zc + 1;     // its z neighbour for the dz = -1 | +1 taps
-  float added[3] = {0.0f, 0.0f, 0.0f};     // kFwdAdd: sums of the residual this lane added
+  double added[3] = {0.0, 0.0, 0.0};       // kFwdAdd: sums of the residual this lane added
   const long long units = (long long)((n + march - 1) / march) * (n / kBlockY) * (n / kBlockZ);
   for (long long u = blockIdx.x; u < units; u += gridDim.x) {
     const ConvUnit cu = conv_unit(u, n, march);
@@ -310,7 +310,7 @@ k_conv16(const unsigned short* __restrict__ in, const unsigned short* __restrict
                 o.fi[(line * n + cu.z0 + 16 * wz + r) * 3 + i] = fold[t][i] + dv;
               else
                 o.add[i][at] = fold[t][i] + dv;
-              added[i] += dv;
+              added[i] += (double)dv;
             }
           }
         } else {
@@ -327,10 +327,10 @@ k_conv16(const unsigned short* __restrict__ in, const unsigned short* __restrict
   if (MODE == kFwdAdd && o.sum && g == 0) {
 #pragma unroll
     for (int i = 0; i < 3; ++i) {
-      float a = added[i];
+      double a = added[i];
 #pragma unroll
       for (int off = 8; off > 0; off >>= 1) a += __shfl_xor(a, off);
-      if (r == 0) atomicAdd(o.sum + i, (double)a);
+      if (r == 0) atomicAdd(o.sum + i, a);
     }
   }
 }
@@ -705,7 +705,10 @@ k_conv_head_r(const unsigned short* __restrict__ in, const unsigned short* __res
                                       : o.f + (g < 3 ? g : 0) * nc;
   constexpr int L = kRollLoads;
   constexpr int F = MODE == kFwdAdd ? kConvTy : 0, S = kConvTy;
-  float added = 0.0f;  // kFwdAdd: this lane's sum of the residual it added (component g)
+  // kFwdAdd: this lane's sum of the residual it added (component g), in
+  // doubles: the kernels group the cells differently, and sums of floats
+  // differed by enough to round the mean apart once in a few states
+  double added = 0.0;
   const long long units = (long long)((n + march - 1) / march) * (n / kBlockY) * (n / kBlockZ);
   for (long long u = blockIdx.x; u < units; u += gridDim.x) {
     const ConvUnit cu = conv_unit(u, n, march);
@@ -748,7 +751,7 @@ k_conv_head_r(const unsigned short* __restrict__ in, const unsigned short* __res
                 o.fi[(line * n + zcell) * 3 + g] = fold[t] + dv;  // lanes g = 0-2 of a cell: 12 contiguous bytes
               else
                 gout[line * o.row + zcell] = fold[t] + dv;
-              added += dv;
+              added += (double)dv;
             } else {
               gout[line * n + zcell] = v;
             }
@@ -776,7 +779,7 @@ k_conv_head_r(const unsigned short* __restrict__ in, const unsigned short* __res
   if (MODE == kFwdAdd && o.sum) {
 #pragma unroll
     for (int off = 8; off > 0; off >>= 1) added += __shfl_xor(added, off);  // within the 16-lane group
-    if (r == 0 && g < 3) atomicAdd(o.sum + g, (double)added);
+    if (r == 0 && g < 3) atomicAdd(o.sum + g, added);
   }
 }
 
@@ -931,7 +934,7 @@ k_conv3h(const unsigned short* __restrict__ in, const unsigned short* __restrict
   float* const gout = g == 0 ? o.add[0] : (g == 1 ? o.add[1] : o.add[2]);
   constexpr int F = kConvTy, S = kConvTy;
   static_assert(2 * kRoll3Loads + 3 * S + 2 * F < 64, "the wait's count fits the counter");
-  float added = 0.0f;
+  double added = 0.0;
   for (long long u = blockIdx.x; u < units; u += gridDim.x) {
     const int z0 = (int)(u % nzb) * kOut3Z;
     const long long t2 = u / nzb;
@@ -981,7 +984,7 @@ k_conv3h(const unsigned short* __restrict__ in, const unsigned short* __restrict
           const float dv = o.scale * v;
           float* dst2 = put ? o.fi + (line * n + zcell) * 3 + g : o.trash + lane;
           *dst2 = fold[t] + dv;
-          if (put) added += dv;
+          if (put) added += (double)dv;
         }
       }
 #pragma unroll
@@ -1016,7 +1019,7 @@ k_conv3h(const unsigned short* __restrict__ in, const unsigned short* __restrict
   if (o.sum) {
 #pragma unroll
     for (int off = 8; off > 0; off >>= 1) added += __shfl_xor(added, off);  // within the 16-lane group
-    if (r == 0 && g < 3) atomicAdd(o.sum + g, (double)added);
+    if (r == 0 && g < 3) atomicAdd(o.sum + g, added);
   }
 }
 
@@ -1774,17 +1777,19 @@ __global__ void k_adam(float* __restrict__ p, float* __restrict__ m, float* __re
 // fine neighbours of the coincident fine cell (2x, 2y, 2z) with weights
 // (ws, 1 - 2 ws, ws) per axis, periodic (ws = 0: the point value, 1/4: full
 // weighting).
-__device__ inline float restrict_fine(const float* __restrict__ f, long long frow, int nf, int x, int y, int z, float ws)
+// Component a (of records f[z][3] per line) of the restricted fine force.
+__device__ inline float restrict_fine(const ForceLines& ff, int comp, int nf, int x, int y, int z, float ws)
 {
-  if (ws == 0.0f) return f[((long long)(2 * x) * nf + 2 * y) * frow + 2 * z];
+  const float* __restrict__ f = ff.f + comp;
+  if (ws == 0.0f) return f[((long long)(2 * x) * nf + 2 * y) * ff.line + 3 * (2 * z)];
   const float w[3] = {ws, 1.0f - 2.0f * ws, ws};
   float s = 0.0f;
   for (int a = 0; a < 3; ++a) {
     const int fx = wrapi(2 * x + a - 1, nf);
     for (int b = 0; b < 3; ++b) {
-      const long long row = ((long long)fx * nf + wrapi(2 * y + b - 1, nf)) * frow;
+      const long long row = ((long long)fx * nf + wrapi(2 * y + b - 1, nf)) * ff.line;
       const float wab = w[a] * w[b];
-      for (int c = 0; c < 3; ++c) s += wab * w[c] * f[row + wrapi(2 * z + c - 1, nf)];
+      for (int c = 0; c < 3; ++c) s += wab * w[c] * f[row + 3 * wrapi(2 * z + c - 1, nf)];
     }
   }
   return s;
@@ -1792,9 +1797,7 @@ __device__ inline float restrict_fine(const float* __restrict__ f, long long fro
 
 // Training pair: feature asinh(delta) * scale (bf16) and target = restricted
 // fine force minus the coarse force (bf16).
-__global__ void k_store_pair(const float* __restrict__ cd, long long crow, const float* __restrict__ c0,
-                             const float* __restrict__ c1, const float* __restrict__ c2, const float* __restrict__ f0,
-                             const float* __restrict__ f1, const float* __restrict__ f2, long long frow, int n,
+__global__ void k_store_pair(const float* __restrict__ cd, long long crow, ForceLines cf, ForceLines ff, int n,
                              float scale, float ws, unsigned short* __restrict__ feat, unsigned short* __restrict__ target)
 {
   const long long cell = (long long)blockIdx.x * kThreads + threadIdx.x;
@@ -1803,11 +1806,9 @@ __global__ void k_store_pair(const float* __restrict__ cd, long long crow, const
   const int z = (int)(cell % n);
   const long long xy = cell / n;
   const int y = (int)(xy % n), x = (int)(xy / n);
-  const long long ca = xy * crow + z;
-  feat[cell] = feature_of(cd[ca], scale);
-  target[cell] = f2bf(restrict_fine(f0, frow, 2 * n, x, y, z, ws) - c0[ca]);
-  target[nc + cell] = f2bf(restrict_fine(f1, frow, 2 * n, x, y, z, ws) - c1[ca]);
-  target[2 * nc + cell] = f2bf(restrict_fine(f2, frow, 2 * n, x, y, z, ws) - c2[ca]);
+  feat[cell] = feature_of(cd[xy * crow + z], scale);
+  const float* __restrict__ c = cf.f + xy * cf.line + 3 * z;
+  for (int a = 0; a < 3; ++a) target[a * nc + cell] = f2bf(restrict_fine(ff, a, 2 * n, x, y, z, ws) - c[a]);
 }
 
 __global__ void __launch_bounds__(kThreads) k_sumsq(const unsigned short* __restrict__ t, long long n, double* out)
@@ -2192,11 +2193,11 @@ int resnet_layer3(ResNet* r, hipStream_t s)
   return kOk;
 }
 
-int resnet_head_add(ResNet* r, float* const out[3], long long row, hipStream_t s)
+int resnet_head_add(ResNet* r, float* f, long long slot, long long line, hipStream_t s)
 {
   ConvOut o;
-  for (int a = 0; a < 3; ++a) o.add[a] = out[a];
-  o.row = row;
+  for (int a = 0; a < 3; ++a) o.add[a] = f + a * slot;
+  o.row = line;
   o.scale = r->out_scale;
   hipLaunchKernelGGL(k_zero3, dim3(1), dim3(64), 0, s, r->d_fsum);
   o.sum = r->d_fsum;
@@ -2204,12 +2205,12 @@ int resnet_head_add(ResNet* r, float* const out[3], long long row, hipStream_t s
   return conv_layer_4(r, kFwdAdd, o, s);
 }
 
-int resnet_layer3_head(ResNet* r, float* const out[3], long long row, hipStream_t s)
+int resnet_layer3_head(ResNet* r, float* f, long long slot, long long line, hipStream_t s)
 {
   COLA_TRY(conv_lds_attributes());
   ConvOut o;
-  for (int a = 0; a < 3; ++a) o.add[a] = out[a];
-  o.row = row;
+  for (int a = 0; a < 3; ++a) o.add[a] = f + a * slot;
+  o.row = line;
   o.scale = r->out_scale;
   hipLaunchKernelGGL(k_zero3, dim3(1), dim3(64), 0, s, r->d_fsum);
   o.sum = r->d_fsum;
@@ -2275,8 +2276,8 @@ int resnet_adam(ResNet* r, float lr, hipStream_t s)
   return resnet_pack(r, s);
 }
 
-int resnet_store_pair(ResNet* r, const float* coarse_delta, long long crow, const float* const cf[3],
-                      const float* const ff[3], long long frow, float a, hipStream_t s)
+int resnet_store_pair(ResNet* r, const float* coarse_delta, long long crow, const ForceLines& cf,
+                      const ForceLines& ff, float a, hipStream_t s)
 {
   const long long nc = (long long)r->n * r->n * r->n;
   unsigned short *feat = nullptr, *target = nullptr;
@@ -2288,8 +2289,8 @@ int resnet_store_pair(ResNet* r, const float* coarse_delta, long long crow, cons
   r->s_feat.push_back(feat);
   r->s_target.push_back(target);
   r->s_a.push_back(a);
-  hipLaunchKernelGGL(k_store_pair, dim3(grid_cells(nc)), dim3(kThreads), 0, s, coarse_delta, crow, cf[0], cf[1], cf[2],
-                     ff[0], ff[1], ff[2], frow, r->n, r->in_scale, r->restrict_side, feat, target);
+  hipLaunchKernelGGL(k_store_pair, dim3(grid_cells(nc)), dim3(kThreads), 0, s, coarse_delta, crow, cf, ff,
+                     r->n, r->in_scale, r->restrict_side, feat, target);
   COLA_HIP(hipGetLastError());
   return kOk;
 }

@@ -217,6 +217,30 @@ def test_force_matches_oracle(eh_table, nc, ng, box):
     assert np.abs(f_gpu - ref["force"]).max() <= 1e-5 * scale
 
 
+@pytest.mark.parametrize("nc,ng", [(4, 4), (4, 8), (8, 6), (6, 10), (8, 18), (12, 20), (12, 30), (20, 50), (32, 54),
+                                   (36, 90), (40, 100), (48, 128), (48, 162)])
+def test_force_of_every_kind_of_plan(eh_table, nc, ng):
+    """Plans whose x pass does not fuse (4, 8: one radix pass), rows of n % 4
+    = 2 (stored 8 bytes a lane), column tiles with an idle part, one, two and
+    four row pairs per workgroup: force grids and particle forces of the
+    oracle to the force's bound, twice on one context (grids reused)."""
+    _say(f"force of plan nc={nc} ng={ng}")
+    box = 50.0
+    parts = _random_particles(nc, box, 11 * nc + ng)
+    wpar = float(np.float32((ng / nc) ** 3))
+    with _context(nc, ng, box, eh_table) as ctx:
+        first = _gpu_forces(ctx, parts)
+        f_gpu = _gpu_forces(ctx, parts)
+        grids = [ctx.get_force_grid(a)[:, :, :ng] for a in range(3)]
+    assert np.array_equal(first, f_gpu)
+    ref = orc.pm_forces(ng, box, wpar, parts, want_grids=True)
+    assert ref["status"] == 0
+    for a in range(3):
+        rg = ref["force_grid"][a][:, :, :ng]
+        assert np.abs(grids[a] - rg).max() <= 1e-5 * np.abs(rg).max(), a
+    assert np.abs(f_gpu - ref["force"]).max() <= 1e-5 * np.abs(ref["force"]).max()
+
+
 def test_plane_wave_force_closed_form(eh_table):
     """A density cos(2 pi n.x/L) sampled on the grid nodes gives the force
     grid (L/2pi) n_a/|n|^2 sin(2 pi n.x/L) (pm.c:322-353 solves del^2 phi =
