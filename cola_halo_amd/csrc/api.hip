@@ -342,6 +342,14 @@ KOpParams pm_kop(const cola_context* c)
   return kp;
 }
 
+// Whether the transforms of the context leave records F[z][3] for the
+// readout (not for the net's last layer, which reads the components apart).
+// On long rows the z c2r of three components loses more than the readout
+// gains: at 1536^3 27.0 ms for 17.4, the readout of 512^3 particles 7.9 for
+// 11.3; at 768^3 3.45 for 3.03, of 256^3 particles 1.08 for 2.16.
+constexpr int kRecordsMaxGrid = 1024;
+bool writes_records(const cola_context* c) { return !c->net && c->ng <= kRecordsMaxGrid; }
+
 int pm_fields(cola_context* c)
 {
   const KOpParams kp = pm_kop(c);
@@ -372,7 +380,7 @@ int pm_fields(cola_context* c)
   c->density_is_real = false;
   // the readout gathers records; the net's last layer reads the components
   // apart and writes the corrected records
-  COLA_TRY(c->pm_fft.forces(c->density, c->fgrid, kp, c->net == nullptr, c->stream));
+  COLA_TRY(c->pm_fft.forces(c->density, c->fgrid, kp, writes_records(c), c->stream));
   if (fused34) {
     phase_begin(c, kPhNetConv34);
     COLA_TRY(resnet_layer3_head(c->net, c->fgrid, c->cic.row, 3 * c->cic.row, c->stream));
@@ -383,7 +391,7 @@ int pm_fields(cola_context* c)
     phase_end(c, kPhNetHead);
   }
   c->fi_force = c->net != nullptr;
-  c->force_records = c->net == nullptr;
+  c->force_records = writes_records(c);
   return kOk;
 }
 
@@ -397,7 +405,12 @@ const double* net_sums(const cola_context* c) { return c->net ? c->net->d_fsum :
 ForceLines force_lines(const cola_context* c)
 {
   if (c->net) return ForceLines{c->net->d_fi, 3LL * c->ng};
-  return ForceLines{c->fgrid, 3 * c->cic.row};
+  return ForceLines{c->fgrid, 3 * c->cic.row, writes_records(c) ? 0 : c->cic.row};
+}
+// The plain force of the last transforms, as they left it.
+ForceLines plain_lines(const cola_context* c)
+{
+  return ForceLines{c->fgrid, 3 * c->cic.row, c->force_records ? 0 : c->cic.row};
 }
 
 int require_particles(cola_context* c)
@@ -946,6 +959,8 @@ int cola_step(cola_context* c, float omega_m, float avel1, float apos1)
   else
     COLA_TRY(step_kernels(c));
   c->density_is_real = false;
+  c->fi_force = c->net != nullptr;  // a replayed step too
+  c->force_records = writes_records(c);
   c->a_v = avel1;
   c->a_x = apos1;
   c->have_force = false;
@@ -1047,7 +1062,7 @@ int ensemble_build(cola_ensemble* e)
     M.t = c->tiles;
     M.b = c->bins;
     M.density = c->density;
-    M.f = force_lines(c);
+    M.f = ForceLines{c->fgrid, 3 * c->cic.row};  // the batch writes records whatever the grid
     M.ring = c->d_mass;
     M.prm = e->d_prm + m;
     M.boxsize = c->boxf;
@@ -1183,6 +1198,7 @@ int cola_ensemble_step(cola_ensemble* e, float omega_m, const float* avel1, cons
     c->a_x = apos1[m];
     c->have_force = false;
     c->fi_force = false;
+    c->force_records = true;
   }
   if (++e->since_check >= cola_ensemble::kSlots / 2) {
     e->since_check = 0;
@@ -1399,7 +1415,7 @@ int cola_get_force_grid(cola_context* c, int axis, float* out, size_t n_out)
   }
   // records F[z][3] per line, of the transforms or of the net's corrected
   // grid: copied a few lines at a time, one component picked on the host
-  const ForceLines fl = fi ? ForceLines{c->net->d_fi, 3LL * c->ng} : ForceLines{c->fgrid, 3 * c->cic.row};
+  const ForceLines fl = fi ? ForceLines{c->net->d_fi, 3LL * c->ng} : plain_lines(c);
   const long long lines = (long long)c->ng * c->ng, hrow = 2 * (c->ng / 2 + 1);
   const long long chunk = std::max(1LL, std::min(lines, (1LL << 24) / (3LL * c->ng)));
   std::vector<float> rec((size_t)(3LL * c->ng * chunk));
@@ -2275,8 +2291,8 @@ int cola_resnet_add_pair(cola_resnet* h, cola_context* coarse, cola_context* fin
   if (!st) st = check_pending(coarse);
   if (!st) st = check_pending(fine);
   if (!st) {
-    st = resnet_store_pair(&h->r, dcopy, coarse->cic.row, ForceLines{coarse->fgrid, 3 * coarse->cic.row},
-                           ForceLines{fine->fgrid, 3 * fine->cic.row}, coarse->a_x, h->stream);
+    st = resnet_store_pair(&h->r, dcopy, coarse->cic.row, plain_lines(coarse), plain_lines(fine), coarse->a_x,
+                           h->stream);
   }
   if (!st && hipStreamSynchronize(h->stream) != hipSuccess) st = kErrHip;
   if (dcopy) (void)hipFree(dcopy);

@@ -249,6 +249,14 @@ constexpr int tile_waves_per_eu(int mode, KOp op, int emax, int rs)
   return 6;
 }
 
+// The fused x pass with radices 3, 4, 8 takes 73 VGPRs: 6 waves per SIMD, but
+// of 1024-thread workgroups only one fits a CU then.  WIDE: 64 registers (some
+// spill) and two of them: 768^3 (8 columns) 2.78 -> 2.27 ms.  Narrower
+// workgroups already share a CU and keep their registers (384^3 0.235 against
+// 0.258 ms; 768^3 with 4 columns 2.52 against 2.71).
+constexpr int fused_waves_per_eu(bool wide) { return wide ? 8 : 1; }
+constexpr int kFusedWideThreads = 768;  // above: WIDE
+
 // What a column pass of wave numbers multiplies by: the position's wave
 // number on the load, or the column's on the store (both 0: nothing).
 enum YScale : int { kYPlain = 0, kYByPosition = 1, kYByColumn = 2 };
@@ -383,7 +391,8 @@ __device__ __forceinline__ void tile_run(const void* in_, void* out_, const floa
           const int j = b - i * p.L;
 #pragma unroll
           for (int s = 1; s < R; ++s) {
-            reg[q * R + s] = twiddle<DIR>(reg[q * R + s], tws[s * j * p.twstep]);
+            const int at = MODE == kCols ? s * __mul24(j, p.twstep) : s * j * p.twstep;
+            reg[q * R + s] = twiddle<DIR>(reg[q * R + s], tws[at]);
           }
         }
         dft<R, DIR>(&reg[q * R]);
@@ -403,10 +412,16 @@ __device__ __forceinline__ void tile_run(const void* in_, void* out_, const floa
         int c, b;
         split(u, p, c, b);
         const int i = (int)fdiv((unsigned)b, (unsigned)p.L, p.magL);
-        const int j = b - i * p.L;
-        const int o = i * R * p.L + j;
+        if constexpr (MODE == kCols) {
+          const int Ls = p.L << log2T;  // as col_store_lds
+          float2* const o = lds + u + __mul24(i, (R - 1) * Ls);
 #pragma unroll
-        for (int t = 0; t < R; ++t) lds[lidx(o + t * p.L, c)] = reg[q * R + t];
+          for (int t = 0; t < R; ++t) o[t * Ls] = reg[q * R + t];
+        } else {
+          const int o = i * R * p.L + (b - i * p.L);
+#pragma unroll
+          for (int t = 0; t < R; ++t) lds[lidx(o + t * p.L, c)] = reg[q * R + t];
+        }
       }
     }
   };
@@ -422,7 +437,7 @@ __device__ __forceinline__ void tile_run(const void* in_, void* out_, const floa
         int c, b;
         split(u, p, c, b);
 #pragma unroll
-        for (int s = 0; s < R; ++s) reg[q * R + s] = lds[lidx(b + s * p.m, c)];
+        for (int s = 0; s < R; ++s) reg[q * R + s] = MODE == kCols ? lds[u + s * nb] : lds[lidx(b + s * p.m, c)];
       }
     }
   };
@@ -603,14 +618,14 @@ __device__ __forceinline__ void c2r3_run(float* data, const float2* __restrict__
         if (u < nb) {
           const int c = (int)fdiv((unsigned)u, (unsigned)p.m, p.magM), b = u - c * p.m;
           const int i = (int)fdiv((unsigned)b, (unsigned)p.L, p.magL);
-          const int j = b - i * p.L;
           if (p.L > 1) {
+            const int j = b - i * p.L;
 #pragma unroll
             for (int s = 1; s < R; ++s) reg[q * R + s] = twiddle<1>(reg[q * R + s], smem[s * j * p.twstep]);
           }
           dft<R, 1>(&reg[q * R]);
           if (!last) {
-            const int o = i * R * p.L + j;
+            const int o = i * R * p.L + (b - i * p.L);
 #pragma unroll
             for (int t = 0; t < R; ++t) lds[c * (n + 1) + o + t * p.L] = reg[q * R + t];
           } else {
@@ -660,6 +675,14 @@ struct ColCtx {
   int tid, nthr, log2T;
 };
 
+// Butterfly u = (b << log2T) + c of a column pass: its LDS inputs lie at u +
+// s (m << log2T), its outputs at u + i ((R - 1) L << log2T) + t (L << log2T)
+// with i = b div L, j = b mod L (o = i R L + j = b + i (R - 1) L), its
+// twiddles at multiples of j twstep: one add per access.  (Rebuilding each
+// index from (o + t L, c), with a 32-bit multiply per twiddle, was most of the
+// fused pass's VALU work, which bounds it: with f1 / k^2 folded into the kept
+// spectrum as well, 270^3 0.163 -> 0.129 ms, 384^3 0.327 -> 0.235, 480^3 0.90
+// -> 0.56, 768^3 2.98 -> 2.78.)
 template <int R, int EMAX, int DIR>
 __device__ inline void col_compute(float2 (&reg)[EMAX], const FftPass& p, const ColCtx& x)
 {
@@ -668,14 +691,12 @@ __device__ inline void col_compute(float2 (&reg)[EMAX], const FftPass& p, const 
   for (int q = 0; q < EMAX / R; ++q) {
     const int u = x.tid + q * x.nthr;
     if (u < nb) {
-      const int b = u >> x.log2T;
       if (p.L > 1) {
+        const int b = u >> x.log2T;
         const int i = (int)fdiv((unsigned)b, (unsigned)p.L, p.magL);
-        const int j = b - i * p.L;
+        const int jt = __mul24(b - __mul24(i, p.L), p.twstep);
 #pragma unroll
-        for (int s = 1; s < R; ++s) {
-          reg[q * R + s] = twiddle<DIR>(reg[q * R + s], x.tws[s * j * p.twstep]);
-        }
+        for (int s = 1; s < R; ++s) reg[q * R + s] = twiddle<DIR>(reg[q * R + s], x.tws[s * jt]);
       }
       dft<R, DIR>(&reg[q * R]);
     }
@@ -685,17 +706,15 @@ __device__ inline void col_compute(float2 (&reg)[EMAX], const FftPass& p, const 
 template <int R, int EMAX>
 __device__ inline void col_store_lds(const float2 (&reg)[EMAX], const FftPass& p, const ColCtx& x)
 {
-  const int nb = p.m << x.log2T;
+  const int nb = p.m << x.log2T, Ls = p.L << x.log2T;
 #pragma unroll
   for (int q = 0; q < EMAX / R; ++q) {
     const int u = x.tid + q * x.nthr;
     if (u < nb) {
-      const int c = u & ((1 << x.log2T) - 1), b = u >> x.log2T;
-      const int i = (int)fdiv((unsigned)b, (unsigned)p.L, p.magL);
-      const int j = b - i * p.L;
-      const int o = i * R * p.L + j;
+      const int i = (int)fdiv((unsigned)(u >> x.log2T), (unsigned)p.L, p.magL);
+      float2* const o = x.lds + u + __mul24(i, (R - 1) * Ls);
 #pragma unroll
-      for (int t = 0; t < R; ++t) x.lds[((o + t * p.L) << x.log2T) + c] = reg[q * R + t];
+      for (int t = 0; t < R; ++t) o[t * Ls] = reg[q * R + t];
     }
   }
 }
@@ -708,13 +727,12 @@ __device__ inline void col_load_lds(float2 (&reg)[EMAX], const FftPass& p, const
   for (int q = 0; q < EMAX / R; ++q) {
     const int u = x.tid + q * x.nthr;
     if (u < nb) {
-      const int c = u & ((1 << x.log2T) - 1), b = u >> x.log2T;
+      const float2* const in = x.lds + u;
 #pragma unroll
-      for (int s = 0; s < R; ++s) reg[q * R + s] = x.lds[((b + s * p.m) << x.log2T) + c];
+      for (int s = 0; s < R; ++s) reg[q * R + s] = in[s * nb];
     }
   }
 }
-
 
 // ---- y inverse of the force spectra ------------------------------------------
 // The x pass leaves two spectra: F_x and the common one G = i f1 / k^2 delta
@@ -885,9 +903,8 @@ __device__ __forceinline__ void fused_run(const float2* __restrict__ in, float2*
   __syncthreads();
   col_compute<R_LAST, EMAX, -1>(keep, pl, x);
 
-  // f1 / k^2 of each kept value (pm.c:339 evaluates (f1 / k^2) * d_axis
-  // left to right, so the quotient is shared by the three axes bit for bit)
-  float green[EMAX];
+  // the common spectrum i f1 / k^2 delta in place of the kept values; n_x
+  // times it is F_x's
 #pragma unroll
   for (int q = 0; q < EMAX / R_LAST; ++q) {
     const int u = tid + q * nthr;
@@ -899,7 +916,9 @@ __device__ __forceinline__ void fused_run(const float2* __restrict__ in, float2*
     for (int t = 0; t < R_LAST; ++t) {
       const int I0 = wave_pm(b + t * pl.m, n);
       const int k2 = K * K + I0 * I0 + J0 * J0;
-      green[q * R_LAST + t] = k2 == 0 ? 0.0f : A.kp.f1 / (float)k2;
+      const float g = k2 == 0 ? 0.0f : A.kp.f1 / (float)k2;
+      const float2 v = keep[q * R_LAST + t];
+      keep[q * R_LAST + t] = k2 == 0 ? make_float2(0.0f, 0.0f) : make_float2(-g * v.y, g * v.x);
     }
   }
 
@@ -910,21 +929,15 @@ __device__ __forceinline__ void fused_run(const float2* __restrict__ in, float2*
 #pragma unroll 1
   for (int axis = 0; axis < 2; ++axis) {
     Tile reg;
-    // inverse pass 0 (L = 1): pm.c:322-346 operator on the forward outputs b + t*m
+    // inverse pass 0 (L = 1) on the forward outputs b + t*m
 #pragma unroll
     for (int q = 0; q < EMAX / R_LAST; ++q) {
-      const int u = tid + q * nthr;
-      const int c = u & tmask, b = u >> log2T;
-      const int col = c0 + c;
-      const int iy = (int)fdiv((unsigned)col, (unsigned)A.nz, A.magNz);
-      const int J0 = wave_pm(iy, n), K = col - iy * A.nz;
+      const int b = (tid + q * nthr) >> log2T;
 #pragma unroll
       for (int t = 0; t < R_LAST; ++t) {
-        const int I0 = wave_pm(b + t * pl.m, n);
-        const float f2 = axis == 0 ? green[q * R_LAST + t] * (float)I0 : green[q * R_LAST + t];
+        const float w = axis == 0 ? (float)wave_pm(b + t * pl.m, n) : 1.0f;
         const float2 v = keep[q * R_LAST + t];
-        reg[q * R_LAST + t] = (I0 == 0 && J0 == 0 && K == 0) ? make_float2(0.0f, 0.0f)
-                                                              : make_float2(-f2 * v.y, f2 * v.x);
+        reg[q * R_LAST + t] = make_float2(w * v.x, w * v.y);
       }
     }
     col_compute<R_LAST, EMAX, 1>(reg, Pinv.pass[0], x);
@@ -963,8 +976,8 @@ __device__ __forceinline__ void fused_run(const float2* __restrict__ in, float2*
   }
 }
 
-template <int R_LAST, int EMAX, int RS>
-__global__ void __launch_bounds__(kFftMaxThreads)
+template <int R_LAST, int EMAX, int RS, bool WIDE>
+__global__ void __launch_bounds__(kFftMaxThreads) __attribute__((amdgpu_waves_per_eu(fused_waves_per_eu(WIDE))))
 fft_x_fused(const float2* __restrict__ in, float2* __restrict__ out0, float2* __restrict__ out1,
             const float2* __restrict__ tw, TileArgs A, FftRadices Pinv)
 {
@@ -1091,8 +1104,8 @@ fft_c2r3_jobs(const TileJob* __restrict__ jobs, const int* __restrict__ start, i
   c2r3_run<EMAX, RS>(static_cast<float*>(J.out), J.tw, J.A, (int)blockIdx.x - start[j]);
 }
 
-template <int EMAX, int RS>
-__global__ void __launch_bounds__(kFftMaxThreads)
+template <int EMAX, int RS, bool WIDE>
+__global__ void __launch_bounds__(kFftMaxThreads) __attribute__((amdgpu_waves_per_eu(fused_waves_per_eu(WIDE))))
 fft_x_fused_jobs(const FusedJob* __restrict__ jobs, const int* __restrict__ start, int njobs)
 {
   const int j = batch_find(start, njobs, blockIdx.x);
@@ -1348,17 +1361,17 @@ static FftRadices reversed(const FftRadices& r)
   return v;
 }
 
-template <int RL, int E, int RS>
+template <int RL, int E, int RS, bool WIDE = false>
 static int launch_fused_e(const FftPassGeom& g, int grid, hipStream_t s, const float2* in, float2* o0, float2* o1,
                           const float2* tw, const TileArgs& A, const FftRadices& Pinv)
 {
   static bool attr = false;
   if (!attr) {
-    COLA_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&fft_x_fused<RL, E, RS>),
+    COLA_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&fft_x_fused<RL, E, RS, WIDE>),
                                  hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
     attr = true;
   }
-  hipLaunchKernelGGL((fft_x_fused<RL, E, RS>), dim3(grid), dim3(g.threads), tile_lds_bytes(kCols, A.P.n, g.log2T), s,
+  hipLaunchKernelGGL((fft_x_fused<RL, E, RS, WIDE>), dim3(grid), dim3(g.threads), tile_lds_bytes(kCols, A.P.n, g.log2T), s,
                      in, o0, o1, tw, A, Pinv);
   return kOk;
 }
@@ -1369,7 +1382,10 @@ static int launch_fused_r(const FftPassGeom& g, int grid, hipStream_t s, const f
 {
   if (g.emax <= 8) {
     if constexpr (RL == 3 || RL == 4 || RL == 8)
-      if (radices_348(A.P)) return launch_fused_e<RL, 8, kRs348>(g, grid, s, in, o0, o1, tw, A, Pinv);
+      if (radices_348(A.P)) {
+        if (g.threads > kFusedWideThreads) return launch_fused_e<RL, 8, kRs348, true>(g, grid, s, in, o0, o1, tw, A, Pinv);
+        return launch_fused_e<RL, 8, kRs348>(g, grid, s, in, o0, o1, tw, A, Pinv);
+      }
     return launch_fused_e<RL, 8, kRsAll>(g, grid, s, in, o0, o1, tw, A, Pinv);
   }
   return launch_fused_e<RL, 12, kRsAll>(g, grid, s, in, o0, o1, tw, A, Pinv);
@@ -1517,16 +1533,16 @@ int launch_jobs(const FftBatchStage& st, hipStream_t s)
   return launch_jobs_e<DIR, MODE, 24, kRsAll>(st, s);
 }
 
-template <int E, int RS>
+template <int E, int RS, bool WIDE = false>
 int launch_fused_jobs_e(const FftBatchStage& st, hipStream_t s)
 {
   static bool attr = false;
   if (!attr) {
-    COLA_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&fft_x_fused_jobs<E, RS>),
+    COLA_HIP(hipFuncSetAttribute(reinterpret_cast<const void*>(&fft_x_fused_jobs<E, RS, WIDE>),
                                  hipFuncAttributeMaxDynamicSharedMemorySize, 160 * 1024));
     attr = true;
   }
-  hipLaunchKernelGGL((fft_x_fused_jobs<E, RS>), dim3(st.blocks), dim3(st.threads), st.lds, s,
+  hipLaunchKernelGGL((fft_x_fused_jobs<E, RS, WIDE>), dim3(st.blocks), dim3(st.threads), st.lds, s,
                      static_cast<const FusedJob*>(st.jobs), st.start, st.njobs);
   return kOk;
 }
@@ -1747,7 +1763,9 @@ int FftForcesBatch::run(hipStream_t s) const
       case 0: COLA_TRY((launch_jobs<-1, kR2C>(st, s))); break;
       case 1: COLA_TRY((launch_jobs<-1, kCols>(st, s))); break;
       case 2:
-        if (st.emax <= 8 && st.rs == kRs348) {
+        if (st.emax <= 8 && st.rs == kRs348 && st.threads > kFusedWideThreads) {
+          COLA_TRY((launch_fused_jobs_e<8, kRs348, true>(st, s)));
+        } else if (st.emax <= 8 && st.rs == kRs348) {
           COLA_TRY((launch_fused_jobs_e<8, kRs348>(st, s)));
         } else if (st.emax <= 8) {
           COLA_TRY((launch_fused_jobs_e<8, kRsAll>(st, s)));

@@ -108,10 +108,12 @@ int launch_grid_contrast(const PosSource& src, int n, float boxsize, const GridB
                          float* grid, double* sums, hipStream_t s);
 
 // A force grid: per line (x ng + y) the records F[z][3], lines `line` floats
-// apart (6 nzp where the transforms left them, 3 ng in the net's grid).
+// apart (6 nzp where the transforms left them, 3 ng in the net's grid), or,
+// slot > 0, the components' rows `slot` floats apart.
 struct ForceLines {
   const float* f = nullptr;
   long long line = 0;
+  long long slot = 0;
 };
 
 // pm.c:359-412 + 505-532: readout of the force grid into p.f.

@@ -1780,8 +1780,9 @@ __global__ void k_adam(float* __restrict__ p, float* __restrict__ m, float* __re
 // Component a (of records f[z][3] per line) of the restricted fine force.
 __device__ inline float restrict_fine(const ForceLines& ff, int comp, int nf, int x, int y, int z, float ws)
 {
-  const float* __restrict__ f = ff.f + comp;
-  if (ws == 0.0f) return f[((long long)(2 * x) * nf + 2 * y) * ff.line + 3 * (2 * z)];
+  const float* __restrict__ f = ff.f + comp * (ff.slot ? ff.slot : 1);
+  const int zs = ff.slot ? 1 : 3;
+  if (ws == 0.0f) return f[((long long)(2 * x) * nf + 2 * y) * ff.line + zs * (2 * z)];
   const float w[3] = {ws, 1.0f - 2.0f * ws, ws};
   float s = 0.0f;
   for (int a = 0; a < 3; ++a) {
@@ -1789,7 +1790,7 @@ __device__ inline float restrict_fine(const ForceLines& ff, int comp, int nf, in
     for (int b = 0; b < 3; ++b) {
       const long long row = ((long long)fx * nf + wrapi(2 * y + b - 1, nf)) * ff.line;
       const float wab = w[a] * w[b];
-      for (int c = 0; c < 3; ++c) s += wab * w[c] * f[row + 3 * wrapi(2 * z + c - 1, nf)];
+      for (int c = 0; c < 3; ++c) s += wab * w[c] * f[row + zs * wrapi(2 * z + c - 1, nf)];
     }
   }
   return s;
@@ -1807,8 +1808,9 @@ __global__ void k_store_pair(const float* __restrict__ cd, long long crow, Force
   const long long xy = cell / n;
   const int y = (int)(xy % n), x = (int)(xy / n);
   feat[cell] = feature_of(cd[xy * crow + z], scale);
-  const float* __restrict__ c = cf.f + xy * cf.line + 3 * z;
-  for (int a = 0; a < 3; ++a) target[a * nc + cell] = f2bf(restrict_fine(ff, a, 2 * n, x, y, z, ws) - c[a]);
+  const float* __restrict__ c = cf.f + xy * cf.line + (cf.slot ? 1 : 3) * z;
+  const long long slot = cf.slot ? cf.slot : 1;
+  for (int a = 0; a < 3; ++a) target[a * nc + cell] = f2bf(restrict_fine(ff, a, 2 * n, x, y, z, ws) - c[a * slot]);
 }
 
 __global__ void __launch_bounds__(kThreads) k_sumsq(const unsigned short* __restrict__ t, long long n, double* out)
