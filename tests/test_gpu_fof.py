@@ -71,6 +71,27 @@ def test_fof_matches_oracle(eh_table, nc, box, ll, nmin):
         _compare(ctx, snap, box, ll, nmin)
 
 
+@pytest.mark.parametrize("nc,box,ll", [(4, 64.0, 0.05), (8, 64.0, 0.5), (4, 3.0, 1.4), (6, 3.0, 1.0), (6, 3.0, 0.9)])
+def test_fof_columns_sparse_and_few(nc, box, ll):
+    """Columns of linking cells mostly empty (64 particles over 1267^2
+    columns), their entries in the first and the last one, and grids of 1, 2
+    and 3 cells per axis, where a column is the whole search: labels and
+    halos of the oracle."""
+    _say(f"fof columns nc={nc} box={box} ll={ll}")
+    rng = np.random.default_rng(nc)
+    snap = np.zeros(nc ** 3, ch.PARTICLE_MIN_DTYPE)
+    snap["x"] = rng.uniform(0, box, (nc ** 3, 3)).astype(np.float32)
+    pairs = nc ** 3 // 4
+    snap["x"][:pairs] = ((snap["x"][pairs:2 * pairs] + np.float32(0.3 * ll)) % box).astype(np.float32)
+    last = np.nextafter(np.float32(box), np.float32(0))
+    snap["x"][-4:] = [(0, 0, 0), (last, last, last), (0, last, 0), (last, 0, last)]
+    snap["v"] = rng.normal(0, 100.0, (nc ** 3, 3)).astype(np.float32)
+    snap["id"] = np.arange(1, nc ** 3 + 1)
+    with ch.Context(nc, nc, box) as ctx:
+        ctx.set_snapshot_records(snap)
+        _compare(ctx, snap, box, ll, 2)
+
+
 def test_fof_evolved_128(eh_table):
     """128^3 particles evolved to z = 0 (L = 250, 384^3 PM grid, 10 steps),
     linking length 0.2 of the mean separation (main.c:353)."""
