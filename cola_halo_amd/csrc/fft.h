@@ -53,6 +53,24 @@ struct KOpParams {
   double box = 0.0;   // lpt.c kvec = n * 2 * pi / Box
 };
 
+// Element offset of position b and column c of a column pass whose positions
+// lie `stride` apart (a whole plane in the x pass).  b runs to n / R - 1 of the
+// pass's radix R: with a small first or last radix the offset passes 2^32 on
+// grids that fit the card (2250 = 2 3^2 5^3: 1124 x 3 planes of 2250 x 1136 =
+// 8.6e9), so it is formed in 64 bits.
+__host__ __device__ inline unsigned long long col_offset(int b, long long stride, int c)
+{
+  return (unsigned long long)(unsigned)b * (unsigned)stride + (unsigned)c;
+}
+
+// Whether every such offset of a pass of m = n / R positions fits 32 bits.  The
+// fused x pass forms them so (in 64 bits it loses a wavefront per SIMD: 480^3
+// 0.56 -> 0.89 ms, 768^3 2.28 -> 2.49); other grids run its passes apart.
+inline bool col_offsets_fit32(int m, long long stride, int log2T)
+{
+  return col_offset(m - 1, stride, (1 << log2T) - 1) <= 0xffffffffULL;
+}
+
 // Launch shape of one axis pass: 2^log2T transforms per workgroup, threads
 // per workgroup, register slots per thread.
 struct FftPassGeom {

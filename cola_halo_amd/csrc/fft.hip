@@ -314,9 +314,9 @@ __device__ __forceinline__ void tile_run(const void* in_, void* out_, const floa
       split(u, p, c, b);
       const bool live = u < nb && c0 + c < A.ncols;
       if (MODE == kCols) {
-        // uniform base per leg s (scalar registers) + 32-bit lane offset b*sr + c
+        // uniform base per leg s (scalar registers) + lane offset b*sr + c
         const float2* in = static_cast<const float2*>(in_) + (long long)batch * A.bs + c0;
-        const unsigned lane = (unsigned)b * (unsigned)A.sr + (unsigned)c;
+        const unsigned long long lane = col_offset(b, A.sr, c);
         int iy = 0, iz = 0;
         if constexpr (OP != KOp::None) {
           const int col = c0 + c;
@@ -456,7 +456,7 @@ __device__ __forceinline__ void tile_run(const void* in_, void* out_, const floa
         if (MODE == kCols) {
           float2* out = static_cast<float2*>(out_) + (long long)batch * A.bs_out + c0;
           if (ROW_OUT) out += (long long)fdiv((unsigned)(c0 + c), (unsigned)A.nz, A.magNz) * (A.row_out - A.nz);
-          const unsigned lane = (unsigned)b * (unsigned)A.sr_out + (unsigned)c;
+          const unsigned long long lane = col_offset(b, A.sr_out, c);
           if (YS && yscale == kYByColumn) {
             const float w = (float)(c0 + c);
 #pragma unroll
@@ -876,7 +876,7 @@ __device__ __forceinline__ void fused_run(const float2* __restrict__ in, float2*
       const int c = u & tmask, b = u >> log2T;
       const bool live = u < nb && c0 + c < A.ncols;
       const float2* base = in + c0;
-      const unsigned lane = (unsigned)b * (unsigned)A.sr + (unsigned)c;
+      const unsigned lane = (unsigned)b * (unsigned)A.sr + (unsigned)c;  // (col_offsets_fit32)
 #pragma unroll
       for (int s = 0; s < R; ++s)
         reg[q * R + s] = live ? base[(long long)(s * p.m) * A.sr + lane] : make_float2(0.0f, 0.0f);
@@ -1394,6 +1394,8 @@ static int launch_fused_r(const FftPassGeom& g, int grid, hipStream_t s, const f
 bool FftPlan::can_fuse() const
 {
   if (rad.npass < 2 || gx.emax > 12) return false;
+  // its loads and stores: plane strides of the density and of a line of three
+  if (!col_offsets_fit32(rad.pass[0].m, 3LL * n * nzp, gx.log2T)) return false;
   const int RL = rad.pass[rad.npass - 1].R;
   return RL == 3 || RL == 4 || RL == 5 || RL == 8;
 }
