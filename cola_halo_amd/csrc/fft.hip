@@ -1236,6 +1236,35 @@ static int cap_log2(int n)
   return l;
 }
 
+// The z c2r of three components, as three groups of threads and their tiles
+// in LDS allow: the row pairs asked for (2^l a workgroup) or the next fewer
+// that fit; else one pair (768^3 3.45 ms against 3.66 of two; 384^3 0.40, 0.45;
+// 270^3 0.160, 0.180) unless that leaves over half of its threads idle, then
+// the fewest with the least idle (192^3: two 0.049 against one 0.062; 480^3:
+// four 0.83 against 0.96 of two and 1.11 of one).
+static FftPassGeom rows3_geom(const FftRadices& rad, int l, bool asked)
+{
+  auto fit = [&](int k) {
+    return c2r3_lds_bytes(rad.n, k) <= 160 * 1024 ? pass_geom(rad, k, kFftC2r3Threads) : FftPassGeom{};
+  };
+  if (asked) {
+    FftPassGeom g = fit(l);
+    while (!g.emax && l > 0) g = fit(--l);
+    return g;
+  }
+  FftPassGeom best;
+  double most = 0.0;
+  for (int k = 0; k <= 2 && !(k == 1 && most >= 0.5); ++k) {
+    const FftPassGeom g = fit(k);
+    const double busy = g.emax ? (double)((long long)rad.n << k) / (8.0 * g.threads) : 0.0;
+    if (busy > most) {
+      most = busy;
+      best = g;
+    }
+  }
+  return best;
+}
+
 int FftPlan::init(int n_, int log2T_cols, int log2T_rows, bool pad_rows, int log2T_xcols, int schedule_)
 {
   n = n_;
@@ -1261,28 +1290,7 @@ int FftPlan::init(int n_, int log2T_cols, int log2T_rows, bool pad_rows, int log
   gy = pick(log2T_cols >= 0 ? log2T_cols : std::min(3, cap_log2(n)), n / 2 + 1);
   grows = pick(log2T_rows >= 0 ? log2T_rows : 1, (long long)n * n / 2);
   if (gx.emax == 0 || gy.emax == 0 || grows.emax == 0) return kErrUnsupported;
-  // the z c2r of three components: the row pairs asked for, or one pair (768^3
-  // 3.45 ms against 3.66 of two; 384^3 0.40, 0.45; 270^3 0.160, 0.180) unless
-  // that leaves over half of its threads idle, then the fewest with the least
-  // idle (192^3: two 0.049 against one 0.062; 480^3: four 0.83 against 0.96 of
-  // two and 1.11 of one), as three groups of threads and their tiles allow
-  double best = 0.0;
-  for (int l = log2T_rows >= 0 ? grows.log2T : 0; l >= 0 && l <= 2;) {
-    const FftPassGeom g =
-        c2r3_lds_bytes(n, l) <= 160 * 1024 ? pass_geom(rad, l, kFftC2r3Threads) : FftPassGeom{};
-    const double busy = g.emax ? (double)((long long)n << l) / (8.0 * g.threads) : 0.0;
-    if (busy > best) {
-      best = busy;
-      gz3 = g;
-    }
-    if (log2T_rows >= 0) {
-      if (gz3.emax) break;
-      --l;
-    } else {
-      if (l == 0 && best >= 0.5) break;
-      ++l;
-    }
-  }
+  gz3 = rows3_geom(rad, grows.log2T, log2T_rows >= 0);
   std::vector<float2> tw(n);
   for (int k = 0; k < n; ++k) {
     const double a = -2.0 * kPiD * (double)k / (double)n;

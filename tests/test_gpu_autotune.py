@@ -80,3 +80,39 @@ def test_fft_launch_shapes_agree_bit_for_bit(eh_table, cols, rows, group, xcols)
             (a, snap), = ch.run_cola(ctx, OM, 1.0, 10, 5, [0.0])
             out.append(snap)
     assert np.array_equal(out[0], out[1])
+
+
+@pytest.mark.parametrize("nc,ng,rows", [(24, 72, 3), (32, 96, 3), (32, 96, 4), (32, 96, 6), (40, 100, 5), (64, 192, 4)])
+def test_wide_row_tiles_agree_bit_for_bit(eh_table, nc, ng, rows):
+    """Row widths of 3 and more (8 to 64 row pairs per workgroup, by either
+    setter), whether or not three components of them fit a workgroup: steps
+    and ensemble steps equal those of the default widths bit for bit."""
+    print(f"row tiles 2^{rows} ng={ng}", flush=True)
+    k, p = eh_table
+
+    def make(shape):
+        c = ch.Context(nc, ng, 100.0)
+        c.power_init_table(k, p, 0.1, 0.8, OM, 1.0 - OM)
+        if shape == "tiles":
+            c.set_fft_tiles(2, rows, 8, 2)
+        elif shape == "tiling":
+            c.set_tiling(2, 2, 4, 3)
+        c.lpt_set_displacement(0.1, OM, 5)
+        c.set_times(c.times()[0], 0.1)
+        return c
+
+    ctxs = [make(s) for s in (None, "tiles", "tiling", "tiles", "tiling")]
+    try:
+        with ch.Ensemble(ctxs[3:]) as ens:
+            for avel1, apos1 in ((0.25, 0.3), (0.45, 0.5)):
+                for c in ctxs[:3]:
+                    c.step(float(np.float32(OM)), avel1, apos1)
+                ens.step(float(np.float32(OM)), avel1, apos1)
+        want = ctxs[0].get_particles()
+        grid = ctxs[0].get_force_grid(1)
+        for c in ctxs[1:]:
+            assert np.array_equal(c.get_particles(), want)
+            assert np.array_equal(c.get_force_grid(1), grid)
+    finally:
+        for c in ctxs:
+            c.close()
