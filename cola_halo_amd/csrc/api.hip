@@ -1521,10 +1521,7 @@ int set_deposit_tiles(cola_context* c, int tx, int ty, int tz)
   COLA_HIP(hipStreamSynchronize(c->stream));
   drop_step_graph(c);
   COLA_TRY(check_pending(c));
-  BinBuffers nb;
-  COLA_TRY(bin_alloc(&nb, t, c->np));
-  bin_free(&c->bins);
-  c->bins = nb;
+  COLA_TRY(bin_retile(&c->bins, t));
   c->tiles = t;
   named();
   return kOk;
@@ -1907,8 +1904,9 @@ int cola_coarse_grid_noalloc(cola_context* c, int n, int source, float* delta_de
   COLA_TRY(noalloc_scratch(&fix));
   double* sums = sums_dev ? sums_dev : reinterpret_cast<double*>(fix + kNoAllocCells);
   // the same kernels as cola_coarse_grid; the accumulators and sums are
-  // cleared by fill kernels on the context's stream, the tile counters are
-  // the context's (made with it, for grids of up to kNoAllocGrid)
+  // cleared by fill kernels on the context's stream, the tile counters (made
+  // with the context, for grids of up to kNoAllocGrid) and the sort's entries
+  // keep their place until the context is destroyed
   return deposit_contrast(c, src, n, n, fix, delta_dev, sums);
 }
 

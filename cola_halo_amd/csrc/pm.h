@@ -60,6 +60,9 @@ struct BinBuffers {
 };
 
 int bin_alloc(BinBuffers* b, const TileGeom& t, long long np);
+// The buffers of other tiles; the entries and the flag, which depend on the
+// particle count alone, stay where they are (the output grids sort there too).
+int bin_retile(BinBuffers* b, const TileGeom& t);
 void bin_free(BinBuffers* b);
 
 // move.c:33-41
@@ -89,9 +92,11 @@ int launch_deposit_tiles(const CicGeom& g, const TileGeom& t, const BinBuffers& 
                          const StepParams* prm, hipStream_t s);
 int launch_zero_mass(double* ring, const StepParams* prm, hipStream_t s);
 // Output grids (coarse_grid.c:95-121): counters and offsets of their tiles.
+// Set 0 is the first one made and keeps its place until grid_bin_free, so work
+// enqueued or captured on it stays valid; set 1 grows with larger grids.
 struct GridBins {
-  int* counts = nullptr;  // tiles (zero between calls), then tiles + 1 offsets, then the scan's sums
-  long long tiles = 0;
+  int* counts[2] = {nullptr, nullptr};  // tiles (zero between calls), then tiles + 1 offsets, then the scan's sums
+  long long tiles[2] = {0, 0};
 };
 TileGeom grid_tile_geom(int n);
 int grid_bin_alloc(GridBins* b, int n);  // at least the tiles of an n^3 grid (keeps what is large enough)

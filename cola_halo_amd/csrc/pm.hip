@@ -1156,30 +1156,56 @@ bool default_tile_geom(int ng, int want[3], TileGeom* t)
   return true;
 }
 
+static void bin_free_tiles(BinBuffers* b)
+{
+  if (b->counts) (void)hipFree(b->counts);
+  if (b->offsets) (void)hipFree(b->offsets);
+  if (b->block_sums) (void)hipFree(b->block_sums);
+  if (b->tile_sums) (void)hipFree(b->tile_sums);
+  b->counts = b->offsets = b->block_sums = nullptr;
+  b->tile_sums = nullptr;
+}
+
 int bin_alloc(BinBuffers* b, const TileGeom& t, long long np)
 {
   bin_free(b);
-  const long long nsums = (t.ntiles + kScanChunk - 1) / kScanChunk;
   b->capacity = 8 * np + 1024;
-  COLA_HIP(hipMalloc(&b->counts, sizeof(int) * t.ntiles));
-  COLA_HIP(hipMalloc(&b->offsets, sizeof(int) * (t.ntiles + 1)));
-  COLA_HIP(hipMalloc(&b->block_sums, sizeof(int) * (nsums + 1)));
   COLA_HIP(hipMalloc(&b->sorted, sizeof(float) * 3 * b->capacity));
   COLA_HIP(hipMalloc(&b->overflow, sizeof(int)));
-  COLA_HIP(hipMalloc(&b->tile_sums, sizeof(double) * t.ntiles));
-  COLA_HIP(hipMemset(b->counts, 0, sizeof(int) * t.ntiles));
   COLA_HIP(hipMemset(b->overflow, 0, sizeof(int)));
+  return bin_retile(b, t);
+}
+
+int bin_retile(BinBuffers* b, const TileGeom& t)
+{
+  const long long nsums = (t.ntiles + kScanChunk - 1) / kScanChunk;
+  BinBuffers nb;
+  auto make = [&]() -> int {
+    COLA_HIP(hipMalloc(&nb.counts, sizeof(int) * t.ntiles));
+    COLA_HIP(hipMalloc(&nb.offsets, sizeof(int) * (t.ntiles + 1)));
+    COLA_HIP(hipMalloc(&nb.block_sums, sizeof(int) * (nsums + 1)));
+    COLA_HIP(hipMalloc(&nb.tile_sums, sizeof(double) * t.ntiles));
+    COLA_HIP(hipMemset(nb.counts, 0, sizeof(int) * t.ntiles));
+    return kOk;
+  };
+  const int st = make();
+  if (st) {
+    bin_free_tiles(&nb);
+    return st;
+  }
+  bin_free_tiles(b);
+  b->counts = nb.counts;
+  b->offsets = nb.offsets;
+  b->block_sums = nb.block_sums;
+  b->tile_sums = nb.tile_sums;
   return kOk;
 }
 
 void bin_free(BinBuffers* b)
 {
-  if (b->counts) (void)hipFree(b->counts);
-  if (b->offsets) (void)hipFree(b->offsets);
-  if (b->block_sums) (void)hipFree(b->block_sums);
+  bin_free_tiles(b);
   if (b->sorted) (void)hipFree(b->sorted);
   if (b->overflow) (void)hipFree(b->overflow);
-  if (b->tile_sums) (void)hipFree(b->tile_sums);
   *b = BinBuffers{};
 }
 
@@ -1251,23 +1277,27 @@ int grid_bin_alloc(GridBins* b, int n)
     set_error("unable to allocate the output grid");
     return kErrAlloc;
   }
-  if (b->tiles >= t.ntiles) return kOk;
-  grid_bin_free(b);
+  const int k = b->counts[0] ? 1 : 0;
+  if (std::max(b->tiles[0], b->tiles[1]) >= t.ntiles) return kOk;
+  if (b->counts[k]) (void)hipFree(b->counts[k]);
+  b->counts[k] = nullptr;
+  b->tiles[k] = 0;
   const long long nsums = (t.ntiles + kScanChunk - 1) / kScanChunk;
-  if (hipMalloc(&b->counts, sizeof(int) * (2 * t.ntiles + nsums + 2)) != hipSuccess) {
+  if (hipMalloc(&b->counts[k], sizeof(int) * (2 * t.ntiles + nsums + 2)) != hipSuccess) {
     (void)hipGetLastError();
-    b->counts = nullptr;
+    b->counts[k] = nullptr;
     set_error("unable to allocate the output grid");
     return kErrAlloc;
   }
-  COLA_HIP(hipMemset(b->counts, 0, sizeof(int) * t.ntiles));
-  b->tiles = t.ntiles;
+  COLA_HIP(hipMemset(b->counts[k], 0, sizeof(int) * t.ntiles));
+  b->tiles[k] = t.ntiles;
   return kOk;
 }
 
 void grid_bin_free(GridBins* b)
 {
-  if (b->counts) (void)hipFree(b->counts);
+  for (int* p : b->counts)
+    if (p) (void)hipFree(p);
   *b = GridBins{};
 }
 
@@ -1293,14 +1323,15 @@ int launch_grid_contrast(const PosSource& src, int n, float boxsize, const GridB
   g.n = n;
   g.dx_inv = n / boxsize;
   const TileGeom t = grid_tile_geom(n);
-  if (n < 1 || t.ntiles > b.tiles || (src.stride != 1 && src.stride != 8)) {
+  const int k = t.ntiles <= b.tiles[0] ? 0 : 1;
+  if (n < 1 || t.ntiles > b.tiles[k] || (src.stride != 1 && src.stride != 8)) {
     set_error("coarse grid: invalid grid size");
     return kErrArg;
   }
   BinBuffers bb;
-  bb.counts = b.counts;
-  bb.offsets = b.counts + b.tiles;
-  bb.block_sums = bb.offsets + b.tiles + 1;
+  bb.counts = b.counts[k];
+  bb.offsets = b.counts[k] + b.tiles[k];
+  bb.block_sums = bb.offsets + b.tiles[k] + 1;
   const int nsplit = grid_split(n, src.np);
   const unsigned nb = bin_blocks(src.np);
   auto bin = [&](auto stride) {

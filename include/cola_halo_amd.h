@@ -253,7 +253,12 @@ int cola_coarse_grid(cola_context* ctx, int n, int source, float* delta_out, dou
    forbid hipMalloc): cola_coarse_grid's kernels in the context's own buffers,
    with the fixed-point sums of cells that several workgroups add to in a
    static device array of the library (16 MiB per GPU, held until the
-   process ends), so the call allocates nothing.  n <= 128 (COLA_ERR_ARG
+   process ends), so the call allocates nothing.  The context's buffers are
+   its density bins (their entries, and counters made with the context): they
+   keep their addresses until cola_context_destroy, whatever grids and tiles
+   are asked for in between, and each step and output grid of the context
+   overwrites them, so replays of captured work are ordered with the
+   context's other calls.  n <= 128 (COLA_ERR_ARG
    beyond).  delta_dev is DEVICE memory for n^3 floats (C order, as
    cola_coarse_grid's delta_out); sums_dev is NULL or DEVICE memory for the
    two sums.  Work is only enqueued on the context's stream: the call does
