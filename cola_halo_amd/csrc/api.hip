@@ -92,7 +92,7 @@ struct cola_context {
   DevParticles p;
   float* pbuf = nullptr;
   float* density = nullptr;
-  float* fgrid = nullptr;  // force lines (ForceLines): 3 cic.row floats per line
+  float* fgrid[3] = {nullptr, nullptr, nullptr};  // force components or their records (ForceLines)
   long long grid_floats = 0;
 
   FftPlan pm_fft, lpt_fft;
@@ -276,10 +276,10 @@ int alloc_grids(cola_context* c)
   if (c->have_grids) return kOk;
   const size_t bytes = sizeof(float) * c->grid_floats;
   COLA_HIP(hipMalloc(&c->density, bytes));
-  COLA_HIP(hipMalloc(&c->fgrid, 3 * bytes));
+  for (int a = 0; a < 3; ++a) COLA_HIP(hipMalloc(&c->fgrid[a], bytes));
   // the row padding is never written by the deposit; keep it finite
   COLA_HIP(hipMemset(c->density, 0, bytes));
-  COLA_HIP(hipMemset(c->fgrid, 0, 3 * bytes));
+  for (int a = 0; a < 3; ++a) COLA_HIP(hipMemset(c->fgrid[a], 0, bytes));
   c->have_grids = true;
   return kOk;
 }
@@ -383,11 +383,11 @@ int pm_fields(cola_context* c)
   COLA_TRY(c->pm_fft.forces(c->density, c->fgrid, kp, writes_records(c), c->stream));
   if (fused34) {
     phase_begin(c, kPhNetConv34);
-    COLA_TRY(resnet_layer3_head(c->net, c->fgrid, c->cic.row, 3 * c->cic.row, c->stream));
+    COLA_TRY(resnet_layer3_head(c->net, c->fgrid, c->cic.row, c->stream));
     phase_end(c, kPhNetConv34);
   } else if (c->net) {
     phase_begin(c, kPhNetHead);
-    COLA_TRY(resnet_head_add(c->net, c->fgrid, c->cic.row, 3 * c->cic.row, c->stream));
+    COLA_TRY(resnet_head_add(c->net, c->fgrid, c->cic.row, c->stream));
     phase_end(c, kPhNetHead);
   }
   c->fi_force = c->net != nullptr;
@@ -400,18 +400,18 @@ bool valid(const cola_context* c) { return c != nullptr; }
 // The learned residual's sums over the grid of the last force (its mean is
 // taken off the particles' forces), or null without a net.
 const double* net_sums(const cola_context* c) { return c->net ? c->net->d_fsum : nullptr; }
-// What the readout gathers from: the transforms' force lines, or with a net
-// its corrected force grid [cell][3].
-ForceLines force_lines(const cola_context* c)
+// The force the transforms leave, as records or as components apart.
+ForceLines grid_lines(const cola_context* c, bool records)
 {
-  if (c->net) return ForceLines{c->net->d_fi, 3LL * c->ng};
-  return ForceLines{c->fgrid, 3 * c->cic.row, writes_records(c) ? 0 : c->cic.row};
+  const float* const f = c->fgrid[0];
+  return ForceLines{f, {0, c->fgrid[1] - f, c->fgrid[2] - f}, c->cic.row, records ? c->pm_fft.rec_row : 0};
 }
+// A net's corrected force grid [cell][3].
+ForceLines net_lines(const cola_context* c) { return ForceLines{c->net->d_fi, {0, 0, 0}, 3LL * c->ng, c->ng}; }
+// What the readout gathers from.
+ForceLines force_lines(const cola_context* c) { return c->net ? net_lines(c) : grid_lines(c, writes_records(c)); }
 // The plain force of the last transforms, as they left it.
-ForceLines plain_lines(const cola_context* c)
-{
-  return ForceLines{c->fgrid, 3 * c->cic.row, c->force_records ? 0 : c->cic.row};
-}
+ForceLines plain_lines(const cola_context* c) { return grid_lines(c, c->force_records); }
 
 int require_particles(cola_context* c)
 {
@@ -544,7 +544,8 @@ int cola_context_destroy(cola_context* c)
   bin_free(&c->bins);
   if (c->pbuf) (void)hipFree(c->pbuf);
   if (c->density) (void)hipFree(c->density);
-  if (c->fgrid) (void)hipFree(c->fgrid);
+  for (float* g : c->fgrid)
+    if (g) (void)hipFree(g);
   if (c->d_mass) (void)hipFree(c->d_mass);
   if (c->step_graph) (void)hipGraphExecDestroy(c->step_graph);
   if (c->h_prm) (void)hipHostFree(c->h_prm);
@@ -1042,7 +1043,7 @@ int ensemble_build(cola_ensemble* e)
   const int n = (int)e->ctx.size();
   std::vector<PmMember> ms(n);
   std::vector<const FftPlan*> plans(n);
-  std::vector<float*> dens(n), outs(n);
+  std::vector<float*> dens(n), outs(3 * n);
   std::vector<KOpParams> kps(n);
   for (int m = 0; m < n; ++m) {
     cola_context* c = e->ctx[m];
@@ -1062,13 +1063,13 @@ int ensemble_build(cola_ensemble* e)
     M.t = c->tiles;
     M.b = c->bins;
     M.density = c->density;
-    M.f = ForceLines{c->fgrid, 3 * c->cic.row};  // the batch writes records whatever the grid
+    M.f = grid_lines(c, true);  // the batch writes records whatever the grid
     M.ring = c->d_mass;
     M.prm = e->d_prm + m;
     M.boxsize = c->boxf;
     plans[m] = &c->pm_fft;
     dens[m] = c->density;
-    outs[m] = c->fgrid;
+    for (int a = 0; a < 3; ++a) outs[3 * m + a] = c->fgrid[a];
     kps[m] = pm_kop(c);
     e->gen[m] = c->config_gen;
   }
@@ -1406,23 +1407,18 @@ int cola_get_force_grid(cola_context* c, int axis, float* out, size_t n_out)
   if (!c->have_grids) return kErrState;
   COLA_HIP(hipStreamSynchronize(c->stream));
   const bool fi = c->fi_force && c->net;
-  if (!fi && !c->force_records) {  // the components apart, one row each per line
-    const long long lines = (long long)c->ng * c->ng, hrow = 2 * (c->ng / 2 + 1);
-    COLA_HIP(hipMemcpy2D(out, sizeof(float) * hrow, c->fgrid + axis * c->cic.row, sizeof(float) * 3 * c->cic.row,
-                         sizeof(float) * c->ng, (size_t)lines, hipMemcpyDeviceToHost));
-    for (long long r = 0; r < lines; ++r) out[r * hrow + c->ng] = out[r * hrow + c->ng + 1] = 0.0f;
-    return kOk;
-  }
-  // records F[z][3] per line, of the transforms or of the net's corrected
-  // grid: copied a few lines at a time, one component picked on the host
-  const ForceLines fl = fi ? ForceLines{c->net->d_fi, 3LL * c->ng} : plain_lines(c);
+  if (!fi && !c->force_records) return grid_to_host(c, c->fgrid[axis], out);
+  // records F[z][3], of the transforms or of the net's corrected grid: copied
+  // a few lines at a time, one component picked on the host
+  const ForceLines fl = fi ? net_lines(c) : plain_lines(c);
   const long long lines = (long long)c->ng * c->ng, hrow = 2 * (c->ng / 2 + 1);
   const long long chunk = std::max(1LL, std::min(lines, (1LL << 24) / (3LL * c->ng)));
   std::vector<float> rec((size_t)(3LL * c->ng * chunk));
   for (long long l0 = 0; l0 < lines; l0 += chunk) {
     const long long nl = std::min(chunk, lines - l0);
-    COLA_HIP(hipMemcpy2D(rec.data(), sizeof(float) * 3 * c->ng, fl.f + l0 * fl.line, sizeof(float) * fl.line,
-                         sizeof(float) * 3 * c->ng, (size_t)nl, hipMemcpyDeviceToHost));
+    for (int t = 0, z = 0; z < c->ng; ++t, z += fl.rec_row)
+      COLA_HIP(hipMemcpy2D(rec.data() + 3 * z, sizeof(float) * 3 * c->ng, fl.f + fl.at[t] + l0 * fl.row, sizeof(float) * fl.row,
+                           sizeof(float) * 3 * std::min(fl.rec_row, c->ng - z), (size_t)nl, hipMemcpyDeviceToHost));
     for (long long l = 0; l < nl; ++l) {
       float* o = out + (l0 + l) * hrow;
       for (int z = 0; z < c->ng; ++z) o[z] = rec[(size_t)((l * c->ng + z) * 3 + axis)];
@@ -2539,11 +2535,11 @@ int cola_fft_time(int n, int reps, double* ms_out)
   FftPlan plan;
   COLA_TRY(plan.init(n, -1, -1, true));  // the PM layout: rows padded to 128 bytes
   const long long floats = (long long)n * n * 2 * plan.nzp;
-  float* buf[3] = {nullptr, nullptr, nullptr};  // work, pristine copy, force lines
+  float* buf[5] = {nullptr, nullptr, nullptr, nullptr, nullptr};  // work, pristine copy, 3 force grids
   hipEvent_t e0 = nullptr, e1 = nullptr;
   int st = kOk;
-  for (int b = 0; b < 3 && !st; ++b)
-    if (hipMalloc(&buf[b], sizeof(float) * floats * (b == 2 ? 3 : 1)) != hipSuccess) st = kErrAlloc;
+  for (int b = 0; b < 5 && !st; ++b)
+    if (hipMalloc(&buf[b], sizeof(float) * floats) != hipSuccess) st = kErrAlloc;
   if (!st && (hipEventCreate(&e0) != hipSuccess || hipEventCreate(&e1) != hipSuccess)) st = kErrHip;
   if (!st) {
     hipLaunchKernelGGL(k_fill_pattern, dim3((unsigned)((floats + 255) / 256)), dim3(256), 0, nullptr, buf[1], floats,
@@ -2563,7 +2559,7 @@ int cola_fft_time(int n, int reps, double* ms_out)
         else if (which == 1)
           st = plan.c2r(nullptr, buf[0], KOp::None, KOpParams{}, nullptr);
         else
-          st = plan.forces(buf[0], buf[2], kp, true, nullptr);
+          st = plan.forces(buf[0], buf + 2, kp, true, nullptr);
         (void)hipEventRecord(e1, nullptr);
         float ms = 0;
         if (!st && (hipEventSynchronize(e1) != hipSuccess || hipEventElapsedTime(&ms, e0, e1) != hipSuccess))

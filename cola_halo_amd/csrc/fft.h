@@ -56,8 +56,8 @@ struct KOpParams {
 // Element offset of position b and column c of a column pass whose positions
 // lie `stride` apart (a whole plane in the x pass).  b runs to n / R - 1 of the
 // pass's radix R: with a small first or last radix the offset passes 2^32 on
-// grids that fit the card (2250 = 2 3^2 5^3: 1124 x 3 planes of 2250 x 1136 =
-// 8.6e9), so it is formed in 64 bits.
+// grids that fit the card (3750 = 2 3 5^4, 211 GB, radix 2 first: 1874 x 3750 x
+// 1876 = 1.3e10), so it is formed in 64 bits.
 __host__ __device__ inline unsigned long long col_offset(int b, long long stride, int c)
 {
   return (unsigned long long)(unsigned)b * (unsigned)stride + (unsigned)c;
@@ -69,6 +69,15 @@ __host__ __device__ inline unsigned long long col_offset(int b, long long stride
 inline bool col_offsets_fit32(int m, long long stride, int log2T)
 {
   return col_offset(m - 1, stride, (1 << log2T) - 1) <= 0xffffffffULL;
+}
+
+// Records F[z][3] of a line per row of three force grids with rows of `row`
+// floats: a third of them, rounded up to what 16-byte (n and the result
+// multiples of 4) or 8-byte stores need.
+inline int record_row(int n, long long row)
+{
+  const int third = (n + 2) / 3, four = (third + 3) / 4 * 4;
+  return n % 4 == 0 && 3LL * four <= row ? four : (third + 1) / 2 * 2;
 }
 
 // Launch shape of one axis pass: 2^log2T transforms per workgroup, threads
@@ -85,6 +94,7 @@ struct FftPlan {
   float2* d_tw = nullptr;  // exp(-2 pi i k / n), k < n
   FftPassGeom grows, gy, gx;
   FftPassGeom gz3;  // z c2r of three components: threads of one component
+  int rec_row = 0;  // its records per row (record_row)
   int xgroup = 8;  // adjacent column tiles per XCD dispatch group (measured best)
   // Complex row stride of the half spectrum (>= n/2+1): rows padded to a
   // multiple of 16 complex values start on 128-byte lines, so column tiles
@@ -114,13 +124,14 @@ struct FftPlan {
   int c2r(const float2* in_k, float* out, KOp op, const KOpParams& kp, hipStream_t s) const;
   // The PM force fields in one sequence (pm.c:282-355): r2c of the padded
   // real density (in place; destroyed), Poisson gradient and c2r of the three
-  // components into `force`: per line (x, y) three slots of 2 nzp floats (on
-  // the way, the components' spectra).  records: the line's first 3 n floats
-  // are its records F[z][3]; else each slot holds its component's n values.
+  // components into the grids force[3] of the density's layout (on the way,
+  // the components' spectra).  records: together they hold the records
+  // F[z][3], a line's first rec_row ones in its row of force[0], the next in
+  // force[1], the rest in force[2]; else each holds its component.
   // Where can_fuse() holds, the forward x pass, the Poisson operator and the
   // inverse x passes run as one fused kernel (hook pass 6) and delta(k) is
   // never written to memory.
-  int forces(float* density, float* force, const KOpParams& kp, bool records, hipStream_t s) const;
+  int forces(float* density, float* const force[3], const KOpParams& kp, bool records, hipStream_t s) const;
   bool can_fuse() const;
 };
 
@@ -147,8 +158,8 @@ struct FftBatchStage {
 struct FftForcesBatch {
   std::vector<FftBatchStage> stages;
   void* d_mem = nullptr;
-  // plans[i] transforms density[i] (destroyed) into force[i] with the
-  // operator parameters kp[i].
+  // plans[i] transforms density[i] (destroyed) into the records of force[3 i]
+  // to force[3 i + 2] with the operator parameters kp[i].
   int init(const FftPlan* const* plans, float* const* density, float* const* force, const KOpParams* kp, int n,
            bool merge_all);
   int run(hipStream_t s) const;

@@ -182,9 +182,7 @@ struct TileArgs {
   int ncols;             // valid columns (kCols) or row pairs (kR2C / kC2R)
   long long sr;          // kCols: stride between positions of one transform
   long long bs;          // kCols: batch stride (blockIdx.y)
-  long long sr_out, bs_out;  // kCols: the same of the outputs
-  long long row_out = 0;     // x pass: row stride of the outputs where it is not nz
-  long long axis_in = 0;     // c2r of force lines: the next component's row
+  int rec_row;           // z c2r of three components: records per row
   long long rs_in;       // kR2C: real row stride (floats); kC2R: complex row stride
   long long rs_out;      // kR2C: complex row stride; kC2R: real row stride (floats)
   int nz;                // x pass: columns are (y, kz) pairs with kz < nz (the row stride)
@@ -193,12 +191,6 @@ struct TileArgs {
   int kz_valid = 0;      // x pass: tiles lying wholly in kz >= kz_valid (row padding) return at once
   KOpParams kp;
 };
-
-void set_strides(TileArgs& A, long long sr, long long bs)
-{
-  A.sr = A.sr_out = sr;
-  A.bs = A.bs_out = bs;
-}
 
 // An x-pass tile of 2^log2T columns starting at c0 that holds only padding
 // columns (kz_valid <= kz < nz within one row).
@@ -263,8 +255,8 @@ enum YScale : int { kYPlain = 0, kYByPosition = 1, kYByColumn = 2 };
 
 // Workgroup blk of a pass whose grid is nblk workgroups (the kernel's own
 // grid, or one job's share of a batched launch).
-// YS: the pass may scale (yscale); ROW_OUT: its outputs have rows of their own.
-template <int DIR, int MODE, KOp OP, int EMAX, int RS, bool YS = false, bool ROW_OUT = false>
+// YS: the pass may scale (yscale).
+template <int DIR, int MODE, KOp OP, int EMAX, int RS, bool YS = false>
 __device__ __forceinline__ void tile_run(const void* in_, void* out_, const float2* __restrict__ tw, const TileArgs& A,
                                          int blk, int nblk, int tid, int yscale = kYPlain, bool stage_twiddles = true)
 {
@@ -454,16 +446,15 @@ __device__ __forceinline__ void tile_run(const void* in_, void* out_, const floa
       if (u < nb && c0 + c < A.ncols) {
         // last pass: L = n / R = m, so b div L = 0 and the outputs sit at b + t*m
         if (MODE == kCols) {
-          float2* out = static_cast<float2*>(out_) + (long long)batch * A.bs_out + c0;
-          if (ROW_OUT) out += (long long)fdiv((unsigned)(c0 + c), (unsigned)A.nz, A.magNz) * (A.row_out - A.nz);
-          const unsigned long long lane = col_offset(b, A.sr_out, c);
+          float2* out = static_cast<float2*>(out_) + (long long)batch * A.bs + c0;
+          const unsigned long long lane = col_offset(b, A.sr, c);
           if (YS && yscale == kYByColumn) {
             const float w = (float)(c0 + c);
 #pragma unroll
             for (int t = 0; t < R; ++t) reg[q * R + t] = make_float2(w * reg[q * R + t].x, w * reg[q * R + t].y);
           }
 #pragma unroll
-          for (int t = 0; t < R; ++t) out[(long long)(t * p.m) * A.sr_out + lane] = reg[q * R + t];
+          for (int t = 0; t < R; ++t) out[(long long)(t * p.m) * A.sr + lane] = reg[q * R + t];
         } else {
           float* out = static_cast<float*>(out_) + (2LL * c0) * A.rs_out;
           const unsigned lane = (unsigned)(2 * c) * (unsigned)A.rs_out + (unsigned)b;
@@ -534,23 +525,23 @@ template <int DIR, int MODE, KOp OP, int EMAX, int RS>
 __global__ void __launch_bounds__(kFftMaxThreads) __attribute__((amdgpu_waves_per_eu(tile_waves_per_eu(MODE, OP, EMAX, RS))))
 fft_tile(const void* __restrict__ in_, void* __restrict__ out_, const float2* __restrict__ tw, TileArgs A)
 {
-  // (the operators of the force spectra write lines of three)
-  constexpr bool row_out = OP == KOp::PmPoisson || OP == KOp::PmCommon;
-  tile_run<DIR, MODE, OP, EMAX, RS, false, row_out>(in_, out_, tw, A, blockIdx.x, gridDim.x, threadIdx.x);
+  tile_run<DIR, MODE, OP, EMAX, RS>(in_, out_, tw, A, blockIdx.x, gridDim.x, threadIdx.x);
 }
 
 // ---- z c2r of the three force components of a line ---------------------------
-// One workgroup: T pairs of lines, whose three half spectra (rows axis_in
-// apart) become one line of records F[z][3] in their place.  A third of the
-// threads takes each component: its two rows are packed into one complex
-// transform as in the row pass; the last pass leaves its component of the
-// records in LDS, and the lines go out whole (storing a component every 12
-// bytes from registers took 3.88 ms at 768^3).  The readout then gathers one
-// record per CIC corner, 4 grid lines per particle instead of 12: the z pass
-// takes 3.45 ms for the three launches' 3.03 at 768^3 (0.83 for 1.09 at 480^3)
-// and the readout of 256^3 particles 1.08 for 2.16.
+// One workgroup: T pairs of lines, whose three half spectra (one in each of
+// three grids) become the lines' records F[z][3] in their place, a third of a
+// line in each grid's row.  A third of the threads takes each component: its
+// two rows are packed into one complex transform as in the row pass; the last
+// pass leaves its component of the records in LDS, and the rows go out whole
+// (storing a component every 12 bytes from registers took 3.88 ms at 768^3).
+// The readout then gathers one record per CIC corner, 4 grid lines per
+// particle instead of 12: the z pass takes 3.45 ms for the three launches'
+// 3.03 at 768^3 (0.83 for 1.09 at 480^3) and the readout of 256^3 particles
+// 1.08 for 2.16.
 template <int EMAX, int RS>
-__device__ __forceinline__ void c2r3_run(float* data, const float2* __restrict__ tw, const TileArgs& A, int blk)
+__device__ __forceinline__ void c2r3_run(float* f0, float* f1, float* f2, const float2* __restrict__ tw,
+                                         const TileArgs& A, int blk)
 {
   extern __shared__ float2 smem[];
   const int n = A.P.n;
@@ -564,7 +555,8 @@ __device__ __forceinline__ void c2r3_run(float* data, const float2* __restrict__
   for (int k = threadIdx.x; k < n; k += (int)blockDim.x) smem[k] = tw[k];
   const int np_ = A.P.npass;
   const int h = n / 2;
-  const float2* in = reinterpret_cast<const float2*>(data) + (2LL * c0) * A.rs_in + axis * A.axis_in;
+  float* const data = axis == 0 ? f0 : axis == 1 ? f1 : f2;
+  const float2* in = reinterpret_cast<const float2*>(data) + (2LL * c0) * A.rs_in;
 
   for (int pi = 0; pi < np_; ++pi) {
     radix_dispatch<RS>(A.P.pass[pi].R, [&](auto Rc) {
@@ -641,19 +633,20 @@ __device__ __forceinline__ void c2r3_run(float* data, const float2* __restrict__
       __syncthreads();
     });
   }
-  // the lines' records, contiguous: 16 bytes a lane (8 where n is no multiple of 4)
+  // the lines' records, each third of the threads its grid's rows: 16 bytes a
+  // lane (8 where a row's records do not end on 16)
   const int lines = 2 * min(1 << log2T, A.ncols - c0);
+  const int first = axis * A.rec_row, count = max(0, min(A.rec_row, n - first));
   auto copy = [&](auto v) {
     using V = decltype(v);
-    constexpr int W = sizeof(V) / sizeof(float);
-    const int per = 3 * n / W;
+    const int per = 3 * count / (int)(sizeof(V) / sizeof(float));
     for (int l = 0; l < lines; ++l) {
       V* const o = reinterpret_cast<V*>(data + (2LL * c0 + l) * A.rs_out);
-      const V* const st = reinterpret_cast<const V*>(stage + 3 * l * n);
-      for (int k = threadIdx.x; k < per; k += (int)blockDim.x) o[k] = st[k];
+      const V* const st = reinterpret_cast<const V*>(stage + 3 * (l * n + first));
+      for (int k = tid; k < per; k += nthr) o[k] = st[k];
     }
   };
-  if (n % 4 == 0)
+  if (n % 4 == 0 && A.rec_row % 4 == 0)
     copy(float4{});
   else
     copy(float2{});
@@ -662,9 +655,9 @@ __device__ __forceinline__ void c2r3_run(float* data, const float2* __restrict__
 template <int EMAX, int RS>
 __global__ void __launch_bounds__(kFftMaxThreads)
     __attribute__((amdgpu_waves_per_eu(tile_waves_per_eu(kC2R, KOp::None, EMAX, RS))))
-fft_c2r3(float* data, const float2* __restrict__ tw, TileArgs A)
+fft_c2r3(float* f0, float* f1, float* f2, const float2* __restrict__ tw, TileArgs A)
 {
-  c2r3_run<EMAX, RS>(data, tw, A, blockIdx.x);
+  c2r3_run<EMAX, RS>(f0, f1, f2, tw, A, blockIdx.x);
 }
 
 // ---- fused x pass: forward x FFT, then Poisson + inverse x FFT twice ---------
@@ -962,11 +955,10 @@ __device__ __forceinline__ void fused_run(const float2* __restrict__ in, float2*
             const int u = tid + q * nthr;
             const int c = u & tmask, b = u >> log2T;
             if (u < nb && c0 + c < A.ncols) {
-              const int iy = (int)fdiv((unsigned)(c0 + c), (unsigned)A.nz, A.magNz);
-              float2* out = (axis == 0 ? out0 : out1) + c0 + (long long)iy * (A.row_out - A.nz);
-              const unsigned lane = (unsigned)b * (unsigned)A.sr_out + (unsigned)c;
+              float2* out = (axis == 0 ? out0 : out1) + c0;
+              const unsigned lane = (unsigned)b * (unsigned)A.sr + (unsigned)c;
 #pragma unroll
-              for (int t = 0; t < R; ++t) out[(long long)(t * p.m) * A.sr_out + lane] = r2[q * R + t];
+              for (int t = 0; t < R; ++t) out[(long long)(t * p.m) * A.sr + lane] = r2[q * R + t];
             }
           }
         }
@@ -1052,8 +1044,7 @@ void set_groups(TileArgs& A, int tpb, int group)
 // outputs are those of the separate launches bit for bit.
 struct TileJob {
   const void* in;
-  void* out;
-  void* out2;  // y inverse: the second output, or null
+  void* out[3];  // y inverse: out[1] the second output, or null; z c2r of three: the grids
   const float2* tw;
   TileArgs A;
   int blocks;
@@ -1077,7 +1068,7 @@ fft_tile_jobs(const TileJob* __restrict__ jobs, const int* __restrict__ start, i
   const TileJob& J = jobs[j];
   const int lb = (int)blockIdx.x - start[j];
   if (lb >= J.blocks) return;  // alignment padding (before any barrier)
-  tile_run<DIR, MODE, KOp::None, EMAX, RS>(J.in, J.out, J.tw, J.A, lb, J.blocks, threadIdx.x);
+  tile_run<DIR, MODE, KOp::None, EMAX, RS>(J.in, J.out[0], J.tw, J.A, lb, J.blocks, threadIdx.x);
 }
 
 // (6 waves per SIMD at 8 values per thread: with 8 the tables' arguments spill)
@@ -1090,8 +1081,8 @@ fft_yinv_jobs(const TileJob* __restrict__ jobs, const int* __restrict__ start, i
   const TileJob& J = jobs[j];
   const int lb = (int)blockIdx.x - start[j];
   if (lb >= J.blocks) return;
-  yinv_run<EMAX, RS>(static_cast<const float2*>(J.in), static_cast<float2*>(J.out), static_cast<float2*>(J.out2), J.tw,
-                     J.A, lb, J.blocks);
+  yinv_run<EMAX, RS>(static_cast<const float2*>(J.in), static_cast<float2*>(J.out[0]), static_cast<float2*>(J.out[1]),
+                     J.tw, J.A, lb, J.blocks);
 }
 
 template <int EMAX, int RS>
@@ -1101,7 +1092,8 @@ fft_c2r3_jobs(const TileJob* __restrict__ jobs, const int* __restrict__ start, i
 {
   const int j = batch_find(start, njobs, blockIdx.x);
   const TileJob& J = jobs[j];
-  c2r3_run<EMAX, RS>(static_cast<float*>(J.out), J.tw, J.A, (int)blockIdx.x - start[j]);
+  c2r3_run<EMAX, RS>(static_cast<float*>(J.out[0]), static_cast<float*>(J.out[1]), static_cast<float*>(J.out[2]), J.tw,
+                     J.A, (int)blockIdx.x - start[j]);
 }
 
 template <int EMAX, int RS, bool WIDE>
@@ -1291,6 +1283,7 @@ int FftPlan::init(int n_, int log2T_cols, int log2T_rows, bool pad_rows, int log
   grows = pick(log2T_rows >= 0 ? log2T_rows : 1, (long long)n * n / 2);
   if (gx.emax == 0 || gy.emax == 0 || grows.emax == 0) return kErrUnsupported;
   gz3 = rows3_geom(rad, grows.log2T, log2T_rows >= 0);
+  rec_row = record_row(n, 2LL * nzp);
   std::vector<float2> tw(n);
   for (int k = 0; k < n; ++k) {
     const double a = -2.0 * kPiD * (double)k / (double)n;
@@ -1329,7 +1322,8 @@ int FftPlan::r2c(float* data, hipStream_t s) const
   // y: columns kz of each x plane
   A.log2T = gy.log2T;
   A.ncols = (int)nz;
-  set_strides(A, np_, (long long)n * np_);
+  A.sr = np_;
+  A.bs = (long long)n * np_;
   set_groups(A, grid_x(nz, gy.log2T), xgroup);
   mark(1, 1);
   COLA_TRY((launch_tile<-1, kCols, KOp::None>(gy, dim3(A.tpb_pad * n), s, cdata, cdata, d_tw, A)));
@@ -1338,7 +1332,8 @@ int FftPlan::r2c(float* data, hipStream_t s) const
   const long long ncols = (long long)n * np_;
   A.log2T = gx.log2T;
   A.ncols = (int)ncols;
-  set_strides(A, ncols, 0);
+  A.sr = ncols;
+  A.bs = 0;
   A.nz = (int)np_;
   A.kz_valid = np_ > nz ? (int)nz : 0;
   set_groups(A, grid_x(ncols, gx.log2T), xgroup);
@@ -1402,8 +1397,7 @@ static int launch_fused_r(const FftPassGeom& g, int grid, hipStream_t s, const f
 bool FftPlan::can_fuse() const
 {
   if (rad.npass < 2 || gx.emax > 12) return false;
-  // its loads and stores: plane strides of the density and of a line of three
-  if (!col_offsets_fit32(rad.pass[0].m, 3LL * n * nzp, gx.log2T)) return false;
+  if (!col_offsets_fit32(rad.pass[0].m, (long long)n * nzp, gx.log2T)) return false;
   const int RL = rad.pass[rad.npass - 1].R;
   return RL == 3 || RL == 4 || RL == 5 || RL == 8;
 }
@@ -1415,18 +1409,18 @@ namespace {
 // the three components.
 struct ForceJobs {
   TileJob zr2c, yfwd, yinv[2];
-  TileJob zc2r, zslot[3];  // records, or the components apart
+  TileJob zc2r, zone[3];  // records, or the components apart
   FusedJob x;
 };
 
-void make_force_jobs(const FftPlan& P, float* density, float* force, const KOpParams& kp, ForceJobs* J)
+void make_force_jobs(const FftPlan& P, float* density, float* const force[3], const KOpParams& kp, ForceJobs* J)
 {
   const int n = P.n;
   const long long nz = n / 2 + 1, np_ = P.nzp;
   const int npairs = n * n / 2;
   float2* cdata = reinterpret_cast<float2*>(density);
-  float2* cforce = reinterpret_cast<float2*>(force);
-  const long long frow = 3 * np_;  // a line of force: three spectra, then n records
+  float2* spec[3];
+  for (int a = 0; a < 3; ++a) spec[a] = reinterpret_cast<float2*>(force[a]);
   TileArgs A;
   A.P = P.rad;
   A.kp = kp;
@@ -1438,24 +1432,24 @@ void make_force_jobs(const FftPlan& P, float* density, float* force, const KOpPa
   A.ncols = npairs;
   A.rs_in = 2 * np_;
   A.rs_out = np_;
-  J->zr2c = TileJob{density, cdata, nullptr, P.d_tw, A, grid_x(npairs, P.grows.log2T)};
+  J->zr2c = TileJob{density, {cdata, nullptr, nullptr}, P.d_tw, A, grid_x(npairs, P.grows.log2T)};
   A.log2T = P.gy.log2T;
   A.ncols = (int)nz;
-  set_strides(A, np_, (long long)n * np_);
+  A.sr = np_;
+  A.bs = (long long)n * np_;
   set_groups(A, grid_x(nz, P.gy.log2T), P.xgroup);
-  J->yfwd = TileJob{cdata, cdata, nullptr, P.d_tw, A, A.tpb_pad * n};
+  J->yfwd = TileJob{cdata, {cdata, nullptr, nullptr}, P.d_tw, A, A.tpb_pad * n};
   // x: forward, Poisson, inverse (row padding tiles return at once)
   const long long ncols = (long long)n * np_;
   A.log2T = P.gx.log2T;
   A.ncols = (int)ncols;
-  set_strides(A, ncols, 0);
-  A.sr_out = n * frow;
-  A.row_out = frow;
+  A.sr = ncols;
+  A.bs = 0;
   A.kz_valid = np_ > nz ? (int)nz : 0;
   set_groups(A, grid_x(ncols, P.gx.log2T), P.xgroup);
   FusedJob& x = J->x;
   x.in = cdata;
-  for (int a = 0; a < 2; ++a) x.out[a] = cforce + a * np_;
+  for (int a = 0; a < 2; ++a) x.out[a] = spec[a];
   x.tw = P.d_tw;
   x.A = A;
   x.Pinv = reversed(P.rad);
@@ -1465,19 +1459,21 @@ void make_force_jobs(const FftPlan& P, float* density, float* force, const KOpPa
   B.kz_valid = 0;
   B.log2T = P.gy.log2T;
   B.ncols = (int)nz;
-  set_strides(B, frow, n * frow);
+  B.sr = np_;
+  B.bs = (long long)n * np_;
   set_groups(B, grid_x(nz, P.gy.log2T), P.xgroup);
-  J->yinv[0] = TileJob{x.out[0], x.out[0], nullptr, P.d_tw, B, B.tpb_pad * n};
-  J->yinv[1] = TileJob{x.out[1], x.out[1], cforce + 2 * np_, P.d_tw, B, B.tpb_pad * n};
+  J->yinv[0] = TileJob{spec[0], {spec[0], nullptr, nullptr}, P.d_tw, B, B.tpb_pad * n};
+  J->yinv[1] = TileJob{spec[1], {spec[1], spec[2], nullptr}, P.d_tw, B, B.tpb_pad * n};
   B.log2T = P.gz3.log2T;
   B.ncols = npairs;
-  B.rs_in = frow;
-  B.axis_in = np_;
-  B.rs_out = 2 * frow;
-  J->zc2r = TileJob{force, force, nullptr, P.d_tw, B, grid_x(npairs, P.gz3.log2T)};
+  B.rs_in = np_;
+  B.rs_out = 2 * np_;
+  B.zero_pad = np_ == nz;
+  B.rec_row = P.rec_row;
+  J->zc2r = TileJob{force[0], {force[0], force[1], force[2]}, P.d_tw, B, grid_x(npairs, P.gz3.log2T)};
   B.log2T = P.grows.log2T;
   for (int a = 0; a < 3; ++a)
-    J->zslot[a] = TileJob{cforce + a * np_, force + 2 * a * np_, nullptr, P.d_tw, B, grid_x(npairs, P.grows.log2T)};
+    J->zone[a] = TileJob{spec[a], {force[a], nullptr, nullptr}, P.d_tw, B, grid_x(npairs, P.grows.log2T)};
 }
 
 // The launchers of the y inverse and the z c2r, one grid or a batch of jobs
@@ -1559,7 +1555,7 @@ int launch_fused_jobs_e(const FftBatchStage& st, hipStream_t s)
 
 }  // namespace
 
-int FftPlan::forces(float* density, float* force, const KOpParams& kp, bool records, hipStream_t s) const
+int FftPlan::forces(float* density, float* const force[3], const KOpParams& kp, bool records, hipStream_t s) const
 {
   if (records && gz3.emax == 0) {
     set_error("force transforms: the grid's rows exceed a workgroup's LDS");
@@ -1571,7 +1567,7 @@ int FftPlan::forces(float* density, float* force, const KOpParams& kp, bool reco
   ForceJobs J;
   make_force_jobs(*this, density, force, kp, &J);
   auto tile = [&](auto dir, auto mode, const FftPassGeom& g, const TileJob& t) {
-    return launch_tile<decltype(dir)::value, decltype(mode)::value, KOp::None>(g, dim3(t.blocks), s, t.in, t.out,
+    return launch_tile<decltype(dir)::value, decltype(mode)::value, KOp::None>(g, dim3(t.blocks), s, t.in, t.out[0],
                                                                               t.tw, t.A);
   };
   using Fwd = std::integral_constant<int, -1>;
@@ -1594,11 +1590,8 @@ int FftPlan::forces(float* density, float* force, const KOpParams& kp, bool reco
     mark(6, 0);
   } else {
     // x forward in place, then the inverse of each spectrum with its operator on the load
-    TileArgs F = x.A;
-    set_strides(F, F.sr, 0);
-    F.row_out = 0;
     mark(2, 1);
-    COLA_TRY((launch_tile<-1, kCols, KOp::None>(gx, dim3(x.blocks), s, x.in, density, d_tw, F)));
+    COLA_TRY((launch_tile<-1, kCols, KOp::None>(gx, dim3(x.blocks), s, x.in, density, d_tw, x.A)));
     mark(2, 0);
     mark(3, 1);
     COLA_TRY((launch_tile<1, kCols, KOp::PmPoisson>(gx, dim3(x.blocks), s, x.in, x.out[0], d_tw, x.A)));
@@ -1610,14 +1603,14 @@ int FftPlan::forces(float* density, float* force, const KOpParams& kp, bool reco
   for (const TileJob& t : J.yinv) {
     mark(4, 1);
     COLA_TRY((launch_variant<YInv>(gy.emax, rs348, dim3(t.blocks), gy.threads, tile_lds_bytes(kCols, n, gy.log2T), s,
-                                   static_cast<const float2*>(t.in), static_cast<float2*>(t.out),
-                                   static_cast<float2*>(t.out2), t.tw, t.A)));
+                                   static_cast<const float2*>(t.in), static_cast<float2*>(t.out[0]),
+                                   static_cast<float2*>(t.out[1]), t.tw, t.A)));
     mark(4, 0);
   }
   using Inv = std::integral_constant<int, 1>;
   for (int a = 0; a < 3 && !records; ++a) {
     mark(5, 1);
-    COLA_TRY(tile(Inv{}, std::integral_constant<int, kC2R>{}, grows, J.zslot[a]));
+    COLA_TRY(tile(Inv{}, std::integral_constant<int, kC2R>{}, grows, J.zone[a]));
     mark(5, 0);
   }
   if (!records) {
@@ -1626,7 +1619,7 @@ int FftPlan::forces(float* density, float* force, const KOpParams& kp, bool reco
   }
   mark(5, 1);
   COLA_TRY((launch_variant<C2R3>(gz3.emax, rs348, dim3(J.zc2r.blocks), 3 * gz3.threads, c2r3_lds_bytes(n, gz3.log2T),
-                                 s, force, static_cast<const float2*>(d_tw), J.zc2r.A)));
+                                 s, force[0], force[1], force[2], static_cast<const float2*>(d_tw), J.zc2r.A)));
   mark(5, 0);
   COLA_HIP(hipGetLastError());
   return kOk;
@@ -1643,7 +1636,7 @@ int FftForcesBatch::init(const FftPlan* const* plans, float* const* density, flo
       set_error("batched force transforms need plans whose x pass fuses");
       return kErrUnsupported;
     }
-    make_force_jobs(*plans[i], density[i], force[i], kp[i], &fj[i]);
+    make_force_jobs(*plans[i], density[i], force + 3 * i, kp[i], &fj[i]);
   }
   // the jobs of the five passes and each job's own launch geometry
   struct Pass {
@@ -1821,7 +1814,8 @@ int FftPlan::c2r(const float2* in_k, float* out, KOp op, const KOpParams& kp, hi
   const long long ncols = (long long)n * np_;
   A.log2T = gx.log2T;
   A.ncols = (int)ncols;
-  set_strides(A, ncols, 0);
+  A.sr = ncols;
+  A.bs = 0;
   A.kz_valid = np_ > nz ? (int)nz : 0;
   set_groups(A, grid_x(ncols, gx.log2T), xgroup);
   const float2* src = in_k ? in_k : cout;
@@ -1842,7 +1836,8 @@ int FftPlan::c2r(const float2* in_k, float* out, KOp op, const KOpParams& kp, hi
   // y
   A.log2T = gy.log2T;
   A.ncols = (int)nz;
-  set_strides(A, np_, (long long)n * np_);
+  A.sr = np_;
+  A.bs = (long long)n * np_;
   A.kz_valid = 0;
   set_groups(A, grid_x(nz, gy.log2T), xgroup);
   mark(4, 1);

@@ -112,14 +112,25 @@ int launch_grid_contrast(const PosSource& src, int n, float boxsize, const GridB
                          long long capacity, int* overflow, unsigned long long* fix, long long row, float nbar_inv,
                          float* grid, double* sums, hipStream_t s);
 
-// A force grid: per line (x ng + y) the records F[z][3], lines `line` floats
-// apart (6 nzp where the transforms left them, 3 ng in the net's grid), or,
-// slot > 0, the components' rows `slot` floats apart.
+// A force grid, as components apart (component a of a cell at f + at[a]) or as
+// records F[z][3]: rows `row` floats apart, a line's (x ng + y) first rec_row
+// records in its row at f, the next in the one at f + at[1], the rest at f +
+// at[2] (rec_row = ng, of a net's grid: all in one row of 3 ng).
 struct ForceLines {
   const float* f = nullptr;
-  long long line = 0;
-  long long slot = 0;
+  long long at[3] = {0, 0, 0};
+  long long row = 0;
+  int rec_row = 0;  // 0: components apart
 };
+
+// Of record z, its place in line 0.
+__device__ inline long long force_record(const ForceLines& fl, int z)
+{
+  const int k = fl.rec_row;
+  long long o = z < k ? 0 : fl.at[1] - 3 * k;
+  o = z < 2 * k ? o : fl.at[2] - 6 * k;
+  return o + 3 * z;
+}
 
 // pm.c:359-412 + 505-532: readout of the force grid into p.f.
 // fsum: null, or the three sums of a residual added to the force grid,

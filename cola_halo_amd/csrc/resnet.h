@@ -87,9 +87,9 @@ int resnet_body(ResNet* r, const float* pa, hipStream_t s);
 // resnet_body in its two launches groups: layer 1 (from d_f1), layers 2-3
 int resnet_layer1(ResNet* r, const float* pa, hipStream_t s);
 int resnet_layers23(ResNet* r, hipStream_t s);
-// force component a (f + a slot, lines `line` floats apart) + out_scale * y[a]
-// into d_fi[cell][a] (d_fsum gets the sums of the residual added)
-int resnet_head_add(ResNet* r, float* f, long long slot, long long line, hipStream_t s);
+// force component f[a] (rows `row` floats apart) + out_scale * y[a] into
+// d_fi[cell][a] (d_fsum gets the sums of the residual added)
+int resnet_head_add(ResNet* r, float* const f[3], long long row, hipStream_t s);
 // The inference path with the first two layers fused (fuse12): h2 straight
 // from the real-space density grid (features, layer 1 and layer 2 in one
 // launch, a read from pa), then layer 3; equal to resnet_features,
@@ -99,7 +99,7 @@ int resnet_layer3(ResNet* r, hipStream_t s);
 // Layer 3 and the last layer in one launch (from h2, after the force
 // transforms): the corrected force into d_fi as resnet_layer3 followed by
 // resnet_head_add, bit for bit, without writing h3.  By input planes only.
-int resnet_layer3_head(ResNet* r, float* f, long long slot, long long line, hipStream_t s);
+int resnet_layer3_head(ResNet* r, float* const f[3], long long row, hipStream_t s);
 // loss against target (bf16 [3][n^3] or fp32 [3][n^3]) and gradient into d_grad
 int resnet_backward(ResNet* r, const unsigned short* target_bf16, const float* target_f32, hipStream_t s);
 int resnet_adam(ResNet* r, float lr, hipStream_t s);

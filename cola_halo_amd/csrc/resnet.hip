@@ -71,7 +71,7 @@ enum ConvMode { kFwdRelu = 0, kFwdLinear = 1, kBwdData = 2, kFwdAdd = 3 };
 
 // Outputs of a convolution by mode: bf16 activations (kFwdRelu; kBwdData
 // masked by relu'(hprev)), the fp32 net output y [3][n^3] (kFwdLinear), or
-// scale * y added to three force components add[a] with lines `row` floats
+// scale * y added to three force components add[a] with rows `row` floats
 // apart (kFwdAdd: the corrected PM force).
 struct ConvOut {
   unsigned short* bf = nullptr;
@@ -1773,24 +1773,26 @@ __global__ void k_adam(float* __restrict__ p, float* __restrict__ m, float* __re
   p[i] -= lr * (mi / c1) / (sqrtf(vi / c2) + eps);
 }
 
+__device__ inline float force_value(const ForceLines& fl, int comp, long long line, int z)
+{
+  return fl.f[line * fl.row + (fl.rec_row ? force_record(fl, z) + comp : fl.at[comp] + z)];
+}
+
 // Fine force restricted to coarse cell (x, y, z): the average over the 3^3
 // fine neighbours of the coincident fine cell (2x, 2y, 2z) with weights
 // (ws, 1 - 2 ws, ws) per axis, periodic (ws = 0: the point value, 1/4: full
 // weighting).
-// Component a (of records f[z][3] per line) of the restricted fine force.
 __device__ inline float restrict_fine(const ForceLines& ff, int comp, int nf, int x, int y, int z, float ws)
 {
-  const float* __restrict__ f = ff.f + comp * (ff.slot ? ff.slot : 1);
-  const int zs = ff.slot ? 1 : 3;
-  if (ws == 0.0f) return f[((long long)(2 * x) * nf + 2 * y) * ff.line + zs * (2 * z)];
+  if (ws == 0.0f) return force_value(ff, comp, (long long)(2 * x) * nf + 2 * y, 2 * z);
   const float w[3] = {ws, 1.0f - 2.0f * ws, ws};
   float s = 0.0f;
   for (int a = 0; a < 3; ++a) {
     const int fx = wrapi(2 * x + a - 1, nf);
     for (int b = 0; b < 3; ++b) {
-      const long long row = ((long long)fx * nf + wrapi(2 * y + b - 1, nf)) * ff.line;
+      const long long line = (long long)fx * nf + wrapi(2 * y + b - 1, nf);
       const float wab = w[a] * w[b];
-      for (int c = 0; c < 3; ++c) s += wab * w[c] * f[row + zs * wrapi(2 * z + c - 1, nf)];
+      for (int c = 0; c < 3; ++c) s += wab * w[c] * force_value(ff, comp, line, wrapi(2 * z + c - 1, nf));
     }
   }
   return s;
@@ -1808,9 +1810,8 @@ __global__ void k_store_pair(const float* __restrict__ cd, long long crow, Force
   const long long xy = cell / n;
   const int y = (int)(xy % n), x = (int)(xy / n);
   feat[cell] = feature_of(cd[xy * crow + z], scale);
-  const float* __restrict__ c = cf.f + xy * cf.line + (cf.slot ? 1 : 3) * z;
-  const long long slot = cf.slot ? cf.slot : 1;
-  for (int a = 0; a < 3; ++a) target[a * nc + cell] = f2bf(restrict_fine(ff, a, 2 * n, x, y, z, ws) - c[a * slot]);
+  for (int a = 0; a < 3; ++a)
+    target[a * nc + cell] = f2bf(restrict_fine(ff, a, 2 * n, x, y, z, ws) - force_value(cf, a, xy, z));
 }
 
 __global__ void __launch_bounds__(kThreads) k_sumsq(const unsigned short* __restrict__ t, long long n, double* out)
@@ -2195,11 +2196,11 @@ int resnet_layer3(ResNet* r, hipStream_t s)
   return kOk;
 }
 
-int resnet_head_add(ResNet* r, float* f, long long slot, long long line, hipStream_t s)
+int resnet_head_add(ResNet* r, float* const f[3], long long row, hipStream_t s)
 {
   ConvOut o;
-  for (int a = 0; a < 3; ++a) o.add[a] = f + a * slot;
-  o.row = line;
+  for (int a = 0; a < 3; ++a) o.add[a] = f[a];
+  o.row = row;
   o.scale = r->out_scale;
   hipLaunchKernelGGL(k_zero3, dim3(1), dim3(64), 0, s, r->d_fsum);
   o.sum = r->d_fsum;
@@ -2207,12 +2208,12 @@ int resnet_head_add(ResNet* r, float* f, long long slot, long long line, hipStre
   return conv_layer_4(r, kFwdAdd, o, s);
 }
 
-int resnet_layer3_head(ResNet* r, float* f, long long slot, long long line, hipStream_t s)
+int resnet_layer3_head(ResNet* r, float* const f[3], long long row, hipStream_t s)
 {
   COLA_TRY(conv_lds_attributes());
   ConvOut o;
-  for (int a = 0; a < 3; ++a) o.add[a] = f + a * slot;
-  o.row = line;
+  for (int a = 0; a < 3; ++a) o.add[a] = f[a];
+  o.row = row;
   o.scale = r->out_scale;
   hipLaunchKernelGGL(k_zero3, dim3(1), dim3(64), 0, s, r->d_fsum);
   o.sum = r->d_fsum;
