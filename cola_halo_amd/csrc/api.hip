@@ -344,11 +344,12 @@ KOpParams pm_kop(const cola_context* c)
 
 // Whether the transforms of the context leave records F[z][3] for the
 // readout (not for the net's last layer, which reads the components apart).
-// On long rows the z c2r of three components loses more than the readout
-// gains: at 1536^3 27.0 ms for 17.4, the readout of 512^3 particles 7.9 for
-// 11.3; at 768^3 3.45 for 3.03, of 256^3 particles 1.08 for 2.16.
-constexpr int kRecordsMaxGrid = 1024;
-bool writes_records(const cola_context* c) { return !c->net && c->ng <= kRecordsMaxGrid; }
+// The z c2r of three components takes longer than three launches and the
+// readout gains more: 3.45 ms for 3.00 and 1.13 for 2.6 (256^3 particles on
+// 768^3, a = 0.5), 7.6 for 6.4 and 6.9 for 15.2 (512^3 on 1024^3), 25.1 for 23.6
+// and 9.4 for 21.8 (512^3 on 1536^3; 7.7 for 12.0 at a = 0.1, where the
+// particles are still near their lattice).
+bool writes_records(const cola_context* c) { return !c->net; }
 
 int pm_fields(cola_context* c)
 {

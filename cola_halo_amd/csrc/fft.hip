@@ -538,7 +538,7 @@ fft_tile(const void* __restrict__ in_, void* __restrict__ out_, const float2* __
 // The readout then gathers one record per CIC corner, 4 grid lines per
 // particle instead of 12: the z pass takes 3.45 ms for the three launches'
 // 3.03 at 768^3 (0.83 for 1.09 at 480^3) and the readout of 256^3 particles
-// 1.08 for 2.16.
+// 1.13 for 2.16.
 template <int EMAX, int RS>
 __device__ __forceinline__ void c2r3_run(float* f0, float* f1, float* f2, const float2* __restrict__ tw,
                                          const TileArgs& A, int blk)
@@ -675,7 +675,7 @@ struct ColCtx {
 // index from (o + t L, c), with a 32-bit multiply per twiddle, was most of the
 // fused pass's VALU work, which bounds it: with f1 / k^2 folded into the kept
 // spectrum as well, 270^3 0.163 -> 0.129 ms, 384^3 0.327 -> 0.235, 480^3 0.90
-// -> 0.56, 768^3 2.98 -> 2.78.)
+// -> 0.56, 768^3 2.98 -> 2.78, all of it with outputs in lines of three.)
 template <int R, int EMAX, int DIR>
 __device__ inline void col_compute(float2 (&reg)[EMAX], const FftPass& p, const ColCtx& x)
 {
@@ -735,8 +735,8 @@ __device__ inline void col_load_lds(float2 (&reg)[EMAX], const FftPass& p, const
 // transforms it twice, unscaled (written times n_z to out2), then times n_y
 // (in place).  Two grids in and three out here and one in and two out in the
 // x pass, where three in and three out and one in and three out were: bound
-// by the HBM as before, at 768^3 the x pass takes 2.98 ms for 3.52, the two y
-// launches 2.41 for the three's 2.45; 480^3 0.90 for 1.00 and 0.76 for 1.16.
+// by the HBM as before, the two y launches take 2.30 ms for the three's 2.45 at
+// 768^3, 0.72 for 1.16 at 480^3, 22.2 for 22.9 at 1536^3.
 // (Reading the tile a second time instead of keeping it: 4.18 ms at 768^3.)
 template <int EMAX, int RS>
 __device__ __forceinline__ void yinv_run(const float2* in, float2* out, float2* out2, const float2* __restrict__ tw,

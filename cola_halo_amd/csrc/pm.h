@@ -134,7 +134,7 @@ __device__ inline long long force_record(const ForceLines& fl, int z)
 
 // pm.c:359-412 + 505-532: readout of the force grid into p.f.
 // fsum: null, or the three sums of a residual added to the force grid,
-// whose mean is taken off every particle's force.
+// whose mean is taken off every particle's force.  f: records.
 int launch_readout(const DevParticles& p, const CicGeom& g, const ForceLines& f, const double* fsum, hipStream_t s);
 // Readout fused with cola.c:104-112 kick and cola.c:142-149 drift.
 int launch_readout_kick_drift(const DevParticles& p, const CicGeom& g, const ForceLines& f, const StepParams* prm,

@@ -808,11 +808,10 @@ struct Gather3 {
 // The three components of the CIC gather at one position, term order of
 // pm.c:397-410, from records F[z][3]: a corner's components are one 12-byte
 // record, so a particle touches four grid lines instead of the twelve of three
-// separate components: the fused readout, bound by those gathers, takes 1.08 ms
-// for 2.16 (256^3 on 768^3), 0.39 for 0.74 (192^3 on 480^3).
-enum Layout : int { kApart = 0, kSplit = 1, kWhole = 2 };  // of ForceLines: rec_row 0, a third of ng, ng
-
-template <Layout LAY>
+// separate components: the fused readout, bound by those gathers, takes 1.13 ms
+// for 2.16 (256^3 on 768^3), 0.42 for 0.74 (192^3 on 480^3).  SPLIT: a line's
+// records lie in three rows (rec_row a third of ng), else in one.
+template <bool SPLIT>
 __device__ inline Gather3 cic_gather(float x, float y, float z, const CicGeom& g, const ForceLines& fl)
 {
   const int ng = g.ng;
@@ -838,13 +837,9 @@ __device__ inline Gather3 cic_gather(float x, float y, float z, const CicGeom& g
   if (J1 >= ng) J1 = 0;
   int K1 = K + 1;
   if (K1 >= ng) K1 = 0;
-  const long long rK = LAY == kSplit ? force_record(fl, K) : LAY == kWhole ? 3 * K : K;
-  const long long rK1 = LAY == kSplit ? force_record(fl, K1) : LAY == kWhole ? 3 * K1 : K1;
-  auto rec = [&](long long line, long long r) {
-    const float* const f = fl.f + line * fl.row + r;
-    if (LAY != kApart) return *reinterpret_cast<const float3*>(f);
-    return make_float3(f[0], f[fl.at[1]], f[fl.at[2]]);
-  };
+  const long long rK = SPLIT ? force_record(fl, K) : 3 * K;
+  const long long rK1 = SPLIT ? force_record(fl, K1) : 3 * K1;
+  auto rec = [&](long long line, long long r) { return *reinterpret_cast<const float3*>(fl.f + line * fl.row + r); };
   if (0 <= iI && iI < ng) {
     const long long a = (long long)iI * ng + J, b = (long long)iI * ng + J1;
     const float3 aK = rec(a, rK), aK1 = rec(a, rK1), bK = rec(b, rK), bK1 = rec(b, rK1);
@@ -866,12 +861,12 @@ __device__ inline Gather3 cic_gather(float x, float y, float z, const CicGeom& g
 
 // Force at a particle: its own gather plus, beyond the ghost threshold, the
 // gather at its ghost position added afterwards (pm.c:526-531).
-template <Layout LAY>
+template <bool SPLIT>
 __device__ inline Gather3 particle_force(float x, float y, float z, const CicGeom& g, const ForceLines& fl)
 {
-  Gather3 f = cic_gather<LAY>(x, y, z, g, fl);
+  Gather3 f = cic_gather<SPLIT>(x, y, z, g, fl);
   if (x > g.x_right) {
-    const Gather3 h = cic_gather<LAY>(x + g.shift, y, z, g, fl);
+    const Gather3 h = cic_gather<SPLIT>(x + g.shift, y, z, g, fl);
 #pragma unroll
     for (int a = 0; a < 3; ++a) f.f[a] += h.f[a];
   }
@@ -888,13 +883,13 @@ __device__ inline void residual_mean(const double* __restrict__ fsum, float inv_
   for (int a = 0; a < 3; ++a) m[a] = fsum ? (float)(fsum[a] * (double)inv_cells) : 0.0f;
 }
 
-template <Layout LAY>
+template <bool SPLIT>
 __global__ void __launch_bounds__(kThreads)
 k_readout(DevParticles p, CicGeom g, ForceLines fl, const double* __restrict__ fsum, float inv_cells)
 {
   const long long i = (long long)xcd_group_remap(blockIdx.x, gridDim.x, g.readout_group) * kThreads + threadIdx.x;
   if (i >= p.np) return;
-  Gather3 f = particle_force<LAY>(p.x[0][i], p.x[1][i], p.x[2][i], g, fl);
+  Gather3 f = particle_force<SPLIT>(p.x[0][i], p.x[1][i], p.x[2][i], g, fl);
   float m[3];
   residual_mean(fsum, inv_cells, m);
 #pragma unroll
@@ -915,7 +910,7 @@ __device__ inline float drift1(float x, float v, float dx1, float dx2, const Dri
 }
 
 // Block blk of nblk (the member's own grid) of the fused readout.
-template <Layout LAY>
+template <bool SPLIT>
 __device__ __forceinline__ void readout_kick_drift_block(const DevParticles& p, const CicGeom& g,
                                                          const ForceLines& fl, const StepParams* __restrict__ prm,
                                                          const double* __restrict__ fsum, float inv_cells, int blk,
@@ -928,7 +923,7 @@ __device__ __forceinline__ void readout_kick_drift_block(const DevParticles& p, 
   float x[3];
 #pragma unroll
   for (int a = 0; a < 3; ++a) x[a] = p.x[a][i];
-  Gather3 f = particle_force<LAY>(x[0], x[1], x[2], g, fl);
+  Gather3 f = particle_force<SPLIT>(x[0], x[1], x[2], g, fl);
   if (fsum) {
     float m[3];
     residual_mean(fsum, inv_cells, m);
@@ -944,12 +939,12 @@ __device__ __forceinline__ void readout_kick_drift_block(const DevParticles& p, 
   }
 }
 
-template <Layout LAY>
+template <bool SPLIT>
 __global__ void __launch_bounds__(kThreads)
 k_readout_kick_drift(DevParticles p, CicGeom g, ForceLines fl, const StepParams* __restrict__ prm,
                      const double* __restrict__ fsum, float inv_cells)
 {
-  readout_kick_drift_block<LAY>(p, g, fl, prm, fsum, inv_cells, blockIdx.x, gridDim.x);
+  readout_kick_drift_block<SPLIT>(p, g, fl, prm, fsum, inv_cells, blockIdx.x, gridDim.x);
 }
 
 __global__ void __launch_bounds__(kThreads) k_kick(DevParticles p, KickFactors kf)
@@ -1086,7 +1081,7 @@ k_readout_kick_drift_batch(const PmMember* __restrict__ ms, const int* __restric
   const int nb = (int)((M.p.np + kThreads - 1) / kThreads);
   const int lb = (int)blockIdx.x - start[m];
   if (lb >= nb) return;  // alignment padding
-  readout_kick_drift_block<kSplit>(M.p, M.g, M.f, M.prm, nullptr, 0.0f, lb, nb);
+  readout_kick_drift_block<true>(M.p, M.g, M.f, M.prm, nullptr, 0.0f, lb, nb);
 }
 
 unsigned blocks_for(long long n) { return (unsigned)((n + kThreads - 1) / kThreads); }
@@ -1364,19 +1359,12 @@ int launch_grid_contrast(const PosSource& src, int n, float boxsize, const GridB
   return kOk;
 }
 
-// The variant for the layout of f.
-template <class K>
-static K layout_of(const ForceLines& f, int ng, K apart, K split, K whole)
-{
-  return f.rec_row == 0 ? apart : f.rec_row < ng ? split : whole;
-}
-
 int launch_readout(const DevParticles& p, const CicGeom& g, const ForceLines& f, const double* fsum, hipStream_t s)
 {
   if (p.np == 0) return kOk;
   const float inv_cells = (float)(1.0 / ((double)g.ng * g.ng * g.ng));
-  hipLaunchKernelGGL(layout_of(f, g.ng, k_readout<kApart>, k_readout<kSplit>, k_readout<kWhole>), dim3(blocks_for(p.np)), dim3(kThreads), 0, s, p, g,
-                     f, fsum, inv_cells);
+  hipLaunchKernelGGL(f.rec_row < g.ng ? k_readout<true> : k_readout<false>, dim3(blocks_for(p.np)), dim3(kThreads), 0,
+                     s, p, g, f, fsum, inv_cells);
   COLA_HIP(hipGetLastError());
   return kOk;
 }
@@ -1386,8 +1374,8 @@ int launch_readout_kick_drift(const DevParticles& p, const CicGeom& g, const For
 {
   if (p.np == 0) return kOk;
   const float inv_cells = (float)(1.0 / ((double)g.ng * g.ng * g.ng));
-  hipLaunchKernelGGL(layout_of(f, g.ng, k_readout_kick_drift<kApart>, k_readout_kick_drift<kSplit>, k_readout_kick_drift<kWhole>), dim3(blocks_for(p.np)),
-                     dim3(kThreads), 0, s, p, g, f, prm, fsum, inv_cells);
+  hipLaunchKernelGGL(f.rec_row < g.ng ? k_readout_kick_drift<true> : k_readout_kick_drift<false>,
+                     dim3(blocks_for(p.np)), dim3(kThreads), 0, s, p, g, f, prm, fsum, inv_cells);
   COLA_HIP(hipGetLastError());
   return kOk;
 }
