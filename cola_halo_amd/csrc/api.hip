@@ -351,9 +351,18 @@ KOpParams pm_kop(const cola_context* c)
 // particles are still near their lattice).
 bool writes_records(const cola_context* c) { return !c->net; }
 
+// The transforms of a force (pm.c:282-355), without a net's layers.
+int force_transforms(cola_context* c)
+{
+  c->density_is_real = false;
+  COLA_TRY(c->pm_fft.forces(c->density, c->fgrid, pm_kop(c), writes_records(c), c->stream));
+  c->fi_force = false;
+  c->force_records = writes_records(c);
+  return kOk;
+}
+
 int pm_fields(cola_context* c)
 {
-  const KOpParams kp = pm_kop(c);
   // the net's features come from the real-space density before the r2c
   // overwrites it; its last layer adds its output to the force grids
   // with fuse34 (by input planes) layer 3 runs with the last layer after the transforms
@@ -378,10 +387,9 @@ int pm_fields(cola_context* c)
     COLA_TRY(resnet_layers23(c->net, c->stream));
     phase_end(c, kPhNetHidden);
   }
-  c->density_is_real = false;
   // the readout gathers records; the net's last layer reads the components
   // apart and writes the corrected records
-  COLA_TRY(c->pm_fft.forces(c->density, c->fgrid, kp, writes_records(c), c->stream));
+  COLA_TRY(force_transforms(c));
   if (fused34) {
     phase_begin(c, kPhNetConv34);
     COLA_TRY(resnet_layer3_head(c->net, c->fgrid, c->cic.row, c->stream));
@@ -392,7 +400,6 @@ int pm_fields(cola_context* c)
     phase_end(c, kPhNetHead);
   }
   c->fi_force = c->net != nullptr;
-  c->force_records = writes_records(c);
   return kOk;
 }
 
@@ -1626,7 +1633,9 @@ int cola_set_fft_tiles_xy(cola_context* c, int log2_ycols, int log2_xcols, int l
 namespace {
 
 // Mean device time of `reps` PM force fields (deposit + transforms) of the
-// current particle state.
+// current particle state, the transforms in the layout the context's steps
+// use: with a net attached its layers are left out (their shapes are fixed and
+// would only add their time and its noise), the components apart are not.
 int time_pm_fields(cola_context* c, int reps, double* ms)
 {
   hipEvent_t e0 = nullptr, e1 = nullptr;
@@ -1636,11 +1645,11 @@ int time_pm_fields(cola_context* c, int reps, double* ms)
     return kErrHip;
   }
   int st = pm_assign(c, false);
-  if (!st) st = pm_fields(c);
+  if (!st) st = force_transforms(c);
   if (!st && hipEventRecord(e0, c->stream) != hipSuccess) st = kErrHip;
   for (int r = 0; r < reps && !st; ++r) {
     st = pm_assign(c, false);
-    if (!st) st = pm_fields(c);
+    if (!st) st = force_transforms(c);
   }
   float t = 0;
   if (!st && (hipEventRecord(e1, c->stream) != hipSuccess || hipEventSynchronize(e1) != hipSuccess ||
@@ -1663,11 +1672,7 @@ int cola_autotune(cola_context* c, int reps, cola_tuning* out)
   COLA_TRY(require_particles(c));
   const bool prof = c->profiling;
   c->profiling = false;
-  // the shapes tuned here are the PM's; the net's kernels have fixed shapes
-  // and would only add their time (and its noise) to every trial
   COLA_TRY(launch_wrap(c->p, c->boxf, c->stream));  // move.c:33-41, as every step begins
-  ResNet* const net = c->net;
-  c->net = nullptr;  // restored below on every path
   cola_tuning best;
   for (int a = 0; a < 3; ++a) best.tile[a] = c->tile_sides[a];
   best.fft_log2_cols = c->fft_log2_tile;
@@ -1738,7 +1743,6 @@ int cola_autotune(cola_context* c, int reps, cola_tuning* out)
     (void)cola_fft_radices(c->ng, best.fft_schedule, best.fft_radices, 8);
   }
   c->profiling = prof;
-  c->net = net;
   *out = best;
   return st;
 }

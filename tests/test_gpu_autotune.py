@@ -116,3 +116,33 @@ def test_wide_row_tiles_agree_bit_for_bit(eh_table, nc, ng, rows):
     finally:
         for c in ctxs:
             c.close()
+
+
+def test_autotune_of_a_corrected_context(eh_table):
+    """With a net attached the tuner times the transforms of the corrected
+    run (the components apart) and leaves the corrected forces as they were;
+    its own last force is the plain one."""
+    print("autotune corrected 64^3 / 96^3", flush=True)
+    k, p = eh_table
+    ng = 96
+    net = ch.ResidualNet(ng)
+    with ch.Context(64, ng, 100.0) as ctx:
+        ctx.power_init_table(k, p, 0.1, 0.8, OM, 1.0 - OM)
+        ctx.lpt_set_displacement(0.1, OM, 3)
+        ctx.move_particles()
+        ctx.pm_calculate_forces()
+        plain = [ctx.get_force_grid(a)[:, :, :ng] for a in range(3)]
+        ctx.set_residual_net(net)
+        ctx.pm_calculate_forces()
+        before, grid = ctx.get_forces(), ctx.get_force_grid(0)
+        tuned = ctx.autotune(reps=2)
+        assert tuned["ms_after"] <= tuned["ms_before"]
+        for a in range(3):
+            scale = np.abs(plain[a]).max()
+            assert np.abs(ctx.get_force_grid(a)[:, :, :ng] - plain[a]).max() <= 2e-6 * scale
+        ctx.set_fft_schedule(0)
+        ctx.pm_calculate_forces()
+        assert np.array_equal(ctx.get_forces(), before)
+        assert np.array_equal(ctx.get_force_grid(0), grid)
+        ctx.set_residual_net(None)
+    net.close()
