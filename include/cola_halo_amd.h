@@ -531,7 +531,11 @@ int cola_write_coarse_grid(const char* filename, float boxsize, int n, const flo
 /* Deposit tile shape (cells per tile along x, y, z: powers of two dividing
    ngrid, x side >= 2, product <= 4096) and FFT tile width (log2 of the transforms per
    workgroup, -1 = automatic).  Results do not depend on either; the
-   autotuner sweeps them for speed. */
+   autotuner sweeps them for speed.  The default tiles are 8 x 8 x 32, partial
+   at the end of an axis they do not divide; the largest dividing sides up to
+   those (2 x 2 x 2 at ngrid 270) are the name by which this call and
+   cola_tuning know them, so there tiles of just those sides, which took 60
+   times as long, cannot be had. */
 int cola_set_tiling(cola_context* ctx, int tx, int ty, int tz, int fft_log2_tile);
 /* Adjacent FFT column tiles dispatched to one XCD (a power of two, 1 to 64). */
 int cola_set_fft_xcd_group(cola_context* ctx, int group);

@@ -146,3 +146,32 @@ def test_autotune_of_a_corrected_context(eh_table):
         assert np.array_equal(ctx.get_force_grid(0), grid)
         ctx.set_residual_net(None)
     net.close()
+
+
+@pytest.mark.parametrize("nc,ng", [(18, 54), (32, 96)])
+def test_tuning_of_partial_tiles_applies_elsewhere(eh_table, nc, ng):
+    """The default tiles go by their dividing sides (2 x 2 x 2 at 54^3) in the
+    tuner's result, which another context takes; 8 x 8 x 32 by name stays
+    refused where it does not divide the grid.  The density is the same."""
+    print(f"tuning of partial tiles ng={ng}", flush=True)
+    k, p = eh_table
+    rng = np.random.default_rng(ng)
+    parts = np.zeros(nc ** 3, ch.PARTICLE_DTYPE)
+    parts["x"] = rng.uniform(0, 100.0, (nc ** 3, 3)).astype(np.float32)
+    parts["id"] = np.arange(1, nc ** 3 + 1)
+    grids = []
+    for tuned in (None, "self", "other"):
+        with ch.Context(nc, ng, 100.0) as ctx:
+            ctx.set_particles(parts, 0.5, 0.5)
+            if tuned == "self":
+                t = ctx.autotune(reps=1)
+                assert all(ng % s == 0 for s in t["tile"])
+            elif tuned == "other":
+                ctx.apply_tuning(t)
+                if ng % 32:
+                    with pytest.raises(ch.ColaError):
+                        ctx.set_tiling(8, 8, 32)
+                    ctx.set_tiling(2, 2, 2)
+            ctx.pm_assign()
+            grids.append(ctx.get_density())
+    assert np.array_equal(grids[0], grids[1]) and np.array_equal(grids[0], grids[2])
