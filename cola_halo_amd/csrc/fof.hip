@@ -98,24 +98,6 @@ k_fof_gather(long long np, const int* __restrict__ sidx, const float* __restrict
   parent[k] = (int)k;
 }
 
-// Column starts: the first sorted entry of every (x, y) column, np past the
-// last.  Entry k fills the columns after its predecessor's up to its own.
-__global__ void __launch_bounds__(kThreads)
-k_fof_columns(long long np, int nd, const unsigned* __restrict__ skeys, int* __restrict__ start)
-{
-  const long long k = (long long)blockIdx.x * kThreads + threadIdx.x;
-  if (k > np) return;
-  const unsigned ncol = (unsigned)nd * (unsigned)nd;
-  const unsigned col = k < np ? skeys[k] / (unsigned)nd : ncol;
-  for (unsigned c = k > 0 ? skeys[k - 1] / (unsigned)nd + 1 : 0; c <= col; ++c) start[c] = (int)k;
-}
-
-struct LinkGeom {
-  long long np;
-  int nd;
-  float box, half, ll2;
-};
-
 // First entry of [lo, hi) whose key is at least `key`.
 __device__ inline long long lower_bound(const unsigned* a, long long lo, long long hi, unsigned key)
 {
@@ -128,6 +110,25 @@ __device__ inline long long lower_bound(const unsigned* a, long long lo, long lo
   }
   return lo;
 }
+
+// Column starts: the first sorted entry of every (x, y) column, np past the
+// last.  A search over all keys per column, 0.049 ms for 1267^2 columns of 256^3
+// particles.  Entries that fill the columns up to their own are as fast there
+// and serial where few have many to fill (64^3 particles on 16 lines of 1600^2
+// columns: a catalogue in 20.9 ms, by search 3.2).
+__global__ void __launch_bounds__(kThreads)
+k_fof_columns(long long np, int nd, const unsigned* __restrict__ skeys, int* __restrict__ start)
+{
+  const long long c = (long long)blockIdx.x * kThreads + threadIdx.x;
+  if (c > (long long)nd * nd) return;
+  start[c] = (int)lower_bound(skeys, 0, np, (unsigned)(c * nd));
+}
+
+struct LinkGeom {
+  long long np;
+  int nd;
+  float box, half, ll2;
+};
 
 // The cells klo..khi lie in one (x, y) column, whose entries are
 // [start[col], start[col + 1]): at ~5 linking cells per particle spacing a
@@ -405,7 +406,7 @@ int fof_run(const FofInput& in, FofResult* out, hipStream_t s)
   g.box = in.boxsize;
   g.half = 0.5f * in.boxsize;
   g.ll2 = in.ll * in.ll;  // fof.c:452
-  hipLaunchKernelGGL(k_fof_columns, dim3(blocks(np + 1)), dim3(kThreads), 0, s, np, nd, skeys, start);
+  hipLaunchKernelGGL(k_fof_columns, dim3(blocks((long long)nd * nd + 1)), dim3(kThreads), 0, s, np, nd, skeys, start);
   hipLaunchKernelGGL(k_fof_link, dim3(blocks(np)), dim3(kThreads), 0, s, g, skeys, start, spos, parent);
   hipLaunchKernelGGL(k_fill<int>, dim3(blocks(np)), dim3(kThreads), 0, s, count, np, 0);
   hipLaunchKernelGGL(k_fill<int>, dim3(blocks(np)), dim3(kThreads), 0, s, minidx, np, INT_MAX);

@@ -92,6 +92,23 @@ def test_fof_columns_sparse_and_few(nc, box, ll):
         _compare(ctx, snap, box, ll, 2)
 
 
+@pytest.mark.parametrize("where", [(0.0, 0.0), (31.0, 17.0), (63.99, 63.99)])
+def test_fof_one_column(eh_table, where):
+    """All particles in one of 1267^2 columns of linking cells (the first, one
+    within, the last), which all others' starts lie before or after."""
+    nc, box, ll = 8, 64.0, 0.05
+    _say(f"fof one column at {where}")
+    rng = np.random.default_rng(5)
+    snap = np.zeros(nc ** 3, ch.PARTICLE_MIN_DTYPE)
+    snap["x"][:, :2] = where
+    snap["x"][:, 2] = rng.uniform(0, box, nc ** 3)
+    snap["v"] = rng.normal(0, 100.0, (nc ** 3, 3)).astype(np.float32)
+    snap["id"] = np.arange(1, nc ** 3 + 1)
+    with ch.Context(nc, nc, box) as ctx:
+        ctx.set_snapshot_records(snap)
+        _compare(ctx, snap, box, ll, 2)
+
+
 def test_fof_evolved_128(eh_table):
     """128^3 particles evolved to z = 0 (L = 250, 384^3 PM grid, 10 steps),
     linking length 0.2 of the mean separation (main.c:353)."""
