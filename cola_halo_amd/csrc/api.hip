@@ -523,7 +523,7 @@ int cola_context_create(int nc, int ngrid, double boxsize, cola_context** out)
   }
   st = bin_alloc(&c->bins, c->tiles, c->np);
   if (st) return fail(kErrAlloc);
-  if (grid_bin_alloc(&c->grid_bins, kNoAllocGrid)) return fail(kErrAlloc);
+  if (grid_bin_alloc(&c->grid_bins, kNoAllocGrid) || grid_share_alloc(&c->grid_bins, c->np)) return fail(kErrAlloc);
   if (hipMalloc(&c->d_mass, sizeof(double) * cola_context::kMassSlots) != hipSuccess) return fail(kErrAlloc);
   if (hipMemset(c->d_mass, 0, sizeof(double) * cola_context::kMassSlots) != hipSuccess) return fail(kErrHip);
   if (hipHostMalloc(&c->h_prm, sizeof(StepParams) * cola_context::kMassSlots) != hipSuccess) return fail(kErrAlloc);

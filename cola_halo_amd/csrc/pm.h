@@ -97,9 +97,12 @@ int launch_zero_mass(double* ring, const StepParams* prm, hipStream_t s);
 struct GridBins {
   int* counts[2] = {nullptr, nullptr};  // tiles (zero between calls), then tiles + 1 offsets, then the scan's sums
   long long tiles[2] = {0, 0};
+  unsigned long long* shared = nullptr;  // cells of tiles that several workgroups sum (zero between calls), then
+  int nshared = 0;                       // their workgroups' arrivals (nshared slots)
 };
 TileGeom grid_tile_geom(int n);
 int grid_bin_alloc(GridBins* b, int n);  // at least the tiles of an n^3 grid (keeps what is large enough)
+int grid_share_alloc(GridBins* b, long long np);  // the slots for np particles
 void grid_bin_free(GridBins* b);
 // Workgroups that share a tile's particles: above 1 the grid needs the
 // fixed-point sums fix[n^3], at 1 none.

@@ -720,31 +720,97 @@ __device__ __forceinline__ void grid_tile_add(const GridGeom& g, const TileGeom&
   }
 }
 
+// Entries of a tile beyond which its workgroup shares them: the sorted entries
+// fall into aligned shares of kGridShare, and a tile of more than two has at
+// least one share to itself, summed by a workgroup of its own.  (A tile with
+// half of 256^3 particles on 400^3 cells kept one workgroup busy for 35 of 61
+// ms, a fifth on 256^3 for 7 of 14; other inputs take as long as without.)
+constexpr int kGridShare = 65536;
+constexpr int kGridCells = 8 * 8 * 32;
+
+struct GridShares {
+  unsigned long long* cells = nullptr;  // [n][kGridCells] sums, zero between calls
+  int* arrived = nullptr;               // [n], zero between calls
+  int n = 0;
+};
+
+// The whole shares [first, last) of a tile's entries, none in a tile of at
+// most two: the tile's slot is the first.
+__device__ inline int2 grid_shares(int beg, int end, int n)
+{
+  if (end - beg <= 2 * kGridShare) return make_int2(0, 0);
+  const int first = (int)(((long long)beg + kGridShare - 1) / kGridShare);
+  return make_int2(first, max(first, min(end / kGridShare, n)));
+}
+
 // SPLIT false: a workgroup owns a tile and writes its contrast (the value and
-// the sums of k_density_contrast).  SPLIT true: nsplit workgroups share a
-// tile's particles and add their cells to the fixed-point grid fix[n^3].
+// the sums of k_density_contrast); of a tile with whole shares its workgroup
+// and the shares' (the grid's first sh.n) add their cells to the tile's slot,
+// and the last of them to arrive writes it.  SPLIT true: nsplit workgroups
+// share a tile's particles and add their cells to the fixed-point grid fix[n^3].
 template <bool SPLIT>
 __global__ void __launch_bounds__(kDepositThreads)
 k_grid_tiles(GridGeom g, TileGeom t, const int* __restrict__ offsets, const float* __restrict__ sorted, int nsplit,
-             long long row, float nbar_inv, unsigned long long* __restrict__ fix, float* __restrict__ grid,
-             double* __restrict__ sums)
+             GridShares sh, long long row, float nbar_inv, unsigned long long* __restrict__ fix,
+             float* __restrict__ grid, double* __restrict__ sums)
 {
   extern __shared__ unsigned long long cells[];
-  const int tile = SPLIT ? (int)(blockIdx.x / (unsigned)nsplit) : (int)blockIdx.x;
+  __shared__ int is_last;
+  const int share = SPLIT ? -1 : (int)blockIdx.x;  // below sh.n: this workgroup's share
+  int tile = SPLIT ? (int)(blockIdx.x / (unsigned)nsplit) : (int)blockIdx.x - sh.n;
+  if (!SPLIT && share < sh.n) {
+    // the tile that holds the share's first entry
+    const int at = share * kGridShare;
+    if (at >= offsets[t.ntiles]) return;
+    int lo = 0, hi = (int)t.ntiles - 1;
+    while (lo < hi) {
+      const int mid = (lo + hi + 1) >> 1;
+      if (offsets[mid] <= at)
+        lo = mid;
+      else
+        hi = mid - 1;
+    }
+    tile = lo;
+  }
   const int tz = tile % t.ntz, ty = (tile / t.ntz) % t.nty, tx = tile / (t.ntz * t.nty);
   const int x0 = tx << t.lx, y0 = ty << t.ly, z0 = tz << t.lz;
   const int ncell = 1 << (t.lx + t.ly + t.lz);
   int beg = offsets[tile], end = offsets[tile + 1];
+  int2 whole = make_int2(0, 0);
   if (SPLIT) {
     const int part = (int)(blockIdx.x % (unsigned)nsplit);
     const int len = (end - beg + nsplit - 1) / nsplit;
     beg = min(end, beg + part * len);
     end = min(end, beg + len);
     if (beg >= end) return;
+  } else {
+    whole = grid_shares(beg, end, sh.n);
+    if (share < sh.n && (share < whole.x || share >= whole.y)) return;
   }
   for (int e = threadIdx.x; e < ncell; e += kDepositThreads) cells[e] = 0ULL;
   __syncthreads();
-  grid_tile_add(g, t, sorted, beg, end, x0, y0, z0, cells);
+  if (!SPLIT && whole.x < whole.y) {
+    if (share < sh.n) {
+      grid_tile_add(g, t, sorted, share * kGridShare, (share + 1) * kGridShare, x0, y0, z0, cells);
+    } else {
+      grid_tile_add(g, t, sorted, beg, whole.x * kGridShare, x0, y0, z0, cells);
+      grid_tile_add(g, t, sorted, whole.y * kGridShare, end, x0, y0, z0, cells);
+    }
+    __syncthreads();
+    unsigned long long* const slot = sh.cells + (long long)whole.x * kGridCells;
+    for (int e = threadIdx.x; e < ncell; e += kDepositThreads)
+      if (cells[e]) atomicAdd(&slot[e], cells[e]);
+    __threadfence();
+    __syncthreads();
+    if (threadIdx.x == 0) is_last = atomicAdd(&sh.arrived[whole.x], 1) == whole.y - whole.x;
+    __syncthreads();
+    if (!is_last) return;
+    __threadfence();
+    for (int e = threadIdx.x; e < ncell; e += kDepositThreads) cells[e] = atomicExch(&slot[e], 0ULL);
+    if (threadIdx.x == 0) (void)atomicExch(&sh.arrived[whole.x], 0);
+  } else {
+    grid_tile_add(g, t, sorted, beg, end, x0, y0, z0, cells);
+  }
   __syncthreads();
   const int zmask = t.tz - 1, ymask = t.ty - 1;
   double s_in = 0.0, s_out = 0.0;
@@ -1292,8 +1358,21 @@ int grid_bin_alloc(GridBins* b, int n)
   return kOk;
 }
 
+int grid_share_alloc(GridBins* b, long long np)
+{
+  // entries average 1.3 a particle; a tile's beyond 2 np its own workgroup sums
+  const int n = (int)(2 * np / kGridShare);
+  if (n == 0) return kOk;
+  const size_t cells = sizeof(unsigned long long) * kGridCells * n, bytes = cells + sizeof(int) * n;
+  COLA_HIP(hipMalloc(&b->shared, bytes));
+  COLA_HIP(hipMemset(b->shared, 0, bytes));
+  b->nshared = n;
+  return kOk;
+}
+
 void grid_bin_free(GridBins* b)
 {
+  if (b->shared) (void)hipFree(b->shared);
   for (int* p : b->counts)
     if (p) (void)hipFree(p);
   *b = GridBins{};
@@ -1347,12 +1426,16 @@ int launch_grid_contrast(const PosSource& src, int n, float boxsize, const GridB
   const size_t lds = sizeof(unsigned long long) * t.tx * t.ty * t.tz;
   COLA_TRY(launch_fill_zero(sums, 2, s));
   if (nsplit <= 1) {
-    hipLaunchKernelGGL(k_grid_tiles<false>, dim3((unsigned)t.ntiles), dim3(kDepositThreads), lds, s, g, t, bb.offsets,
-                       sorted, 1, row, nbar_inv, fix, grid, sums);
+    GridShares sh;
+    sh.cells = b.shared;
+    sh.n = b.nshared;
+    sh.arrived = reinterpret_cast<int*>(b.shared + (long long)sh.n * kGridCells);
+    hipLaunchKernelGGL(k_grid_tiles<false>, dim3((unsigned)(t.ntiles + sh.n)), dim3(kDepositThreads), lds, s, g, t,
+                       bb.offsets, sorted, 1, sh, row, nbar_inv, fix, grid, sums);
   } else {
     COLA_TRY(launch_fill_zero(fix, (long long)n * n * n, s));
     hipLaunchKernelGGL(k_grid_tiles<true>, dim3((unsigned)(t.ntiles * nsplit)), dim3(kDepositThreads), lds, s, g, t,
-                       bb.offsets, sorted, nsplit, row, nbar_inv, fix, grid, sums);
+                       bb.offsets, sorted, nsplit, GridShares{}, row, nbar_inv, fix, grid, sums);
     COLA_TRY(launch_density_contrast(n, row, nbar_inv, fix, grid, sums, s));
   }
   COLA_HIP(hipGetLastError());

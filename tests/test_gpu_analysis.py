@@ -170,3 +170,34 @@ def test_output_grid_cells_exact(nc, n):
     assert np.array_equal(delta, ref)
     assert np.array_equal(again, ref)
     assert sums[0] == pytest.approx(npart, rel=1e-6)
+
+
+@pytest.mark.parametrize("nc,n,parts", [(64, 64, (0.9,)), (64, 100, (0.51, 0.49)), (96, 96, (0.3, 0.16, 0.16, 0.3)),
+                                        (96, 130, (1.0,))])
+def test_output_grid_of_a_clump(nc, n, parts):
+    """Tiles that hold a large part of all particles (one just beyond two
+    shares of 65536 entries, several, all), which several workgroups sum:
+    every cell equals the fixed-point sum, in call after call, also where the
+    clump moves in between."""
+    box = 40.0
+    print(f"output grid clump nc={nc} n={n} {parts}", flush=True)
+    rng = np.random.default_rng(n)
+    npart = nc ** 3
+    with ch.Context(nc, nc, box) as ctx:
+        for turn in range(2):
+            x = rng.uniform(0, box, (npart, 3)).astype(np.float32)
+            at = 0
+            for f in parts:
+                m = int(f * npart)
+                tile = rng.integers(0, n // 32, 3) * np.array([32, 32, 32])
+                lo = (tile + np.array([0.1, 0.1, 0.1])) * box / n
+                x[at:at + m] = lo + rng.uniform(0, 1, (m, 3)) * np.array([6.8, 6.8, 30.8]) * box / n
+                at += m
+            snap = np.zeros(npart, ch.PARTICLE_MIN_DTYPE)
+            snap["x"], snap["id"] = x, np.arange(1, npart + 1)
+            ctx.set_snapshot_records(snap)
+            ref = _contrast_exact(x, n, box)
+            for call in range(2):
+                delta, sums = ctx.coarse_grid(n, "snapshot")
+                assert np.array_equal(delta, ref), (turn, call)
+                assert sums[0] == pytest.approx(npart, rel=1e-6)
