@@ -1783,7 +1783,7 @@ int position_source(cola_context* c, int source, PosSource* src)
 // Buffers of an output grid of n^3 cells held in `floats` floats.
 int ensure_aux(cola_context* c, int n, long long floats)
 {
-  const long long cells = grid_split(n, c->np) > 1 ? (long long)n * n * n : 0;
+  const long long cells = grid_needs_fix(n, c->np) ? (long long)n * n * n : 0;
   COLA_TRY(grid_bin_alloc(&c->grid_bins, n));
   if (!c->d_aux) COLA_HIP(hipMalloc(&c->d_aux, sizeof(double) * (2 + 3 * kMaxShellBins)));
   if (c->aux_floats < floats) {

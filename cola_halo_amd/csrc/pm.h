@@ -104,9 +104,8 @@ TileGeom grid_tile_geom(int n);
 int grid_bin_alloc(GridBins* b, int n);  // at least the tiles of an n^3 grid (keeps what is large enough)
 int grid_share_alloc(GridBins* b, long long np);  // the slots for np particles
 void grid_bin_free(GridBins* b);
-// Workgroups that share a tile's particles: above 1 the grid needs the
-// fixed-point sums fix[n^3], at 1 none.
-int grid_split(int n, long long np);
+// Whether the grid of np positions needs the fixed-point sums fix[n^3].
+bool grid_needs_fix(int n, long long np);
 // coarse_grid.c:49-70 on n^3 cells: counting sort of the positions into tiles
 // (sorted: scratch of `capacity` >= 8 np entries of three floats), CIC sums
 // in LDS, grid = nbar_inv * rho - 1 with rows of `row` floats, sums = the

@@ -686,6 +686,20 @@ k_sum_doubles(const double* __restrict__ v, long long n, double* ring, const Ste
   sum_doubles_block(v, n, ring, prm, blockIdx.x);
 }
 
+// The eight cells and weights of a position (coarse_grid.c:103-120).
+template <class F>
+__device__ __forceinline__ void grid_add(const GridAxis& ax, const GridAxis& ay, const GridAxis& az, F&& add)
+{
+  add(ax.i0, ay.i0, az.i0, ax.w * ay.w * az.w);
+  add(ax.i0, ay.i1, az.i0, ax.w * (1 - ay.w) * az.w);
+  add(ax.i0, ay.i0, az.i1, ax.w * ay.w * (1 - az.w));
+  add(ax.i0, ay.i1, az.i1, ax.w * (1 - ay.w) * (1 - az.w));
+  add(ax.i1, ay.i0, az.i0, (1 - ax.w) * ay.w * az.w);
+  add(ax.i1, ay.i1, az.i0, (1 - ax.w) * (1 - ay.w) * az.w);
+  add(ax.i1, ay.i0, az.i1, (1 - ax.w) * ay.w * (1 - az.w));
+  add(ax.i1, ay.i1, az.i1, (1 - ax.w) * (1 - ay.w) * (1 - az.w));
+}
+
 // ---- output grids: one workgroup per tile, or several -----------------------
 // The eight weights of coarse_grid.c:103-120 of the entries [beg, end) added
 // to the tile's LDS cells (fixed point as above, so the grid is the same bit
@@ -697,26 +711,21 @@ k_sum_doubles(const double* __restrict__ v, long long n, double* ring, const Ste
 // added in LDS and a cell is written once: 1.57 ms at 256^3 (count .47,
 // scatter .54, tiles .57) and 4.6 ms.  The floor, positions read and cells
 // written once, is 0.05 and 0.34 ms; the rest is the sort and, on coarse
-// grids, lanes of a wavefront adding to the same cells.
+// grids, lanes of a wavefront adding to the same cells.  Only positions in
+// random order, which share no tiles within a workgroup, can lose: 256^3 on
+// 128^3 6.6 ms for 5.8 (0.65 for 3.9 in lattice order), 64^3 on 128^3 0.20 for
+// 0.12.
 __device__ __forceinline__ void grid_tile_add(const GridGeom& g, const TileGeom& t, const float* __restrict__ sorted,
                                               int beg, int end, int x0, int y0, int z0, unsigned long long* cells)
 {
   for (int k = beg + (int)threadIdx.x; k < end; k += kDepositThreads) {
     const GridAxis ax = grid_axis(sorted[3LL * k + 0], g), ay = grid_axis(sorted[3LL * k + 1], g),
                    az = grid_axis(sorted[3LL * k + 2], g);
-    auto add = [&](int i, int j, int kk, float w) {
+    grid_add(ax, ay, az, [&](int i, int j, int kk, float w) {
       const unsigned li = (unsigned)(i - x0), lj = (unsigned)(j - y0), lk = (unsigned)(kk - z0);
       if (li < (unsigned)t.tx && lj < (unsigned)t.ty && lk < (unsigned)t.tz)
         atomicAdd(&cells[(((li << t.ly) + lj) << t.lz) + lk], (unsigned long long)rintf(w * kFix));
-    };
-    add(ax.i0, ay.i0, az.i0, ax.w * ay.w * az.w);
-    add(ax.i0, ay.i1, az.i0, ax.w * (1 - ay.w) * az.w);
-    add(ax.i0, ay.i0, az.i1, ax.w * ay.w * (1 - az.w));
-    add(ax.i0, ay.i1, az.i1, ax.w * (1 - ay.w) * (1 - az.w));
-    add(ax.i1, ay.i0, az.i0, (1 - ax.w) * ay.w * az.w);
-    add(ax.i1, ay.i1, az.i0, (1 - ax.w) * (1 - ay.w) * az.w);
-    add(ax.i1, ay.i0, az.i1, (1 - ax.w) * ay.w * (1 - az.w));
-    add(ax.i1, ay.i1, az.i1, (1 - ax.w) * (1 - ay.w) * (1 - az.w));
+    });
   }
 }
 
@@ -843,6 +852,20 @@ k_grid_tiles(GridGeom g, TileGeom t, const int* __restrict__ offsets, const floa
       unsafeAtomicAdd(&sums[threadIdx.x], tot);
     }
   }
+}
+
+// The same weights straight to the grid: one thread per particle, eight 64-bit
+// atomics.
+__global__ void __launch_bounds__(kThreads)
+k_grid_direct(PosSource src, GridGeom g, unsigned long long* __restrict__ fix)
+{
+  const long long i = (long long)blockIdx.x * kThreads + threadIdx.x;
+  if (i >= src.np) return;
+  const GridAxis ax = grid_axis(src.x[0][i * src.stride], g), ay = grid_axis(src.x[1][i * src.stride], g),
+                 az = grid_axis(src.x[2][i * src.stride], g);
+  grid_add(ax, ay, az, [&](int x, int y, int z, float w) {
+    atomicAdd(&fix[((long long)x * g.n + y) * g.n + z], (unsigned long long)rintf(w * kFix));
+  });
 }
 
 template <int STRIDE>
@@ -1358,10 +1381,17 @@ int grid_bin_alloc(GridBins* b, int n)
   return kOk;
 }
 
+// Up to as many particles the weights go straight to the grid: the sort's
+// launches cost more than it saves.  Direct against sorted, evolved particles:
+// 16^3 on 16^3 0.025 against 0.051 ms, 32^3 on 32^3 0.034, 0.061, on 128^3
+// 0.044, 0.068, 48^3 on 48^3 0.055, 0.068; 54^3 on 54^3 0.068, 0.068; 64^3 on
+// 64^3 0.103, 0.071.
+constexpr long long kGridDirect = 1LL << 17;
+
 int grid_share_alloc(GridBins* b, long long np)
 {
   // entries average 1.3 a particle; a tile's beyond 2 np its own workgroup sums
-  const int n = (int)(2 * np / kGridShare);
+  const int n = np <= kGridDirect ? 0 : (int)(2 * np / kGridShare);
   if (n == 0) return kOk;
   const size_t cells = sizeof(unsigned long long) * kGridCells * n, bytes = cells + sizeof(int) * n;
   COLA_HIP(hipMalloc(&b->shared, bytes));
@@ -1386,11 +1416,13 @@ void grid_bin_free(GridBins* b)
 // 1.24, 1.32, 1.00, 0.36 ms), 8192 and 16384 in between.
 constexpr long long kGridTileShare = 4096;
 
-int grid_split(int n, long long np)
+static int grid_split(int n, long long np)
 {
   const long long per = np / grid_tile_geom(n).ntiles;
   return (int)std::min<long long>(1024, (per + kGridTileShare - 1) / kGridTileShare);
 }
+
+bool grid_needs_fix(int n, long long np) { return np <= kGridDirect || grid_split(n, np) > 1; }
 
 int launch_grid_contrast(const PosSource& src, int n, float boxsize, const GridBins& b, float* sorted,
                          long long capacity, int* overflow, unsigned long long* fix, long long row, float nbar_inv,
@@ -1409,6 +1441,13 @@ int launch_grid_contrast(const PosSource& src, int n, float boxsize, const GridB
   bb.counts = b.counts[k];
   bb.offsets = b.counts[k] + b.tiles[k];
   bb.block_sums = bb.offsets + b.tiles[k] + 1;
+  COLA_TRY(launch_fill_zero(sums, 2, s));
+  if (src.np <= kGridDirect) {
+    COLA_TRY(launch_fill_zero(fix, (long long)n * n * n, s));
+    hipLaunchKernelGGL(k_grid_direct, dim3(blocks_for(src.np)), dim3(kThreads), 0, s, src, g, fix);
+    COLA_HIP(hipGetLastError());
+    return launch_density_contrast(n, row, nbar_inv, fix, grid, sums, s);
+  }
   const int nsplit = grid_split(n, src.np);
   const unsigned nb = bin_blocks(src.np);
   auto bin = [&](auto stride) {
@@ -1424,7 +1463,6 @@ int launch_grid_contrast(const PosSource& src, int n, float boxsize, const GridB
   else
     COLA_TRY(bin(std::integral_constant<int, 8>{}));
   const size_t lds = sizeof(unsigned long long) * t.tx * t.ty * t.tz;
-  COLA_TRY(launch_fill_zero(sums, 2, s));
   if (nsplit <= 1) {
     GridShares sh;
     sh.cells = b.shared;

@@ -201,3 +201,10 @@ def test_output_grid_of_a_clump(nc, n, parts):
                 delta, sums = ctx.coarse_grid(n, "snapshot")
                 assert np.array_equal(delta, ref), (turn, call)
                 assert sums[0] == pytest.approx(npart, rel=1e-6)
+
+
+@pytest.mark.parametrize("n", [1, 2, 9, 33, 70, 128])
+def test_sorted_output_grid_cells_exact(n):
+    """As test_output_grid_cells_exact, with more particles than go straight
+    to the grid (2^17): tiles larger than the grid, ragged and whole ones."""
+    test_output_grid_cells_exact(54, n)
