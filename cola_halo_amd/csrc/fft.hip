@@ -249,19 +249,15 @@ constexpr int tile_waves_per_eu(int mode, KOp op, int emax, int rs)
 constexpr int fused_waves_per_eu(bool wide) { return wide ? 8 : 1; }
 constexpr int kFusedWideThreads = 768;  // above: WIDE
 
-// What a column pass of wave numbers multiplies by: the position's wave
-// number on the load, or the column's on the store (both 0: nothing).
-enum YScale : int { kYPlain = 0, kYByPosition = 1, kYByColumn = 2 };
-
 // Workgroup blk of a pass whose grid is nblk workgroups (the kernel's own
 // grid, or one job's share of a batched launch).
-// YS: the pass may scale (yscale).
-template <int DIR, int MODE, KOp OP, int EMAX, int RS, bool YS = false>
+template <int DIR, int MODE, KOp OP, int EMAX, int RS>
 __device__ __forceinline__ void tile_run(const void* in_, void* out_, const float2* __restrict__ tw, const TileArgs& A,
-                                         int blk, int nblk, int tid, int yscale = kYPlain, bool stage_twiddles = true)
+                                         int blk, int nblk)
 {
   extern __shared__ float2 smem[];
   const int n = A.P.n;
+  const int tid = threadIdx.x;
   const int nthr = blockDim.x;
   const int log2T = A.log2T;
   const int T = 1 << log2T;
@@ -278,8 +274,7 @@ __device__ __forceinline__ void tile_run(const void* in_, void* out_, const floa
   }
   float2* tws = smem;
   float2* lds = smem + n;
-  if (stage_twiddles)
-    for (int k = tid; k < n; k += nthr) tws[k] = tw[k];
+  for (int k = tid; k < n; k += nthr) tws[k] = tw[k];
 
   auto lidx = [&](int r, int c) { return MODE == kCols ? (r << log2T) + c : c * (n + 1) + r; };
   auto split = [&](int u, const FftPass& p, int& c, int& b) {
@@ -319,13 +314,6 @@ __device__ __forceinline__ void tile_run(const void* in_, void* out_, const floa
         for (int s = 0; s < R; ++s) {
           const float2* leg = in + (long long)(s * p.m) * A.sr;
           reg[q * R + s] = live ? leg[lane] : make_float2(0.0f, 0.0f);
-        }
-        if (YS && yscale == kYByPosition) {
-#pragma unroll
-          for (int s = 0; s < R; ++s) {
-            const float w = (float)wave_pm(b + s * p.m, n);
-            reg[q * R + s] = make_float2(w * reg[q * R + s].x, w * reg[q * R + s].y);
-          }
         }
         // the operator runs after all of this butterfly's loads are issued
         if constexpr (OP != KOp::None) {
@@ -448,11 +436,6 @@ __device__ __forceinline__ void tile_run(const void* in_, void* out_, const floa
         if (MODE == kCols) {
           float2* out = static_cast<float2*>(out_) + (long long)batch * A.bs + c0;
           const unsigned long long lane = col_offset(b, A.sr, c);
-          if (YS && yscale == kYByColumn) {
-            const float w = (float)(c0 + c);
-#pragma unroll
-            for (int t = 0; t < R; ++t) reg[q * R + t] = make_float2(w * reg[q * R + t].x, w * reg[q * R + t].y);
-          }
 #pragma unroll
           for (int t = 0; t < R; ++t) out[(long long)(t * p.m) * A.sr + lane] = reg[q * R + t];
         } else {
@@ -525,7 +508,7 @@ template <int DIR, int MODE, KOp OP, int EMAX, int RS>
 __global__ void __launch_bounds__(kFftMaxThreads) __attribute__((amdgpu_waves_per_eu(tile_waves_per_eu(MODE, OP, EMAX, RS))))
 fft_tile(const void* __restrict__ in_, void* __restrict__ out_, const float2* __restrict__ tw, TileArgs A)
 {
-  tile_run<DIR, MODE, OP, EMAX, RS>(in_, out_, tw, A, blockIdx.x, gridDim.x, threadIdx.x);
+  tile_run<DIR, MODE, OP, EMAX, RS>(in_, out_, tw, A, blockIdx.x, gridDim.x);
 }
 
 // ---- z c2r of the three force components of a line ---------------------------
@@ -1068,7 +1051,7 @@ fft_tile_jobs(const TileJob* __restrict__ jobs, const int* __restrict__ start, i
   const TileJob& J = jobs[j];
   const int lb = (int)blockIdx.x - start[j];
   if (lb >= J.blocks) return;  // alignment padding (before any barrier)
-  tile_run<DIR, MODE, KOp::None, EMAX, RS>(J.in, J.out[0], J.tw, J.A, lb, J.blocks, threadIdx.x);
+  tile_run<DIR, MODE, KOp::None, EMAX, RS>(J.in, J.out[0], J.tw, J.A, lb, J.blocks);
 }
 
 // (6 waves per SIMD at 8 values per thread: with 8 the tables' arguments spill)
