@@ -1416,20 +1416,26 @@ int cola_get_force_grid(cola_context* c, int axis, float* out, size_t n_out)
   COLA_HIP(hipStreamSynchronize(c->stream));
   const bool fi = c->fi_force && c->net;
   if (!fi && !c->force_records) return grid_to_host(c, c->fgrid[axis], out);
-  // records F[z][3], of the transforms or of the net's corrected grid: copied
-  // a few lines at a time, one component picked on the host
+  // records F[z][3], of the transforms or of the net's corrected grid: whole
+  // rows a few lines at a time (rows cut to their floats would be copied one
+  // by one), one component picked on the host
   const ForceLines fl = fi ? net_lines(c) : plain_lines(c);
   const long long lines = (long long)c->ng * c->ng, hrow = 2 * (c->ng / 2 + 1);
-  const long long chunk = std::max(1LL, std::min(lines, (1LL << 24) / (3LL * c->ng)));
-  std::vector<float> rec((size_t)(3LL * c->ng * chunk));
+  const int parts = (c->ng + fl.rec_row - 1) / fl.rec_row;
+  const long long chunk = std::max(1LL, std::min(lines, (1LL << 24) / (parts * fl.row)));
+  std::vector<float> rec((size_t)(parts * fl.row * chunk));
   for (long long l0 = 0; l0 < lines; l0 += chunk) {
     const long long nl = std::min(chunk, lines - l0);
-    for (int t = 0, z = 0; z < c->ng; ++t, z += fl.rec_row)
-      COLA_HIP(hipMemcpy2D(rec.data() + 3 * z, sizeof(float) * 3 * c->ng, fl.f + fl.at[t] + l0 * fl.row, sizeof(float) * fl.row,
-                           sizeof(float) * 3 * std::min(fl.rec_row, c->ng - z), (size_t)nl, hipMemcpyDeviceToHost));
+    for (int t = 0; t < parts; ++t)
+      COLA_HIP(hipMemcpy(rec.data() + t * chunk * fl.row, fl.f + fl.at[t] + l0 * fl.row, sizeof(float) * nl * fl.row,
+                         hipMemcpyDeviceToHost));
     for (long long l = 0; l < nl; ++l) {
       float* o = out + (l0 + l) * hrow;
-      for (int z = 0; z < c->ng; ++z) o[z] = rec[(size_t)((l * c->ng + z) * 3 + axis)];
+      for (int t = 0; t < parts; ++t) {
+        const float* r = rec.data() + (t * chunk + l) * fl.row + axis;
+        const int z0 = t * fl.rec_row, nz = std::min(fl.rec_row, c->ng - z0);
+        for (int z = 0; z < nz; ++z) o[z0 + z] = r[3 * z];
+      }
       o[c->ng] = o[c->ng + 1] = 0.0f;
     }
   }
