@@ -243,7 +243,8 @@ constexpr int tile_waves_per_eu(int mode, KOp op, int emax, int rs)
 
 // The fused x pass with radices 3, 4, 8 takes 73 VGPRs: 6 waves per SIMD, but
 // of 1024-thread workgroups only one fits a CU then.  WIDE: 64 registers (some
-// spill) and two of them: 768^3 (8 columns) 2.78 -> 2.27 ms.  Narrower
+// spill) and two of them: 768^3 (8 columns) 2.78 -> 2.27 ms, with a
+// grid per component 1.97.  Narrower
 // workgroups already share a CU and keep their registers (384^3 0.235 against
 // 0.258 ms; 768^3 with 4 columns 2.52 against 2.71).
 constexpr int fused_waves_per_eu(bool wide) { return wide ? 8 : 1; }
@@ -658,7 +659,7 @@ struct ColCtx {
 // index from (o + t L, c), with a 32-bit multiply per twiddle, was most of the
 // fused pass's VALU work, which bounds it: with f1 / k^2 folded into the kept
 // spectrum as well, 270^3 0.163 -> 0.129 ms, 384^3 0.327 -> 0.235, 480^3 0.90
-// -> 0.56, 768^3 2.98 -> 2.78, all of it with outputs in lines of three.)
+// -> 0.56, 768^3 2.98 -> 2.78, before each spectrum had a grid of its own.)
 template <int R, int EMAX, int DIR>
 __device__ inline void col_compute(float2 (&reg)[EMAX], const FftPass& p, const ColCtx& x)
 {

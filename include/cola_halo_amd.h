@@ -596,8 +596,8 @@ int cola_bandwidth_probe(size_t bytes, int reps, double* gbps);
 int cola_fft_r2c_3d(int n, float* data);
 /* Device time of this library's transforms on an n^3 grid resident in HBM
    (mean over reps after one warm-up, HIP events on the stream): ms_out[0]
-   r2c, ms_out[1] c2r, ms_out[2] the PM force sequence (r2c, then for each of
-   three axes the Poisson gradient and a c2r into its own grid).  For
+   r2c, ms_out[1] c2r, ms_out[2] the PM force sequence (r2c, Poisson gradient
+   and c2r of the three components, left as records for the readout).  For
    comparison with other FFT libraries; no reference counterpart. */
 int cola_fft_time(int n, int reps, double* ms_out);
 int cola_fft_c2r_3d(int n, float* data);
