@@ -251,7 +251,7 @@ int cola_coarse_grid(cola_context* ctx, int n, int source, float* delta_out, dou
 /* No counterpart in the reference.  For callers that cannot allocate device
    memory (code under HIP graph capture, tight serving loops, harnesses that
    forbid hipMalloc): cola_coarse_grid's kernels in the context's own buffers,
-   with the fixed-point sums of cells that several workgroups add to in a
+   with the fixed-point sums, where several workgroups add to a cell, in a
    static device array of the library (16 MiB per GPU, held until the
    process ends), so the call allocates nothing.  The context's buffers are
    its density bins (their entries, and counters made with the context): they
